@@ -58,16 +58,15 @@ __device__ __forceinline__ void finish(int v, T (&r)[PPT], long B, long PS, long
 //   gobj : objective gradient g (5 fields) or null; added by the x sweep
 // The x sweep (LAST) completes the stage: mode 0..3 RK4 update with step dt
 // (negative for the backward integration), mode 4 writes the RHS.
-template <typename T, typename Q, int DIR, bool PER>
+template <typename T, typename Q, int DIR, typename Lines>
 __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
                                             const double *const *__restrict__ q0p, T *__restrict__ rhs,
-                                            const double *__restrict__ gobj, const LineOp<T> &op,
+                                            const double *__restrict__ gobj, const Op<T> &op,
                                             const SweepGeom &g, double gamma, double inv_h, long N, int mode,
                                             double *__restrict__ qn, T *__restrict__ acc, T *qs_out,
-                                            double dt) {
+                                            double dt, Lines &ln) {
   constexpr bool FIRST = DIR == 2, LAST = DIR == 0;
   const double *__restrict__ q = *q0p;
-  __shared__ LineLds<T> lds;
   const long B = tp.base, PS = g.PS;
   const T ih = T(inv_h), gam = T(gamma), gm1 = T(gamma - 1.0), ggm = T(gamma / (gamma - 1.0));
   T ud[PPT], irho[PPT], S[PPT], R5[PPT], f[PPT], x[PPT], r[PPT];
@@ -88,11 +87,11 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
       }
     }
     // P = D p
-    line_solve<T, PER>(op, lds, tp, f, x);
+    ln.solve(op, f, x);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) S[m] = qs5[m] * irho[m] * (x[m] * ih);
     // E = D qs5
-    line_solve<T, PER>(op, lds, tp, qs5, x);
+    ln.solve(op, qs5, x);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       const T E = x[m] * ih;
@@ -102,7 +101,7 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
     }
   }
   // F = D(-u_d qs5)
-  line_solve<T, PER>(op, lds, tp, f, x);
+  ln.solve(op, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) R5[m] = R5[m] + gm1 * (x[m] * ih);
   // B_d = D qs_{d+2} completes r5 (the fences keep each group of loads next
@@ -113,7 +112,7 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
   {
     asm volatile("" ::: "memory");
     ld<DIR>(qs + (1 + DIR) * N, B, PS, f);
-    line_solve<T, PER>(op, lds, tp, f, x);
+    ln.solve(op, f, x);
     asm volatile("" ::: "memory");
     if (!FIRST) ld<DIR>(rhs + 4 * N, B, PS, r);
 #pragma unroll
@@ -131,7 +130,7 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
   __shared__ T stash[PPT][NT];
   asm volatile("" ::: "memory");
   ld<DIR>(qs, B, PS, f);
-  line_solve<T, PER>(op, lds, tp, f, x);
+  ln.solve(op, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) stash[m][threadIdx.x] = Ta[m] + x[m] * ih;
   // B_m = D qs_{m+2}, m != d
@@ -141,7 +140,7 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
     T um[PPT];
     asm volatile("" ::: "memory");
     ld<DIR>(qs + (1 + i) * N, B, PS, f);
-    line_solve<T, PER>(op, lds, tp, f, x);
+    ln.solve(op, f, x);
     asm volatile("" ::: "memory");
     ld<DIR>(q + (1 + i) * N, B, PS, um);
     if (!FIRST) ld<DIR>(rhs + (1 + i) * N, B, PS, r);
@@ -171,11 +170,12 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
 template <typename T, typename Q, int DIR, bool PER>
 __global__ __launch_bounds__(NT) void k_asweep(const Q *qs, const double *const *__restrict__ q0p,
                                                T *__restrict__ rhs, const double *__restrict__ gobj,
-                                               LineOp<T> op, SweepGeom g, double gamma, double inv_h, long N,
+                                               Op<T> op, SweepGeom g, double gamma, double inv_h, long N,
                                                int mode, double *__restrict__ qn, T *__restrict__ acc,
                                                T *qs_out, double dt) {
-  asweep_body<T, Q, DIR, PER>(thread_pos<DIR>(g), qs, q0p, rhs, gobj, op, g, gamma, inv_h, N, mode, qn, acc, qs_out,
-                              dt);
+  const ThreadPos tp = thread_pos<DIR>(g);
+  auto ln = make_lines<T, PER>(op, tp);
+  asweep_body<T, Q, DIR>(tp, qs, q0p, rhs, gobj, op, g, gamma, inv_h, N, mode, qn, acc, qs_out, dt, ln);
 }
 
 // characteristic_qs_k1d (src/boundaries/nonreflecting.f90:453-554) on the
@@ -282,39 +282,6 @@ __global__ __launch_bounds__(256) void k_bc_sponge_qs(Q *__restrict__ qs,
     const double x = double(qs[v * N + o]);
     qs[v * N + o] = Q(x - s * x);
   }
-}
-
-// The forward state of the next backward step: the step counter *ntp (set
-// by the host before the loop) selects trajectory slot nt (or the only slot
-// of a one-slot trajectory), then counts down.  One thread writes.
-__global__ void k_adjoint_slot(const double **q0p, int *ntp, const double *traj, long stride,
-                               int nslots) {
-  if (threadIdx.x != 0) return;
-  const int nt = *ntp;
-  q0p[0] = traj + (long)(nslots > 1 ? nt - 1 : 0) * stride;
-  ntp[0] = nt - 1;
-}
-
-// Subset checkpoints inside a recorded period: the subset counter *sp
-// (device cell) names the checkpoint to restore; every thread copies its
-// share of that state into q (grid-stride, 16-byte pairs; the stride of a
-// state, 5 N, is even or handled by the tail thread).
-__global__ __launch_bounds__(256) void k_restore_ckpt(double *__restrict__ q, const double *__restrict__ ckpt,
-                                                      const int *__restrict__ sp, long M) {
-  const int s = *sp;
-  const double *src = ckpt + (long)s * M;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < M; i += (long)gridDim.x * 256) q[i] = src[i];
-}
-
-// Set an int cell (counter) from the stream, so that a recorded graph can
-// reset it without a memset node.
-__global__ void k_set_int(int *p, int v, int delta) {
-  if (threadIdx.x == 0) p[0] = v == INT_MIN ? p[0] + delta : v;
-}
-
-// Point the forward-state cell at a given state.  One thread writes.
-__global__ void k_set_state_ptr(const double **q0p, const double *q) {
-  if (threadIdx.x == 0) q0p[0] = q;
 }
 
 }  // namespace cruna

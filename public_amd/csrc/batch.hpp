@@ -30,7 +30,7 @@ struct BatchMember {
   const double *traj;               // forward trajectory slots
   const double *ckpt;               // subset checkpoints
   int traj_slots;
-  LineOp<double> op[3], fop[3];
+  RecOp op[3], fop[3];
   SweepGeom geom[3], fgeom[3];
   Phys ph;
   long N;
@@ -63,9 +63,9 @@ __global__ __launch_bounds__(NT) void kb_sweep1(const BatchMember *__restrict__ 
   const int e = batch_entry(L);
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.geom[DIR], blockIdx.x - L->start[e]);
-  __shared__ LineLds<double> lds;
-  sweep1_body<double, double, DIR, PER, RHS_CART>(tp, from_qs ? b.qs : b.qn, b.rhs, b.G, b.op[DIR], b.geom[DIR],
-                                                  b.ph, b.N, Metric<double>{}, Penal<double>{}, lds);
+  auto ln = make_lines<double, PER>(b.op[DIR], tp);
+  sweep1_body<double, double, DIR, RHS_CART>(tp, from_qs ? b.qs : b.qn, b.rhs, b.G, b.op[DIR], b.geom[DIR], b.ph, b.N,
+                                             Metric<double>{}, Penal<double>{}, ln);
 }
 
 // viscous sweep; the x sweep finishes RK4 stage `mode` (FF: the last stage
@@ -76,9 +76,9 @@ __global__ __launch_bounds__(NT) void kb_sweep2(const BatchMember *__restrict__ 
   const int e = batch_entry(L);
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.geom[DIR], blockIdx.x - L->start[e]);
-  sweep2_body<double, DIR, PER, RHS_CART, FF>(tp, b.rhs, b.G, b.op[DIR], b.fop[DIR], b.geom[DIR], b.ph, b.N, mode,
-                                               b.qn, b.acc, b.qs, b.dt, Metric<double>{}, nullptr,
-                                               Penal<double>{});
+  auto ln = make_lines<double, PER>(b.op[DIR], tp);
+  sweep2_body<double, DIR, RHS_CART, FF>(tp, b.rhs, b.G, b.op[DIR], b.fop[DIR], b.geom[DIR], b.ph, b.N, mode, b.qn,
+                                         b.acc, b.qs, b.dt, Metric<double>{}, nullptr, Penal<double>{}, ln);
 }
 
 // the z first-derivative and viscous sweeps as one kernel (k_sweep12_z)
@@ -88,13 +88,12 @@ __global__ __launch_bounds__(NT) void kb_sweep12_z(const BatchMember *__restrict
   const int e = batch_entry(L);
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<2, true>(b.geom[2], blockIdx.x - L->start[e]);
-  __shared__ LineLds<double> lds;
-  __shared__ double mom[3][PPT][NT];
+  auto ln = make_lines<double, PER>(b.op[2], tp);
   ZCarry<double> zc;
-  zc.mom = mom;
-  sweep1_body<double, double, 2, PER, RHS_CART, true>(tp, from_qs ? b.qs : b.qn, b.rhs, b.G, b.op[2], b.geom[2],
-                                                      b.ph, b.N, Metric<double>{}, Penal<double>{}, lds, &zc);
-  viscous_z_carry<double, PER>(tp, b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N, lds, zc);
+  z_carry_slots(zc);
+  sweep1_body<double, double, 2, RHS_CART, true>(tp, from_qs ? b.qs : b.qn, b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N,
+                                                 Metric<double>{}, Penal<double>{}, ln, &zc);
+  viscous_z_carry<double>(tp, b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N, ln, zc);
 }
 
 // filter of the direct (adj = 0) or adjoint state in place
@@ -105,7 +104,8 @@ __global__ __launch_bounds__(NT) void kb_filter(const BatchMember *__restrict__ 
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.fgeom[DIR], blockIdx.x - L->start[e]);
   double *q = adj ? b.qa : b.qn;
-  filter_body<double, DIR, PER, double>(tp, q, q, b.fop[DIR], b.fgeom[DIR], b.N, 5, (double *)nullptr);
+  auto ln = make_lines<double, PER>(b.fop[DIR], tp);
+  filter_body<double, DIR, double>(tp, q, q, b.fop[DIR], b.fgeom[DIR], b.N, 5, (double *)nullptr, ln);
 }
 
 // adjoint sweep (backward in time: dt -> -dt); stage input qs^n (from_qs = 0) or qs
@@ -115,9 +115,9 @@ __global__ __launch_bounds__(NT) void kb_asweep(const BatchMember *__restrict__ 
   const int e = batch_entry(L);
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.geom[DIR], blockIdx.x - L->start[e]);
-  asweep_body<double, double, DIR, PER>(tp, from_qs ? b.qs : b.qa, (const double *const *)b.q0p, b.rhs, nullptr,
-                                        b.op[DIR], b.geom[DIR], b.gamma, b.ph.inv_h[DIR], b.N, mode, b.qa, b.acc,
-                                        b.qs, -b.dt);
+  auto ln = make_lines<double, PER>(b.op[DIR], tp);
+  asweep_body<double, double, DIR>(tp, from_qs ? b.qs : b.qa, (const double *const *)b.q0p, b.rhs, nullptr, b.op[DIR],
+                                   b.geom[DIR], b.gamma, b.ph.inv_h[DIR], b.N, mode, b.qa, b.acc, b.qs, -b.dt, ln);
 }
 
 // Per-member bookkeeping of a batched step, one work-group row per member

@@ -14,14 +14,27 @@
 #include <vector>
 
 #include "line_ops.hpp"
+#include "line_rec.hpp"
 #include "boundary.hpp"
 #include "sweeps.hpp"
 #include "curvilinear.hpp"
 #include "weighted_filter.hpp"
 #include "adjoint.hpp"
+#include "counters.hpp"
 #include "closure.hpp"
 #include "residual.hpp"
 #include "batch.hpp"
+#include "instances.hpp"
+
+// defined in sweeps_*.hip
+INST_GROUP_PERIODIC64(extern)
+INST_GROUP_OPEN64(extern)
+INST_GROUP_CURV64(extern)
+INST_GROUP_CURV64O(extern)
+INST_GROUP_FP32(extern)
+INST_GROUP_FP32B(extern)
+INST_GROUP_CURV32(extern)
+INST_GROUP_ADJOINT(extern)
 
 using namespace cruna;
 
@@ -52,8 +65,10 @@ const char *kKernelNames[KID_COUNT] = {"sweep1_x", "sweep1_y",    "sweep1_z", "s
                                        "filter_z", "diff",        "asweep_x_rk", "asweep_y",
                                        "asweep_z", "closure",     "sweep12_z"};
 
+// Line operators on the device: the block tables of the cyclic reduction
+// (FP32, and FP64 filters that the recursions do not take) ...
 template <typename T>
-struct DevOp {
+struct BlockOp {
   T *buf = nullptr;
   LineOp<T> op{};
   int upload(const HostLineOp &h) {
@@ -85,6 +100,25 @@ struct DevOp {
     buf = nullptr;
   }
 };
+// ... and the FP64 recursions (line_rec.hpp)
+struct RecursionOp {
+  double *buf = nullptr;  // ends of an open line
+  RecOp op{};
+  bool rec = false;       // the recursion engine takes this operator
+  int upload(const HostRecOp &h) {
+    rec = h.usable;
+    op = h.op;
+    if (h.tab.empty()) return CRUNA_HIP_OK;
+    HIP_TRY(hipMalloc(&buf, h.tab.size() * sizeof(double)));
+    HIP_TRY(hipMemcpy(buf, h.tab.data(), h.tab.size() * sizeof(double), hipMemcpyHostToDevice));
+    op.tab = buf;
+    return CRUNA_HIP_OK;
+  }
+  void release() {
+    if (buf) (void)hipFree(buf);
+    buf = nullptr;
+  }
+};
 
 }  // namespace
 
@@ -107,8 +141,9 @@ struct cruna_hip_ctx {
   int fwg[3] = {0, 0, 0};
   SweepGeom sgeom[3]{};  // Cartesian viscous sweeps (FP32: up to 32 y/z lines per work-group)
   int swg[3] = {0, 0, 0};
-  DevOp<double> dop64[3], fop64[3];
-  DevOp<float> dop32[3], fop32[3];
+  RecursionOp dop64[3], fop64[3];
+  BlockOp<float> dop32[3], fop32[3];
+  BlockOp<double> fcr64[3];  // FP64 filters that the recursions do not take
   Phys phys{};
   // device state
   double *qn = nullptr, *acc = nullptr, *qref = nullptr, *shape = nullptr, *tmp = nullptr;
@@ -312,31 +347,31 @@ int check_launch() {
 #define DISPATCH_DIR(c, d, KER, TARGS, ...)                                                 \
   do {                                                                                      \
     const dim3 grid_((c)->geom[d].ntiles), block_((c)->wg[d]);                              \
+    const size_t lds_ = line_lds_bytes<TARGS>((c)->wg[d]);                                  \
     const bool per_ = (c)->cfg.scheme[d] == CRUNA_HIP_PERIODIC;                            \
     if (d == 0) {                                                                           \
-      if (per_) hipLaunchKernelGGL((KER<TARGS, 0, true>), grid_, block_, 0, (c)->stream, __VA_ARGS__); \
-      else hipLaunchKernelGGL((KER<TARGS, 0, false>), grid_, block_, 0, (c)->stream, __VA_ARGS__);     \
+      if (per_) hipLaunchKernelGGL((KER<TARGS, 0, true>), grid_, block_, lds_, (c)->stream, __VA_ARGS__); \
+      else hipLaunchKernelGGL((KER<TARGS, 0, false>), grid_, block_, lds_, (c)->stream, __VA_ARGS__);     \
     } else if (d == 1) {                                                                    \
-      if (per_) hipLaunchKernelGGL((KER<TARGS, 1, true>), grid_, block_, 0, (c)->stream, __VA_ARGS__); \
-      else hipLaunchKernelGGL((KER<TARGS, 1, false>), grid_, block_, 0, (c)->stream, __VA_ARGS__);     \
+      if (per_) hipLaunchKernelGGL((KER<TARGS, 1, true>), grid_, block_, lds_, (c)->stream, __VA_ARGS__); \
+      else hipLaunchKernelGGL((KER<TARGS, 1, false>), grid_, block_, lds_, (c)->stream, __VA_ARGS__);     \
     } else {                                                                                \
-      if (per_) hipLaunchKernelGGL((KER<TARGS, 2, true>), grid_, block_, 0, (c)->stream, __VA_ARGS__); \
-      else hipLaunchKernelGGL((KER<TARGS, 2, false>), grid_, block_, 0, (c)->stream, __VA_ARGS__);     \
+      if (per_) hipLaunchKernelGGL((KER<TARGS, 2, true>), grid_, block_, lds_, (c)->stream, __VA_ARGS__); \
+      else hipLaunchKernelGGL((KER<TARGS, 2, false>), grid_, block_, lds_, (c)->stream, __VA_ARGS__);     \
     }                                                                                       \
   } while (0)
 
+// derivative and filter operators in the precision T
 template <typename T>
-DevOp<T> *dops(cruna_hip_ctx *c);
-template <>
-DevOp<double> *dops<double>(cruna_hip_ctx *c) { return c->dop64; }
-template <>
-DevOp<float> *dops<float>(cruna_hip_ctx *c) { return c->dop32; }
+auto *dops(cruna_hip_ctx *c) {
+  if constexpr (sizeof(T) == 8) return c->dop64;
+  else return c->dop32;
+}
 template <typename T>
-DevOp<T> *fops(cruna_hip_ctx *c);
-template <>
-DevOp<double> *fops<double>(cruna_hip_ctx *c) { return c->fop64; }
-template <>
-DevOp<float> *fops<float>(cruna_hip_ctx *c) { return c->fop32; }
+auto *fops(cruna_hip_ctx *c) {
+  if constexpr (sizeof(T) == 8) return c->fop64;
+  else return c->fop32;
+}
 
 template <typename T>
 Metric<T> metric(cruna_hip_ctx *c);
@@ -519,33 +554,35 @@ int closure_term(cruna_hip_ctx *c, const Q *in);
 template <typename T, typename Q, int DIR, int FORM>
 void launch_sweep1_form(cruna_hip_ctx *c, const Q *in) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
+  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
   T *rhs = (T *)c->rhs, *G = (T *)c->G;
-  const LineOp<T> &op = dops<T>(c)[DIR].op;
+  const Op<T> &op = dops<T>(c)[DIR].op;
   if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC)
-    hipLaunchKernelGGL((k_sweep1<T, Q, DIR, true, FORM>), grid, block, 0, c->stream, in, rhs, G, op,
+    hipLaunchKernelGGL((k_sweep1<T, Q, DIR, true, FORM>), grid, block, lds, c->stream, in, rhs, G, op,
                        c->geom[DIR], c->phys, c->N, metric<T>(c), penal<T>(c));
   else
-    hipLaunchKernelGGL((k_sweep1<T, Q, DIR, false, FORM>), grid, block, 0, c->stream, in, rhs, G, op,
+    hipLaunchKernelGGL((k_sweep1<T, Q, DIR, false, FORM>), grid, block, lds, c->stream, in, rhs, G, op,
                        c->geom[DIR], c->phys, c->N, metric<T>(c), penal<T>(c));
 }
 
 template <typename T, typename Q, int DIR>
 void launch_curv_sweep1(cruna_hip_ctx *c, const Q *in) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
+  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
   T *rhs = (T *)c->rhs, *G = (T *)c->G, *TG = (T *)c->tg;
-  const LineOp<T> &op = dops<T>(c)[DIR].op;
+  const Op<T> &op = dops<T>(c)[DIR].op;
   const bool per = c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC;
   if (per && c->ev)
-    hipLaunchKernelGGL((k_curv_sweep1<T, Q, DIR, true, true>), grid, block, 0, c->stream, in, rhs, G, TG, op,
+    hipLaunchKernelGGL((k_curv_sweep1<T, Q, DIR, true, true>), grid, block, lds, c->stream, in, rhs, G, TG, op,
                        c->geom[DIR], c->phys, c->N, curv_metric<T>(c), penal<T>(c));
   else if (per)
-    hipLaunchKernelGGL((k_curv_sweep1<T, Q, DIR, true, false>), grid, block, 0, c->stream, in, rhs, G, TG, op,
+    hipLaunchKernelGGL((k_curv_sweep1<T, Q, DIR, true, false>), grid, block, lds, c->stream, in, rhs, G, TG, op,
                        c->geom[DIR], c->phys, c->N, curv_metric<T>(c), penal<T>(c));
   else if (c->ev)
-    hipLaunchKernelGGL((k_curv_sweep1<T, Q, DIR, false, true>), grid, block, 0, c->stream, in, rhs, G, TG, op,
+    hipLaunchKernelGGL((k_curv_sweep1<T, Q, DIR, false, true>), grid, block, lds, c->stream, in, rhs, G, TG, op,
                        c->geom[DIR], c->phys, c->N, curv_metric<T>(c), penal<T>(c));
   else
-    hipLaunchKernelGGL((k_curv_sweep1<T, Q, DIR, false, false>), grid, block, 0, c->stream, in, rhs, G, TG, op,
+    hipLaunchKernelGGL((k_curv_sweep1<T, Q, DIR, false, false>), grid, block, lds, c->stream, in, rhs, G, TG, op,
                        c->geom[DIR], c->phys, c->N, curv_metric<T>(c), penal<T>(c));
 }
 
@@ -554,13 +591,14 @@ void launch_curv_sweep1(cruna_hip_ctx *c, const Q *in) {
 template <typename T, typename Q, int FORM>
 void launch_sweep12z_form(cruna_hip_ctx *c, const Q *in) {
   const dim3 grid(c->geom[2].ntiles), block(c->wg[2]);
+  const size_t lds = z_lds_bytes<T>(c->wg[2], FORM == RHS_CART);
   T *rhs = (T *)c->rhs, *G = (T *)c->G;
-  const LineOp<T> &op = dops<T>(c)[2].op;
+  const Op<T> &op = dops<T>(c)[2].op;
   if (c->cfg.scheme[2] == CRUNA_HIP_PERIODIC)
-    hipLaunchKernelGGL((k_sweep12_z<T, Q, true, FORM>), grid, block, 0, c->stream, in, rhs, G, op, c->geom[2],
+    hipLaunchKernelGGL((k_sweep12_z<T, Q, true, FORM>), grid, block, lds, c->stream, in, rhs, G, op, c->geom[2],
                        c->phys, c->N, metric<T>(c), penal<T>(c));
   else
-    hipLaunchKernelGGL((k_sweep12_z<T, Q, false, FORM>), grid, block, 0, c->stream, in, rhs, G, op, c->geom[2],
+    hipLaunchKernelGGL((k_sweep12_z<T, Q, false, FORM>), grid, block, lds, c->stream, in, rhs, G, op, c->geom[2],
                        c->phys, c->N, metric<T>(c), penal<T>(c));
 }
 
@@ -579,45 +617,48 @@ int launch_sweep12z(cruna_hip_ctx *c, const Q *in) {
 template <typename T, typename Q, int DIR>
 int launch_sweep1(cruna_hip_ctx *c, const Q *in) {
   ProfScope p(c, DIR == 0 ? KID_S1X : (DIR == 1 ? KID_S2Y : KID_S3Z));
-  if (c->curv)
+  if (c->curv) {
     launch_curv_sweep1<T, Q, DIR>(c, in);
-  else if (c->gt)
-    launch_sweep1_form<T, Q, DIR, RHS_GT>(c, in);
-  else if (c->ev)
-    launch_sweep1_form<T, Q, DIR, RHS_EV>(c, in);
-  else
-    launch_sweep1_form<T, Q, DIR, RHS_CART>(c, in);
+  } else if constexpr (DIR != 2) {  // z: launch_sweep12z
+    if (c->gt)
+      launch_sweep1_form<T, Q, DIR, RHS_GT>(c, in);
+    else if (c->ev)
+      launch_sweep1_form<T, Q, DIR, RHS_EV>(c, in);
+    else
+      launch_sweep1_form<T, Q, DIR, RHS_CART>(c, in);
+  }
   return check_launch();
 }
 
 template <typename T, int DIR, int FORM>
 void launch_sweep2_form(cruna_hip_ctx *c, int mode, bool fuse_filter) {
   const dim3 grid(c->sgeom[DIR].ntiles), block(c->swg[DIR]);
+  const size_t lds = line_lds_bytes<T>(c->swg[DIR]);
   T *rhs = (T *)c->rhs, *qs = (T *)c->qs;
   const T *G = (const T *)c->G;
-  const LineOp<T> &op = dops<T>(c)[DIR].op, &fop = fops<T>(c)[DIR].op;
+  const Op<T> &op = dops<T>(c)[DIR].op, &fop = fops<T>(c)[DIR].op;
   const T *force = (const T *)(DIR == 0 && c->cnn ? c->force : nullptr);
   const bool per = c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC;
   // the fused x filter exists on the last stage of the x sweep only
   if constexpr (DIR == 0) {
     if (fuse_filter && mode == 3) {
       if (per)
-        hipLaunchKernelGGL((k_sweep2<T, DIR, true, FORM, true>), grid, block, 0, c->stream, rhs, G, op, fop,
+        hipLaunchKernelGGL((k_sweep2<T, DIR, true, FORM, true>), grid, block, lds, c->stream, rhs, G, op, fop,
                            c->sgeom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, qs, c->cfg.dt, metric<T>(c), force,
                            penal<T>(c));
       else
-        hipLaunchKernelGGL((k_sweep2<T, DIR, false, FORM, true>), grid, block, 0, c->stream, rhs, G, op, fop,
+        hipLaunchKernelGGL((k_sweep2<T, DIR, false, FORM, true>), grid, block, lds, c->stream, rhs, G, op, fop,
                            c->sgeom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, qs, c->cfg.dt, metric<T>(c), force,
                            penal<T>(c));
       return;
     }
   }
   if (per) {
-    hipLaunchKernelGGL((k_sweep2<T, DIR, true, FORM, false>), grid, block, 0, c->stream, rhs, G, op, fop,
+    hipLaunchKernelGGL((k_sweep2<T, DIR, true, FORM, false>), grid, block, lds, c->stream, rhs, G, op, fop,
                        c->sgeom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, qs, c->cfg.dt, metric<T>(c), force,
                            penal<T>(c));
   } else {
-    hipLaunchKernelGGL((k_sweep2<T, DIR, false, FORM, false>), grid, block, 0, c->stream, rhs, G, op, fop,
+    hipLaunchKernelGGL((k_sweep2<T, DIR, false, FORM, false>), grid, block, lds, c->stream, rhs, G, op, fop,
                        c->sgeom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, qs, c->cfg.dt, metric<T>(c), force,
                            penal<T>(c));
   }
@@ -626,14 +667,15 @@ void launch_sweep2_form(cruna_hip_ctx *c, int mode, bool fuse_filter) {
 template <typename T, int DIR, bool PER, bool FF>
 void launch_curv_sweep2_k(cruna_hip_ctx *c, int mode) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
+  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
   const T *force = (const T *)(DIR == 0 && c->cnn ? c->force : nullptr);
   if (c->ev)
-    hipLaunchKernelGGL((k_curv_sweep2<T, DIR, PER, FF, true>), grid, block, 0, c->stream, (T *)c->rhs,
+    hipLaunchKernelGGL((k_curv_sweep2<T, DIR, PER, FF, true>), grid, block, lds, c->stream, (T *)c->rhs,
                        (const T *)c->G, (const T *)c->tg, dops<T>(c)[DIR].op, fops<T>(c)[DIR].op,
                        c->geom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, (T *)c->qs, c->cfg.dt,
                        curv_metric<T>(c), force, penal<T>(c));
   else
-    hipLaunchKernelGGL((k_curv_sweep2<T, DIR, PER, FF, false>), grid, block, 0, c->stream, (T *)c->rhs,
+    hipLaunchKernelGGL((k_curv_sweep2<T, DIR, PER, FF, false>), grid, block, lds, c->stream, (T *)c->rhs,
                        (const T *)c->G, (const T *)c->tg, dops<T>(c)[DIR].op, fops<T>(c)[DIR].op,
                        c->geom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, (T *)c->qs, c->cfg.dt,
                        curv_metric<T>(c), force, penal<T>(c));
@@ -661,14 +703,16 @@ void launch_curv_sweep2(cruna_hip_ctx *c, int mode, bool fuse_filter) {
 template <typename T, int DIR>
 int launch_sweep2(cruna_hip_ctx *c, int mode, bool fuse_filter) {
   ProfScope p(c, DIR == 2 ? KID_S4Z : (DIR == 1 ? KID_S5Y : KID_S6X));
-  if (c->curv)
+  if (c->curv) {
     launch_curv_sweep2<T, DIR>(c, mode, fuse_filter);
-  else if (c->gt)
-    launch_sweep2_form<T, DIR, RHS_GT>(c, mode, fuse_filter);
-  else if (c->ev)
-    launch_sweep2_form<T, DIR, RHS_EV>(c, mode, fuse_filter);
-  else
-    launch_sweep2_form<T, DIR, RHS_CART>(c, mode, fuse_filter);
+  } else if constexpr (DIR != 2) {  // z: launch_sweep12z
+    if (c->gt)
+      launch_sweep2_form<T, DIR, RHS_GT>(c, mode, fuse_filter);
+    else if (c->ev)
+      launch_sweep2_form<T, DIR, RHS_EV>(c, mode, fuse_filter);
+    else
+      launch_sweep2_form<T, DIR, RHS_CART>(c, mode, fuse_filter);
+  }
   return check_launch();
 }
 
@@ -735,12 +779,24 @@ int rk4_step(cruna_hip_ctx *c, bool fuse_filter = false) {
 template <typename T, int DIR, typename S>
 void launch_filter(cruna_hip_ctx *c, const S *src, double *q64, int nv, T *copy) {
   const dim3 grid(c->fgeom[DIR].ntiles), block(c->fwg[DIR]);
-  const LineOp<T> &op = fops<T>(c)[DIR].op;
-  if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC)
-    hipLaunchKernelGGL((k_filter<T, DIR, true, S>), grid, block, 0, c->stream, src, q64, op, c->fgeom[DIR],
+  const bool per = c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC;
+  if constexpr (sizeof(T) == 8) {
+    if (!c->fop64[DIR].rec) {
+      const LineOp<double> &op = c->fcr64[DIR].op;
+      if (per)
+        hipLaunchKernelGGL((k_filter_cr<DIR, true>), grid, block, 0, c->stream, src, q64, op, c->fgeom[DIR], c->N, nv);
+      else
+        hipLaunchKernelGGL((k_filter_cr<DIR, false>), grid, block, 0, c->stream, src, q64, op, c->fgeom[DIR], c->N, nv);
+      return;
+    }
+  }
+  const size_t lds = line_lds_bytes<T>(c->fwg[DIR]);
+  const Op<T> &op = fops<T>(c)[DIR].op;
+  if (per)
+    hipLaunchKernelGGL((k_filter<T, DIR, true, S>), grid, block, lds, c->stream, src, q64, op, c->fgeom[DIR],
                        c->N, nv, copy);
   else
-    hipLaunchKernelGGL((k_filter<T, DIR, false, S>), grid, block, 0, c->stream, src, q64, op, c->fgeom[DIR],
+    hipLaunchKernelGGL((k_filter<T, DIR, false, S>), grid, block, lds, c->stream, src, q64, op, c->fgeom[DIR],
                        c->N, nv, copy);
 }
 
@@ -797,7 +853,7 @@ int step_once(cruna_hip_ctx *c, int nt, bool weighted = true, bool *converged = 
   // come between them (or the residual needs the unfiltered new state);
   // then it runs inside the update's x sweep
   const bool fuse_fx = !check && !c->has_bcq && !c->has_bclate && c->cfg.filter_freq[0] > 0 &&
-                       nt % c->cfg.filter_freq[0] == 0;
+                       nt % c->cfg.filter_freq[0] == 0 && (mixed || c->fop64[0].rec);
   int rc = mixed ? rk4_step<float>(c, fuse_fx) : rk4_step<double>(c, fuse_fx);
   if (rc) return rc;
   if (check) {
@@ -1002,15 +1058,16 @@ template <typename T, typename Q, int DIR>
 int launch_asweep(cruna_hip_ctx *c, const Q *in, const double *g, int mode) {
   ProfScope p(c, DIR == 0 ? KID_AX : (DIR == 1 ? KID_AY : KID_AZ));
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
+  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
   T *rhs = (T *)c->rhs, *qs = (T *)c->qs;
   const double dt = -c->cfg.dt;  // backward in time (rk_o4_e.f90:62-105)
   if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC)
-    hipLaunchKernelGGL((k_asweep<T, Q, DIR, true>), grid, block, 0, c->stream, in,
+    hipLaunchKernelGGL((k_asweep<T, Q, DIR, true>), grid, block, lds, c->stream, in,
                        (const double *const *)c->q0p, rhs, g,
                        dops<T>(c)[DIR].op, c->geom[DIR], c->cfg.gamma, c->phys.inv_h[DIR], c->N,
                        mode, c->qa, (T *)c->acc, qs, dt);
   else
-    hipLaunchKernelGGL((k_asweep<T, Q, DIR, false>), grid, block, 0, c->stream, in,
+    hipLaunchKernelGGL((k_asweep<T, Q, DIR, false>), grid, block, lds, c->stream, in,
                        (const double *const *)c->q0p, rhs, g,
                        dops<T>(c)[DIR].op, c->geom[DIR], c->cfg.gamma, c->phys.inv_h[DIR], c->N,
                        mode, c->qa, (T *)c->acc, qs, dt);
@@ -1327,8 +1384,11 @@ int cruna_hip_create(const cruna_hip_cfg *cfg, cruna_hip_ctx **out) {
       HostLineOp dd = build_line_op(dk, cfg->scheme[d] == CRUNA_HIP_PERIODIC, cfg->n[d], 0.0);
       HostLineOp ff =
           build_line_op(OP_FILTER, cfg->scheme[d] == CRUNA_HIP_PERIODIC, cfg->n[d], cfg->filter_alpha);
-      if (int rc = c->dop64[d].upload(dd)) return rc;
-      if (int rc = c->fop64[d].upload(ff)) return rc;
+      const bool per = cfg->scheme[d] == CRUNA_HIP_PERIODIC;
+      if (int rc = c->dop64[d].upload(build_rec_op(dk, per, cfg->n[d], 0.0))) return rc;
+      if (int rc = c->fop64[d].upload(build_rec_op(OP_FILTER, per, cfg->n[d], cfg->filter_alpha))) return rc;
+      if (!c->fop64[d].rec)
+        if (int rc = c->fcr64[d].upload(ff)) return rc;
       if (int rc = c->dop32[d].upload(dd)) return rc;
       if (int rc = c->fop32[d].upload(ff)) return rc;
     } catch (const std::exception &e) {
@@ -1379,6 +1439,7 @@ int cruna_hip_destroy(cruna_hip_ctx *c) {
   for (int d = 0; d < 3; ++d) {
     c->dop64[d].release();
     c->fop64[d].release();
+    c->fcr64[d].release();
     c->dop32[d].release();
     c->fop32[d].release();
   }
@@ -2175,7 +2236,7 @@ int batch_period(const cruna_hip_ensemble *e, int nsteps) {
     for (int d = 0; d < 3; ++d) {
       if (c->cfg.scheme[d] != c0->cfg.scheme[d] || c->cfg.wfilter_freq[d] > 0) return 0;
       const int f = c->cfg.filter_freq[d], f0 = c0->cfg.filter_freq[d];
-      if ((f > 1) || (f0 > 1) || ((f > 0) != (f0 > 0))) return 0;
+      if ((f > 1) || (f0 > 1) || ((f > 0) != (f0 > 0)) || !c->fop64[d].rec) return 0;
     }
     if (e->role[i] == CRUNA_HIP_ADJOINT) {
       const int si = e->subm[i] ? c->sub_steps : 0;
@@ -2315,40 +2376,42 @@ struct BatchSlot {
 
 // launch of a batched kernel over list (grp, kind, d) of the bin; nothing for
 // an empty list
-#define BATCH_LAUNCH(S, grp, kind, d, KER, ...)                                                          \
+#define BATCH_LAUNCH(S, grp, kind, d, LDS, KER, ...)                                                     \
   do {                                                                                                   \
     if ((S).bb().blocks[grp][kind][d] > 0)                                                               \
-      hipLaunchKernelGGL(KER, dim3((S).bb().blocks[grp][kind][d]), dim3((S).bb().wg[grp][kind][d]), 0,   \
-                         (S).s, (S).mem(), (S).list(grp, kind, d), __VA_ARGS__);                         \
+      hipLaunchKernelGGL(KER, dim3((S).bb().blocks[grp][kind][d]), dim3((S).bb().wg[grp][kind][d]),      \
+                         LDS((S).bb().wg[grp][kind][d]), (S).s, (S).mem(), (S).list(grp, kind, d),       \
+                         __VA_ARGS__);                                                                   \
   } while (0)
+inline size_t batch_z_lds(int threads) { return z_lds_bytes<double>(threads, true); }
 
 template <int DIR>
 void batch_sweep1(const BatchSlot &S, int from_qs) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, (kb_sweep1<DIR, true>), from_qs);
-  else BATCH_LAUNCH(S, 0, 0, DIR, (kb_sweep1<DIR, false>), from_qs);
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep1<DIR, true>), from_qs);
+  else BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep1<DIR, false>), from_qs);
 }
 
 void batch_sweep12z(const BatchSlot &S, int from_qs) {
-  if (S.e->bper[2]) BATCH_LAUNCH(S, 0, 0, 2, (kb_sweep12_z<true>), from_qs);
-  else BATCH_LAUNCH(S, 0, 0, 2, (kb_sweep12_z<false>), from_qs);
+  if (S.e->bper[2]) BATCH_LAUNCH(S, 0, 0, 2, batch_z_lds, (kb_sweep12_z<true>), from_qs);
+  else BATCH_LAUNCH(S, 0, 0, 2, batch_z_lds, (kb_sweep12_z<false>), from_qs);
 }
 
 template <int DIR, bool FF>
 void batch_sweep2(const BatchSlot &S, int mode) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, (kb_sweep2<DIR, true, FF>), mode);
-  else BATCH_LAUNCH(S, 0, 0, DIR, (kb_sweep2<DIR, false, FF>), mode);
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep2<DIR, true, FF>), mode);
+  else BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep2<DIR, false, FF>), mode);
 }
 
 template <int DIR>
 void batch_filter(const BatchSlot &S, int grp) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, grp, 1, DIR, (kb_filter<DIR, true>), grp);
-  else BATCH_LAUNCH(S, grp, 1, DIR, (kb_filter<DIR, false>), grp);
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, grp, 1, DIR, rec_lds_bytes, (kb_filter<DIR, true>), grp);
+  else BATCH_LAUNCH(S, grp, 1, DIR, rec_lds_bytes, (kb_filter<DIR, false>), grp);
 }
 
 template <int DIR>
 void batch_asweep(const BatchSlot &S, int mode, int from_qs) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 1, 0, DIR, (kb_asweep<DIR, true>), mode, from_qs);
-  else BATCH_LAUNCH(S, 1, 0, DIR, (kb_asweep<DIR, false>), mode, from_qs);
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 1, 0, DIR, rec_lds_bytes, (kb_asweep<DIR, true>), mode, from_qs);
+  else BATCH_LAUNCH(S, 1, 0, DIR, rec_lds_bytes, (kb_asweep<DIR, false>), mode, from_qs);
 }
 
 // One forward step of the bin's group 0 (step_once of each member: RK4 with

@@ -37,11 +37,11 @@ struct CurvMetric {
 template <typename T, typename Q, int DIR, bool PER, bool EV>
 __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T *__restrict__ rhs,
                                                     T *__restrict__ G, T *__restrict__ TG,
-                                                    LineOp<T> op, SweepGeom g, Phys ph, long N,
+                                                    Op<T> op, SweepGeom g, Phys ph, long N,
                                                     CurvMetric<T> mt, Penal<T> pe) {
   constexpr bool FIRST = DIR == 0;
-  __shared__ LineLds<T> lds;
   const ThreadPos tp = thread_pos<DIR>(g);
+  auto ln = make_lines<T, PER>(op, tp);
   const long B = tp.base, PS = g.PS;
   const T ih = T(ph.inv_h[DIR]);
   // In FP64, rho, and in the periodic x sweep the momenta, stay in
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
       const T c = i == 0 ? M0[m] : (i == 1 ? M1[m] : M2[m]);
       uh[m] = i == 0 ? c * ui[m] : uh[m] + c * ui[m];
     }
-    line_solve<T, PER>(op, lds, tp, ui, x);
+    ln.solve(op, ui, x);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) x[m] = x[m] * ih;
     T d[PPT];
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
     for (int m = 0; m < PPT; ++m) mu[m] = viscosity(ph, f[m]);
     st<DIR>(G + 6 * N, B, PS, mu);
   }
-  line_solve<T, PER>(op, lds, tp, f, x);
+  ln.solve(op, f, x);
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     T d[PPT];
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
   // pressure gradient along DIR: -M(DIR,i) a(p) in momentum i (:194 etc.),
   // u_hat a(p) in the pressure bracket
   T ap[PPT];
-  line_solve<T, PER>(op, lds, tp, p, ap);
+  ln.solve(op, p, ap);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) ap[m] = ap[m] * ih;
 
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
     if constexpr (!KEEPR) ld<DIR>(qs, B, PS, rho);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * rho[m]) * uh[m] : rho[m] * uh[m];
-    line_solve<T, PER>(op, lds, tp, f, x);
+    ln.solve(op, f, x);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) x[m] = div(m, -(x[m] * ih));
     acc(rhs, x);
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
     }
 #pragma unroll
     for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * mom[m]) * uh[m] : mom[m] * uh[m];
-    line_solve<T, PER>(op, lds, tp, f, x);
+    ln.solve(op, f, x);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       const T c = i == 0 ? M0[m] : (i == 1 ? M1[m] : M2[m]);
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
   // pressure bracket: gamma/(gamma-1) (-a(p u_hat)) + u_hat a(p) (:245-250)
 #pragma unroll
   for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * p[m]) * uh[m] : p[m] * uh[m];
-  line_solve<T, PER>(op, lds, tp, f, x);
+  ln.solve(op, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) x[m] = div(m, T(ph.gt) * (-(x[m] * ih))) + uh[m] * ap[m];
   acc(rhs + 4 * N, x);
@@ -194,16 +194,16 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
 
 template <typename T, int DIR, bool PER, bool FF, bool EV>
 __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T *__restrict__ G,
-                                                    const T *__restrict__ TG, LineOp<T> op,
-                                                    LineOp<T> fop, SweepGeom g, Phys ph, long N,
+                                                    const T *__restrict__ TG, Op<T> op,
+                                                    Op<T> fop, SweepGeom g, Phys ph, long N,
                                                     int mode, double *__restrict__ qn,
                                                     T *__restrict__ acc,
                                                     T *__restrict__ qs_out, double dt,
                                                     CurvMetric<T> mt, const T *__restrict__ force,
                                                     Penal<T> pe) {
   constexpr bool LAST = DIR == 0;
-  __shared__ LineLds<T> lds;
   const ThreadPos tp = thread_pos<DIR>(g);
+  auto ln = make_lines<T, PER>(op, tp);
   const long B = tp.base, PS = g.PS;
   const T ih = T(ph.inv_h[DIR]);
   T M0[PPT], M1[PPT], M2[PPT], mu[PPT];
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
       ld<DIR>(TG + j * N, B, PS, f);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) f[m] = lj[m] * f[m];
-      line_solve<T, PER>(op, lds, tp, f, x);
+      ln.solve(op, f, x);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) {
         const T c = j == 0 ? M0[m] : (j == 1 ? M1[m] : M2[m]);
@@ -310,7 +310,9 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
       T f[PPT], x[PPT];
 #pragma unroll
       for (int m = 0; m < PPT; ++m) f[m] = T(a[m]);
-      line_solve<T, PER>(fop, lds, tp, f, x);
+      ln.bind(fop);
+      ln.template solve<true>(fop, f, x);
+      ln.bind(op);
       st<DIR>(qn + v * N, B, PS, x);
     } else {
       rk_update<DIR, T>(mode, v, k, B, PS, N, rhs, qn, acc, qs_out, dt);
@@ -348,7 +350,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     T x[PPT];
-    line_solve<T, PER>(op, lds, tp, i == 0 ? t1 : (i == 1 ? t2 : t3), x);
+    ln.solve(op, i == 0 ? t1 : (i == 1 ? t2 : t3), x);
     asm volatile("" ::: "memory");
     T k[PPT];
     ld<DIR>(rhs + (1 + i) * N, B, PS, k);

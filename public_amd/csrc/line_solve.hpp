@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include "line_ops.hpp"
+#include "line_rec.hpp"
 
 namespace cruna {
 
@@ -314,6 +315,333 @@ __device__ __forceinline__ void line_solve(const LineOp<T> &op, LineLds<T, NTM> 
       }
     }
   }
+}
+
+// ----------------------------------------------------------------------------
+// FP64 engine (line_rec.hpp: the recursions, why and what they cost).
+
+// LDS of the engine: REC_STRIDE doubles per thread (and a slot of zeros, what
+// lies beyond an open line), value k of slot t at t REC_STRIDE + k: the halo
+// values (2 H per field: two derivative fields with H = 2, or one filter field
+// with H = 3), then u_L and x_F of up to two fields.  Every solve of a kernel,
+// derivative or filter, keeps u_L and x_F in the same places: a value of one
+// solve is rewritten by the next only after a barrier that follows its last
+// read (halo: read before the second barrier, u_L before the third, x_F before
+// the next solve's first).  The odd stride spreads consecutive lanes over all
+// banks, and with the slots' addresses kept per thread every value is an
+// immediate offset away.  Dynamic LDS, so that a work-group takes what its own
+// size needs.
+constexpr int REC_STRIDE = 13, REC_HALO = 8, REC_UL = 8, REC_XF = 10;
+inline size_t rec_lds_bytes(int threads) { return (size_t)(threads + 1) * REC_STRIDE * sizeof(double); }
+
+template <typename T>
+struct OpOf {
+  typedef LineOp<T> type;
+};
+template <>
+struct OpOf<double> {
+  typedef RecOp type;
+};
+template <typename T>
+using Op = typename OpOf<T>::type;
+
+// The engine's arithmetic is written with explicit fused multiply-adds and
+// contracts nothing else (also not with the operands' own products), so that
+// a line gives the same bits in every kernel that it is inlined into.
+
+// The lines of a work-group: solve(op, f, x) is x = B^-1 A f on the thread's
+// block, solve2 two independent fields at once (all threads together, in the
+// same order).  CR: the cyclic reduction above; one field after the other.
+template <typename T, bool PER, int NTM>
+struct CrLines {
+  LineLds<T, NTM> &lds;
+  const ThreadPos &tp;
+  template <bool FILT = false>
+  __device__ __forceinline__ void solve(const LineOp<T> &op, const T (&f)[PPT], T (&x)[PPT]) {
+    line_solve<T, PER>(op, lds, tp, f, x);
+  }
+  __device__ __forceinline__ void solve2(const LineOp<T> &op, const T (&f1)[PPT], T (&x1)[PPT], const T (&f2)[PPT],
+                                         T (&x2)[PPT]) {
+    line_solve<T, PER>(op, lds, tp, f1, x1);
+    line_solve<T, PER>(op, lds, tp, f2, x2);
+  }
+  __device__ __forceinline__ void bind(const LineOp<T> &) {}
+};
+
+template <bool PER>
+struct RecLines {
+  char *lds;                   // dynamic LDS
+  int own;                     // byte offset of the thread's slot
+  int lf[REC_WIN], rt[REC_WIN];  // slots of blocks b-1, b-2, ... and b+1, b+2, ...
+  int b, NB, BS, line;         // block, blocks per line, slot stride of blocks, slot of block 0
+  int nthreads;
+  bool wave_line;
+  double pwl, pwr;             // open: mu^(8 b - pf), mu^(n-1 - (8 b - pf) - 7)
+
+  static constexpr int SLOT = REC_STRIDE * int(sizeof(double));
+  __device__ __forceinline__ double get(int slot, int cell) const {
+    return *reinterpret_cast<const double *>(lds + slot + cell * int(sizeof(double)));
+  }
+  __device__ __forceinline__ void put(int cell, double v) const {
+    *reinterpret_cast<double *>(lds + own + cell * int(sizeof(double))) = v;
+  }
+  // slot of block t of the thread's line, 0 <= t < NB
+  __device__ __forceinline__ int slot_of(int t) const { return (line + t * BS) * SLOT; }
+
+  __device__ __forceinline__ RecLines(char *mem, const RecOp &op, const ThreadPos &tp) : lds(mem) {
+    b = tp.b;
+    NB = op.NB;
+    BS = tp.BS;
+    line = tp.l * tp.LS;
+    nthreads = blockDim.x;
+    wave_line = tp.wave_line;
+    own = int(threadIdx.x) * SLOT;
+    const int zero = nthreads * SLOT;
+    int l = b, r = b;
+#pragma unroll
+    for (int m = 0; m < REC_WIN; ++m) {
+      --l;
+      ++r;
+      if (PER) {
+        l = l < 0 ? l + NB : l;
+        r = r >= NB ? r - NB : r;
+        lf[m] = slot_of(l);
+        rt[m] = slot_of(r);
+      } else {
+        lf[m] = l >= 0 ? slot_of(l) : zero;
+        rt[m] = r < NB ? slot_of(r) : zero;
+      }
+    }
+    if (!PER) {
+      for (int t = threadIdx.x; t < REC_STRIDE; t += nthreads)
+        *reinterpret_cast<double *>(lds + zero + t * int(sizeof(double))) = 0.0;
+      lds_barrier();
+      bind(op);
+    }
+  }
+  // the powers of mu of an open line's op (the constructor binds its own)
+  __device__ __forceinline__ void bind(const RecOp &op) {
+    if (!PER) {
+      pwl = op.tab[REC_PW + 2 * b];
+      pwr = op.tab[REC_PW + 2 * b + 1];
+    }
+  }
+  __device__ __forceinline__ void sync() const { line_sync(wave_line); }
+
+  // sum_m rho^m value(block b -+ (1 + m)) of cell
+  __device__ __forceinline__ double window(const RecOp &op, const int (&at)[REC_WIN], int dir, int cell) const {
+#pragma clang fp contract(off)
+    double v[REC_WIN];
+#pragma unroll
+    for (int m = 0; m < REC_WIN; ++m) v[m] = get(at[m], cell);
+    if (!op.slow) {
+      double s = v[REC_WIN - 1];
+#pragma unroll
+      for (int m = REC_WIN - 2; m >= 0; --m) s = __builtin_fma(s, op.rho, v[m]);
+      return s;
+    }
+    // slowly decaying filters: M terms, M at most the blocks of the line
+    double s = 0.0;
+    for (int m = op.M - 1; m >= 0; --m) {
+      int t = b + dir * (1 + m);
+      double u = 0.0;
+      if (PER) {
+        t = t < 0 ? t + NB : (t >= NB ? t - NB : t);
+        u = get(slot_of(t), cell);
+      } else if (t >= 0 && t < NB) {
+        u = get(slot_of(t), cell);
+      }
+      s = __builtin_fma(s, op.rho, u);
+    }
+    return s * op.norm;
+  }
+
+  template <int NF, bool FILT>
+  __device__ __forceinline__ void run(const RecOp &op, const double (&f)[NF][PPT], double (&x)[NF][PPT]) {
+#pragma clang fp contract(off)
+    constexpr int H = FILT ? 3 : 2, CELL = 2 * H;
+    static_assert(NF * CELL <= REC_HALO && NF <= 2, "the fields' halo cells");
+#pragma unroll
+    for (int v = 0; v < NF; ++v)
+#pragma unroll
+      for (int m = 0; m < H; ++m) {
+        put(v * CELL + m, f[v][m]);
+        put(v * CELL + H + m, f[v][PPT - H + m]);
+      }
+    sync();
+#pragma unroll
+    for (int v = 0; v < NF; ++v) {
+      double fe[PPT + 2 * H];
+#pragma unroll
+      for (int m = 0; m < H; ++m) {
+        fe[m] = get(lf[0], v * CELL + H + m);
+        fe[H + PPT + m] = get(rt[0], v * CELL + m);
+      }
+#pragma unroll
+      for (int i = 0; i < PPT; ++i) fe[H + i] = f[v][i];
+#pragma unroll
+      for (int i = 0; i < PPT; ++i) {
+        const double *e = fe + H + i;
+        if (FILT)
+          x[v][i] = __builtin_fma(op.s[0], e[0], __builtin_fma(op.s[1], e[1] + e[-1],
+                                                              __builtin_fma(op.s[2], e[2] + e[-2], op.s[3] * (e[H] + e[-H]))));
+        else
+          x[v][i] = __builtin_fma(op.s[1], e[1] - e[-1], op.s[2] * (e[2] - e[-2]));
+      }
+      if (!PER) {
+        // the closures' own rows and the padding of the two end blocks
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const bool mine = b == (e == 0 ? 0 : NB - 1);
+          if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
+#pragma unroll
+          for (int r = 0; r < PPT; ++r) {
+            if ((op.srow[e] >> r) & 1) {
+              const cptr<double> a = launder_uniform(op.tab + e * REC_END + r * FE + HALO - H);
+              double acc = 0.0;
+#pragma unroll
+              for (int j = 0; j < PPT + 2 * H; ++j) acc = __builtin_fma(a[j], fe[j], acc);
+              if (mine) x[v][r] = acc;
+            } else if ((op.zrow[e] >> r) & 1) {
+              if (mine) x[v][r] = 0.0;
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 1; i < PPT; ++i) x[v][i] = __builtin_fma(op.mu, x[v][i - 1], x[v][i]);
+      put(REC_UL + v, x[v][PPT - 1]);
+    }
+    sync();
+#pragma unroll
+    for (int v = 0; v < NF; ++v) {
+      const double U = window(op, lf, -1, REC_UL + v);
+#pragma unroll
+      for (int i = 0; i < PPT; ++i) x[v][i] = __builtin_fma(op.lp[i], U, x[v][i]);
+      if (!PER && op.zrow[1] != 0) {  // nothing comes back from behind the last point
+        const bool mine = b == NB - 1;
+        if (__builtin_amdgcn_ballot_w64(mine) != 0)
+#pragma unroll
+          for (int r = 0; r < PPT; ++r)
+            if (((op.zrow[1] >> r) & 1) && mine) x[v][r] = 0.0;
+      }
+#pragma unroll
+      for (int i = PPT - 2; i >= 0; --i) x[v][i] = __builtin_fma(op.mu, x[v][i + 1], x[v][i]);
+      put(REC_XF + v, x[v][0]);
+    }
+    sync();
+#pragma unroll
+    for (int v = 0; v < NF; ++v) {
+      const double X = window(op, rt, +1, REC_XF + v);
+#pragma unroll
+      for (int i = 0; i < PPT; ++i) x[v][i] = __builtin_fma(op.lp[PPT - 1 - i], X, x[v][i]);
+    }
+    if (!PER) ends<NF, FILT>(op, f, x);
+  }
+
+  // end corrections of an open line, then the padding rows
+  template <int NF, bool FILT>
+  __device__ __forceinline__ void ends(const RecOp &op, const double (&f)[NF][PPT], double (&x)[NF][PPT]) {
+#pragma clang fp contract(off)
+        const bool end[2] = {b == 0, b == NB - 1};
+    if (op.nend) {
+      double kap[NF];
+#pragma unroll
+      for (int v = 0; v < NF; ++v) kap[v] = 0.0;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        if (__builtin_amdgcn_ballot_w64(end[e]) == 0) continue;
+        const cptr<double> c = launder_uniform(op.tab + e * REC_END + PPT * FE);
+#pragma unroll
+        for (int v = 0; v < NF; ++v) {
+          double a = 0.0, k = 0.0;
+#pragma unroll
+          for (int r = 0; r < PPT; ++r) {
+            a = __builtin_fma(c[r], x[v][r], a);
+            k = __builtin_fma(c[PPT + r], x[v][r], k);
+          }
+          if (end[e]) {
+            put(REC_UL + v, a);  // u_L has been read (the exchange of x_F lies between)
+            kap[v] = k;
+          }
+        }
+      }
+      sync();
+      if (__builtin_amdgcn_ballot_w64(fabs(pwl) > 1e-19 || fabs(pwr) > 1e-19) != 0) {
+        const cptr<double> t = launder_uniform(op.tab + REC_SCAL);
+#pragma unroll
+        for (int v = 0; v < NF; ++v) {
+          const double al = get(line * SLOT, REC_UL + v), ar = get(slot_of(NB - 1), REC_UL + v);
+          const double sl = __builtin_fma(t[0], al, t[1] * ar), sr = __builtin_fma(t[2], ar, t[3] * al);
+          const double l = sl * pwl, r = sr * pwr;
+          x[v][0] += l;
+          x[v][PPT - 1] += r;
+#pragma unroll
+          for (int i = 1; i < PPT; ++i) {
+            x[v][i] = __builtin_fma(op.lp[i - 1], l, x[v][i]);
+            x[v][PPT - 1 - i] = __builtin_fma(op.lp[i - 1], r, x[v][PPT - 1 - i]);
+          }
+          const double k = __builtin_fma(end[0] ? t[4] : t[5], end[0] ? sr : sl, kap[v]);
+#pragma unroll
+          for (int r2 = 0; r2 < PPT; ++r2) {
+            if (r2 == op.rend[0] && end[0]) x[v][r2] += k;
+            if (r2 == op.rend[1] && end[1]) x[v][r2] += k;
+          }
+        }
+      }
+    }
+    if ((op.zrow[0] | op.zrow[1]) != 0) {
+#pragma unroll
+      for (int v = 0; v < NF; ++v)
+#pragma unroll
+        for (int r = 0; r < PPT; ++r)
+          if ((((op.zrow[0] >> r) & 1) && end[0]) || (((op.zrow[1] >> r) & 1) && end[1])) x[v][r] = FILT ? f[v][r] : 0.0;
+    }
+  }
+
+  template <bool FILT = false>
+  __device__ __forceinline__ void solve(const RecOp &op, const double (&f)[PPT], double (&x)[PPT]) {
+    double a[1][PPT], r[1][PPT];
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) a[0][i] = f[i];
+    run<1, FILT>(op, a, r);
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) x[i] = r[0][i];
+  }
+  __device__ __forceinline__ void solve2(const RecOp &op, const double (&f1)[PPT], double (&x1)[PPT],
+                                         const double (&f2)[PPT], double (&x2)[PPT]) {
+    double a[2][PPT], r[2][PPT];
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+      a[0][i] = f1[i];
+      a[1][i] = f2[i];
+    }
+    run<2, false>(op, a, r);
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+      x1[i] = r[0][i];
+      x2[i] = r[1][i];
+    }
+  }
+};
+
+// The engine of a kernel in precision T (NTM: the largest work-group of the
+// FP32 form's static LDS; FP64 launches pass rec_lds_bytes(threads))
+extern __shared__ __align__(16) char line_dyn[];
+
+template <typename T, bool PER, int NTM = NT>
+__device__ __forceinline__ auto make_lines(const Op<T> &op, const ThreadPos &tp) {
+  if constexpr (sizeof(T) == 8) {
+    return RecLines<PER>(line_dyn, op, tp);
+  } else {
+    __shared__ LineLds<T, NTM> lds;
+    return CrLines<T, PER, NTM>{lds, tp};
+  }
+}
+// bytes of dynamic LDS that the engine takes in a work-group of `threads`
+template <typename T>
+size_t line_lds_bytes(int threads) {
+  return sizeof(T) == 8 ? rec_lds_bytes(threads) : 0;
 }
 
 }  // namespace cruna

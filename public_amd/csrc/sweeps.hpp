@@ -229,17 +229,41 @@ constexpr int sweep_nt() { return sizeof(T) == 4 ? NT_SWEEP32 : NT; }
 // z sweep completes (s13 = u_z + w_x, s23 = v_z + w_y, w_z) and the
 // viscosity in registers; the momentum RHS of the block in LDS (the thread's
 // own slots) instead of a store and a reload through HBM.
+// In FP64 the slots are thread-major with a stride of 25 values (odd: no bank
+// conflicts) in the dynamic LDS behind the line engine's; in FP32 a static
+// array.
+constexpr int ZC_STRIDE = 3 * PPT + 1;
 template <typename T>
 struct ZCarry {
   T s13[PPT], s23[PPT], wz[PPT], mu[PPT];
-  T (*mom)[PPT][NT];  // LDS: [3][PPT][NT] momentum RHS (x, y, z)
+  T *slots;   // LDS: momentum RHS (x, y, z) of the block
+  int tid;
+  __device__ __forceinline__ T &mom(int i, int m) const {
+    return sizeof(T) == 8 ? slots[i * PPT + m] : slots[(i * PPT + m) * NT + tid];
+  }
 };
+template <typename T>
+__device__ __forceinline__ void z_carry_slots(ZCarry<T> &zc) {
+  zc.tid = threadIdx.x;
+  if constexpr (sizeof(T) == 8) {
+    zc.slots = reinterpret_cast<double *>(line_dyn) + (blockDim.x + 1) * REC_STRIDE + threadIdx.x * ZC_STRIDE;
+  } else {
+    __shared__ T mom[3 * PPT * NT];
+    zc.slots = mom;
+  }
+}
+// dynamic LDS of the fused z kernel in a work-group of `threads`
+template <typename T>
+size_t z_lds_bytes(int threads, bool carry) {
+  return line_lds_bytes<T>(threads) + (sizeof(T) == 8 && carry ? (size_t)threads * ZC_STRIDE * sizeof(double) : 0);
+}
 
-template <typename T, typename Q, int DIR, bool PER, int FORM, bool FUSE = false>
+
+template <typename T, typename Q, int DIR, int FORM, bool FUSE = false, typename Lines>
 __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__restrict__ qs, T *__restrict__ rhs,
-                                            T *__restrict__ G, const LineOp<T> &op, const SweepGeom &g,
+                                            T *__restrict__ G, const Op<T> &op, const SweepGeom &g,
                                             const Phys &ph, long N, const Metric<T> &mt, const Penal<T> &pe,
-                                            LineLds<T> &lds, ZCarry<T> *zc = nullptr) {
+                                            Lines &ln, ZCarry<T> *zc = nullptr) {
   constexpr bool GT = FORM == RHS_GT, EV = FORM == RHS_EV;
   static_assert(!FUSE || (DIR == 2 && FORM == RHS_CART), "the fused z sweep is Cartesian");
   const long B = tp.base, PS = g.PS;
@@ -263,7 +287,7 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
                     : (DIR == 1 ? (i == 0 ? 3 : (i == 1 ? 1 : 5)) : (i == 0 ? 4 : (i == 1 ? 5 : 2)));
   };
   auto gsum = [](int i) -> bool { return (DIR == 1 && i == 0) || (DIR == 2 && i < 2); };
-  T irho[PPT], mom[PPT], p[PPT], f[PPT], x[PPT], r[PPT];
+  T irho[PPT], mom[PPT], p[PPT], f[PPT], x[PPT], y[PPT], r[PPT];
   ld<DIR>(qs, B, PS, f);
   ld<DIR>(qs + (1 + DIR) * N, B, PS, mom);
 #pragma unroll
@@ -280,117 +304,105 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
     if (gsum(i)) ld<DIR>(G + gslot(i) * N, B, PS, gs);
     issue_loads();
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) ui[m] = ui[m] * irho[m];
-    line_solve<T, PER>(op, lds, tp, ui, x);
-#pragma unroll
     for (int m = 0; m < PPT; ++m) {
-      x[m] = x[m] * ih;
-      if (gsum(i)) x[m] = x[m] + gs[m];
-    }
-    st<DIR>(G + gslot(i) * N, B, PS, x);
-    if constexpr (FUSE) {
-#pragma unroll
-      for (int m = 0; m < PPT; ++m) (k == 0 ? zc->s13 : zc->s23)[m] = x[m];
+      ui[m] = ui[m] * irho[m];
+      f[m] = EV ? (PH[m] * mom[m]) * ui[m] : mom[m] * ui[m];
     }
     if (DIR != 0) ld<DIR>(rhs + (1 + i) * N, B, PS, r);
     if (k == 1) ld<DIR>(qs + 4 * N, B, PS, p);  // in flight for the pressure terms
+    ln.solve2(op, ui, y, f, x);
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * mom[m]) * ui[m] : mom[m] * ui[m];
-    line_solve<T, PER>(op, lds, tp, f, x);
+    for (int m = 0; m < PPT; ++m) {
+      y[m] = y[m] * ih;
+      if (gsum(i)) y[m] = y[m] + gs[m];
+    }
+    st<DIR>(G + gslot(i) * N, B, PS, y);
+    if constexpr (FUSE) {
+#pragma unroll
+      for (int m = 0; m < PPT; ++m) (k == 0 ? zc->s13 : zc->s23)[m] = y[m];
+    }
 #pragma unroll
     for (int m = 0; m < PPT; ++m) r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
     if constexpr (FUSE) {
 #pragma unroll
-      for (int m = 0; m < PPT; ++m) zc->mom[i][m][threadIdx.x] = r[m];
+      for (int m = 0; m < PPT; ++m) zc->mom(i, m) = r[m];
     } else {
       st<DIR>(rhs + (1 + i) * N, B, PS, r);
     }
   }
 
-  // d(u_DIR)/dx_DIR
+  // d(u_DIR)/dx_DIR, and mass: -d/dx_DIR (rho u_DIR) (:131-135)
   T ud[PPT];
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) ud[m] = mom[m] * irho[m];
-  line_solve<T, PER>(op, lds, tp, ud, x);
+  for (int m = 0; m < PPT; ++m) {
+    ud[m] = mom[m] * irho[m];
+    f[m] = EV ? PH[m] * mom[m] : mom[m];
+  }
+  if (DIR != 0) ld<DIR>(rhs, B, PS, r);
+  ln.solve2(op, ud, y, f, x);
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) x[m] = x[m] * ih;
-  st<DIR>(G + DIR * N, B, PS, x);
+  for (int m = 0; m < PPT; ++m) y[m] = y[m] * ih;
+  st<DIR>(G + DIR * N, B, PS, y);
   if constexpr (FUSE) {
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) zc->wz[m] = x[m];
-  }
-
-  // mass: -d/dx_DIR (rho u_DIR) (:131-135)
-  if (DIR != 0) ld<DIR>(rhs, B, PS, r);
-  if (EV) {
-#pragma unroll
-    for (int m = 0; m < PPT; ++m) f[m] = PH[m] * mom[m];
-    line_solve<T, PER>(op, lds, tp, f, x);
-  } else {
-    line_solve<T, PER>(op, lds, tp, mom, x);
+    for (int m = 0; m < PPT; ++m) zc->wz[m] = y[m];
   }
 #pragma unroll
   for (int m = 0; m < PPT; ++m) r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
   st<DIR>(rhs, B, PS, r);
 
-  // pressure gradient p_DIR
+  // pressure gradient p_DIR, and momentum DIR: -d/dx_DIR (rho u_DIR u_DIR) - p_DIR
   T pd[PPT];
-  line_solve<T, PER>(op, lds, tp, p, pd);
-#pragma unroll
-  for (int m = 0; m < PPT; ++m) pd[m] = pd[m] * ih;
-
-  // momentum DIR: -d/dx_DIR (rho u_DIR u_DIR) - p_DIR
   if (DIR != 0) ld<DIR>(rhs + (1 + DIR) * N, B, PS, r);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * mom[m]) * ud[m] : mom[m] * ud[m];
-  line_solve<T, PER>(op, lds, tp, f, x);
+  ln.solve2(op, p, pd, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) {
+    pd[m] = pd[m] * ih;
     r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
     r[m] = r[m] - pd[m];
   }
   if constexpr (FUSE) {
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) zc->mom[DIR][m][threadIdx.x] = r[m];
+    for (int m = 0; m < PPT; ++m) zc->mom(DIR, m) = r[m];
   } else {
     st<DIR>(rhs + (1 + DIR) * N, B, PS, r);
   }
 
-  // pressure-equation bracket: gamma/(gamma-1) (-d(p u_DIR)) + u_DIR p_DIR (:180-187)
-  T e[PPT];
-#pragma unroll
-  for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * p[m]) * ud[m] : p[m] * ud[m];
-  line_solve<T, PER>(op, lds, tp, f, x);
-#pragma unroll
-  for (int m = 0; m < PPT; ++m) e[m] = div(m, T(ph.gt) * (-(x[m] * ih))) + ud[m] * pd[m];
-
-  // heat flux d/dx_DIR (lambda d/dx_DIR T) (:189-199); the x sweep evaluates
-  // the viscosity law and leaves mu in G6 for the later sweeps of the stage
-  T mu[PPT], Jv[PPT];
+  // pressure-equation bracket: gamma/(gamma-1) (-d(p u_DIR)) + u_DIR p_DIR
+  // (:180-187), and the inner derivative of the heat flux d/dx_DIR (lambda
+  // d/dx_DIR T) (:189-199); the x sweep evaluates the viscosity law and leaves
+  // mu in G6 for the later sweeps of the stage
+  T e[PPT], tk[PPT], mu[PPT], Jv[PPT];
   if (DIR != 0) {
     ld<DIR>(rhs + 4 * N, B, PS, r);
     ld<DIR>(G + 6 * N, B, PS, mu);
+  }
+  if (GT) ld<DIR>(mt.J, B, PS, Jv);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    f[m] = EV ? (PH[m] * p[m]) * ud[m] : p[m] * ud[m];
+    tk[m] = temperature(ph, irho[m], p[m]);
+  }
+  if (DIR == 0) {
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) mu[m] = viscosity(ph, tk[m]);
+    st<DIR>(G + 6 * N, B, PS, mu);
   }
   if constexpr (FUSE) {
 #pragma unroll
     for (int m = 0; m < PPT; ++m) zc->mu[m] = mu[m];
   }
-  if (GT) ld<DIR>(mt.J, B, PS, Jv);
-#pragma unroll
-  for (int m = 0; m < PPT; ++m) f[m] = temperature(ph, irho[m], p[m]);
-  if (DIR == 0) {
-#pragma unroll
-    for (int m = 0; m < PPT; ++m) mu[m] = viscosity(ph, f[m]);
-    st<DIR>(G + 6 * N, B, PS, mu);
-  }
-  line_solve<T, PER>(op, lds, tp, f, x);
+  ln.solve2(op, f, x, tk, y);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) {
+    e[m] = div(m, T(ph.gt) * (-(x[m] * ih))) + ud[m] * pd[m];
     const T lam = GT ? lambda_of(ph, mu[m]) * Jv[m]
                      : (EV ? PH[m] * lambda_of(ph, mu[m]) : lambda_of(ph, mu[m]));
-    f[m] = lam * (x[m] * hin);
+    f[m] = lam * (y[m] * hin);
   }
-  line_solve<T, PER>(op, lds, tp, f, x);
+  ln.solve(op, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) {
     e[m] = e[m] + div(m, x[m] * hout);
@@ -401,10 +413,11 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
 
 template <typename T, typename Q, int DIR, bool PER, int FORM>
 __global__ __launch_bounds__(NT) void k_sweep1(const Q *__restrict__ qs, T *__restrict__ rhs,
-                                                          T *__restrict__ G, LineOp<T> op, SweepGeom g,
+                                                          T *__restrict__ G, Op<T> op, SweepGeom g,
                                                           Phys ph, long N, Metric<T> mt, Penal<T> pe) {
-  __shared__ LineLds<T> lds;
-  sweep1_body<T, Q, DIR, PER, FORM>(thread_pos<DIR>(g), qs, rhs, G, op, g, ph, N, mt, pe, lds);
+  const ThreadPos tp = thread_pos<DIR>(g);
+  auto ln = make_lines<T, PER>(op, tp);
+  sweep1_body<T, Q, DIR, FORM>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln);
 }
 
 // RK4 stage update of variable v from its complete RHS k (rk_o4_e.f90:45-50,
@@ -484,16 +497,15 @@ __device__ __forceinline__ void rk_update(int mode, int v, const T (&k)[PPT], lo
 // last sweep multiplies every equation by X_jacobian and the dissipation once
 // more (ns_rho_rhou_p_grid_transform.f90:190-276).
 // EV: d/dx_d (phi tau_id), times the stored 1/phi (ns_rho_rhou_p_ev_phi.f90:161-201).
-template <typename T, int DIR, bool PER, int FORM, bool FF>
+template <typename T, int DIR, int FORM, bool FF, typename Lines>
 __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__ rhs, const T *__restrict__ G,
-                                            const LineOp<T> &op, const LineOp<T> &fop, const SweepGeom &g,
+                                            const Op<T> &op, const Op<T> &fop, const SweepGeom &g,
                                             const Phys &ph, long N, int mode, double *__restrict__ qn,
                                             T *__restrict__ acc, T *__restrict__ qs_out, double dt,
                                             const Metric<T> &mt, const T *__restrict__ force,
-                                            const Penal<T> &pe) {
+                                            const Penal<T> &pe, Lines &ln) {
   constexpr bool GT = FORM == RHS_GT, EV = FORM == RHS_EV;
   constexpr bool LAST = DIR == 0;
-  __shared__ LineLds<T, sweep_nt<T>()> lds;
   const long B = tp.base, PS = g.PS;
   const T ih = GT ? T(ph.inv_h[DIR]) * mt.m[DIR][tp.lidx] : T(ph.inv_h[DIR]);
   T t1[PPT], t2[PPT], t3[PPT], diss[PPT];
@@ -550,7 +562,9 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
       T f[PPT], x[PPT];
 #pragma unroll
       for (int m = 0; m < PPT; ++m) f[m] = T(a[m]);
-      line_solve<T, PER>(fop, lds, tp, f, x);
+      ln.bind(fop);
+      ln.template solve<true>(fop, f, x);
+      ln.bind(op);
       st<DIR>(qn + v * N, B, PS, x);
     } else {
       rk_update<DIR, T>(mode, v, k, B, PS, N, rhs, qn, acc, qs_out, dt);
@@ -610,7 +624,7 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     T x[PPT];
-    line_solve<T, PER>(op, lds, tp, i == 0 ? t1 : (i == 1 ? t2 : t3), x);
+    ln.solve(op, i == 0 ? t1 : (i == 1 ? t2 : t3), x);
     asm volatile("" ::: "memory");
     T k[PPT];
     ld<DIR>(rhs + (1 + i) * N, B, PS, k);
@@ -630,13 +644,14 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
 
 template <typename T, int DIR, bool PER, int FORM, bool FF>
 __global__ __launch_bounds__(sweep_nt<T>()) void k_sweep2(T *__restrict__ rhs, const T *__restrict__ G,
-                                                          LineOp<T> op, LineOp<T> fop, SweepGeom g, Phys ph,
+                                                          Op<T> op, Op<T> fop, SweepGeom g, Phys ph,
                                                           long N, int mode, double *__restrict__ qn,
                                                           T *__restrict__ acc, T *__restrict__ qs_out,
                                                           double dt, Metric<T> mt, const T *__restrict__ force,
                                                           Penal<T> pe) {
-  sweep2_body<T, DIR, PER, FORM, FF>(thread_pos<DIR>(g), rhs, G, op, fop, g, ph, N, mode, qn, acc, qs_out, dt, mt,
-                                     force, pe);
+  const ThreadPos tp = thread_pos<DIR>(g);
+  auto ln = make_lines<T, PER, sweep_nt<T>()>(op, tp);
+  sweep2_body<T, DIR, FORM, FF>(tp, rhs, G, op, fop, g, ph, N, mode, qn, acc, qs_out, dt, mt, force, pe, ln);
 }
 
 // S3 + S4: the z first-derivative sweep and the z viscous sweep as one
@@ -648,10 +663,10 @@ __global__ __launch_bounds__(sweep_nt<T>()) void k_sweep2(T *__restrict__ rhs, c
 // momentum RHS in LDS between the two parts (ZCarry), so the viscous part
 // reads only u_x and v_y and writes the momentum RHS once; the deformed-grid
 // and penalised forms run the two sweep bodies one after the other.
-template <typename T, bool PER>
+template <typename T, typename Lines>
 __device__ __forceinline__ void viscous_z_carry(const ThreadPos &tp, T *__restrict__ rhs, const T *__restrict__ G,
-                                                const LineOp<T> &op, const SweepGeom &g, const Phys &ph, long N,
-                                                LineLds<T> &lds, const ZCarry<T> &zc) {
+                                                const Op<T> &op, const SweepGeom &g, const Phys &ph, long N,
+                                                Lines &ln, const ZCarry<T> &zc) {
   const long B = tp.base, PS = g.PS;
   const T ih = T(ph.inv_h[2]);
   T t1[PPT], t2[PPT], t3[PPT];
@@ -669,33 +684,35 @@ __device__ __forceinline__ void viscous_z_carry(const ThreadPos &tp, T *__restri
       t3[m] = md + 2 * mu * wz;  // tau_33
     }
   }
+  T x[PPT], y[PPT];
+  auto put = [&](int i, T(&v)[PPT]) {
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    T x[PPT], k[PPT];
-    line_solve<T, PER>(op, lds, tp, i == 0 ? t1 : (i == 1 ? t2 : t3), x);
-#pragma unroll
-    for (int m = 0; m < PPT; ++m) k[m] = zc.mom[i][m][threadIdx.x] + x[m] * ih;
-    st<2>(rhs + (1 + i) * N, B, PS, k);
-  }
+    for (int m = 0; m < PPT; ++m) v[m] = zc.mom(i, m) + v[m] * ih;
+    st<2>(rhs + (1 + i) * N, B, PS, v);
+  };
+  ln.solve2(op, t1, x, t2, y);
+  put(0, x);
+  put(1, y);
+  ln.solve(op, t3, x);
+  put(2, x);
 }
 
 template <typename T, typename Q, bool PER, int FORM>
 __global__ __launch_bounds__(NT) void k_sweep12_z(const Q *__restrict__ qs, T *__restrict__ rhs,
-                                                   T *__restrict__ G, LineOp<T> op, SweepGeom g, Phys ph,
+                                                   T *__restrict__ G, Op<T> op, SweepGeom g, Phys ph,
                                                    long N, Metric<T> mt, Penal<T> pe) {
   const ThreadPos tp = thread_pos<2>(g);
-  __shared__ LineLds<T> lds;
+  auto ln = make_lines<T, PER>(op, tp);
   if constexpr (FORM == RHS_CART) {
-    __shared__ T mom[3][PPT][NT];
     ZCarry<T> zc;
-    zc.mom = mom;
-    sweep1_body<T, Q, 2, PER, FORM, true>(tp, qs, rhs, G, op, g, ph, N, mt, pe, lds, &zc);
-    viscous_z_carry<T, PER>(tp, rhs, G, op, g, ph, N, lds, zc);
+    z_carry_slots(zc);
+    sweep1_body<T, Q, 2, FORM, true>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln, &zc);
+    viscous_z_carry<T>(tp, rhs, G, op, g, ph, N, ln, zc);
   } else {
-    sweep1_body<T, Q, 2, PER, FORM>(tp, qs, rhs, G, op, g, ph, N, mt, pe, lds);
+    sweep1_body<T, Q, 2, FORM>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln);
     asm volatile("" ::: "memory");
-    sweep2_body<T, 2, PER, FORM, false>(tp, rhs, G, op, op, g, ph, N, 0, nullptr, nullptr, nullptr, 0.0, mt,
-                                        nullptr, pe);
+    sweep2_body<T, 2, FORM, false>(tp, rhs, G, op, op, g, ph, N, 0, nullptr, nullptr, nullptr, 0.0, mt, nullptr, pe,
+                                   ln);
   }
 }
 
@@ -704,12 +721,12 @@ __global__ __launch_bounds__(NT) void k_sweep12_z(const Q *__restrict__ qs, T *_
 // Single derivative (Dx1/2/3) of one field: out = (B^-1 A in) / h.
 template <typename T, int DIR, bool PER>
 __global__ __launch_bounds__(NT) void k_diff(const T *__restrict__ in, T *__restrict__ out,
-                                             LineOp<T> op, SweepGeom g, double inv_h) {
-  __shared__ LineLds<T> lds;
+                                             Op<T> op, SweepGeom g, double inv_h) {
   const ThreadPos tp = thread_pos<DIR>(g);
+  auto ln = make_lines<T, PER>(op, tp);
   T f[PPT], x[PPT];
   ld<DIR>(in, tp.base, g.PS, f);
-  line_solve<T, PER>(op, lds, tp, f, x);
+  ln.solve(op, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) x[m] = x[m] * T(inv_h);
   st<DIR>(out, tp.base, g.PS, x);
@@ -723,10 +740,9 @@ constexpr int filter_nt() { return sizeof(T) == 4 ? NT_FILTER32 : NT; }
 // the filtered FP64 fields go (null: nowhere); copy: the filtered fields in
 // the compute precision (null: nowhere).  src may be q64 or copy (in place:
 // every thread loads its block before the line solve that the stores follow).
-template <typename T, int DIR, bool PER, typename S>
-__device__ __forceinline__ void filter_body(const ThreadPos &tp, const S *src, double *q64, const LineOp<T> &op,
-                                            const SweepGeom &g, long N, int nv, T *copy) {
-  __shared__ LineLds<T, filter_nt<T>()> lds;
+template <typename T, int DIR, typename S, typename LOp, typename Lines>
+__device__ __forceinline__ void filter_body(const ThreadPos &tp, const S *src, double *q64, const LOp &op,
+                                            const SweepGeom &g, long N, int nv, T *copy, Lines &ln) {
   double a[PPT];
   ld<DIR>(src, tp.base, g.PS, a);
   for (int v = 0; v < nv; ++v) {
@@ -735,7 +751,7 @@ __device__ __forceinline__ void filter_body(const ThreadPos &tp, const S *src, d
     for (int m = 0; m < PPT; ++m) f[m] = T(a[m]);
     // the next field's loads fly while this one is filtered
     if (v + 1 < nv) ld<DIR>(src + (v + 1) * N, tp.base, g.PS, a);
-    line_solve<T, PER>(op, lds, tp, f, x);
+    ln.template solve<true>(op, f, x);
     if (q64) st<DIR>(q64 + v * N, tp.base, g.PS, x);
     // the filtered state in the compute precision, when the next RK stage
     // or filter pass reads it (it equals the FP64 value converted back)
@@ -744,9 +760,22 @@ __device__ __forceinline__ void filter_body(const ThreadPos &tp, const S *src, d
 }
 
 template <typename T, int DIR, bool PER, typename S>
-__global__ __launch_bounds__(filter_nt<T>()) void k_filter(const S *src, double *q64, LineOp<T> op, SweepGeom g,
+__global__ __launch_bounds__(filter_nt<T>()) void k_filter(const S *src, double *q64, Op<T> op, SweepGeom g,
                                                            long N, int nv, T *copy) {
-  filter_body<T, DIR, PER, S>(thread_pos<DIR>(g), src, q64, op, g, N, nv, copy);
+  const ThreadPos tp = thread_pos<DIR>(g);
+  auto ln = make_lines<T, PER, filter_nt<T>()>(op, tp);
+  filter_body<T, DIR, S>(tp, src, q64, op, g, N, nv, copy, ln);
+}
+
+// The FP64 filter on the cyclic reduction, for the filter parameters that the
+// recursions do not take (HostRecOp::usable).
+template <int DIR, bool PER>
+__global__ __launch_bounds__(NT) void k_filter_cr(const double *src, double *q64, LineOp<double> op, SweepGeom g,
+                                                  long N, int nv) {
+  __shared__ LineLds<double> lds;
+  const ThreadPos tp = thread_pos<DIR>(g);
+  CrLines<double, PER, NT> ln{lds, tp};
+  filter_body<double, DIR, double>(tp, src, q64, op, g, N, nv, (double *)nullptr, ln);
 }
 
 }  // namespace cruna
