@@ -31,22 +31,29 @@ namespace cruna {
 
 // Hand the accumulated variable v on: intermediate sweeps store it; the last
 // sweep adds g and applies the RK4 stage update.
-template <int DIR, typename T, bool LAST>
-__device__ __forceinline__ void finish(int v, T (&r)[PPT], long B, long PS, long N, T *rhs,
-                                       const double *__restrict__ gobj, int mode,
-                                       double *__restrict__ qn, T *__restrict__ acc,
-                                       T *qs_out, double dt) {
-  if (!LAST) {
+template <int DIR, typename T, bool LAST, int RK>
+__device__ __forceinline__ void finish(int v, T (&r)[PPT], long B, long PS, long N, T *__restrict__ rhs,
+                                       const double *__restrict__ gobj, const RkArgs<T> &rk) {
+  if constexpr (!LAST) {
     st<DIR>(rhs + v * N, B, PS, r);
-    return;
-  }
-  if (gobj) {
-    double gg[PPT];
-    ld<DIR>(gobj + v * N, B, PS, gg);
+  } else {
+    RkIn<RK, T> in;
+    if constexpr (RK != RK_YLAST) rk_load<DIR, RK, T>(rk, v, B, PS, N, in);
+    if (gobj) {
+      double gg[PPT];
+      ld<DIR>(gobj + v * N, B, PS, gg);
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) r[m] = r[m] + T(gg[m]);
+      for (int m = 0; m < PPT; ++m) r[m] = r[m] + T(gg[m]);
+    }
+    if constexpr (RK == RK_YLAST) {
+      double q1[PPT];
+      materialize(r);
+      rk_ylast<DIR>(rk, v, r, B, PS, N, q1);
+      st<DIR>(rk.qn + v * N, B, PS, q1);
+    } else {
+      rk_store<DIR, RK, T>(rk, v, r, in, B, PS, N, rhs);
+    }
   }
-  rk_update<DIR, T>(mode, v, r, B, PS, N, rhs, qn, acc, qs_out, dt);
 }
 
 // One adjoint sweep along DIR.
@@ -56,15 +63,14 @@ __device__ __forceinline__ void finish(int v, T (&r)[PPT], long B, long PS, long
 //          serve every step of a backward loop (the slot is set on the device)
 //   rhs  : 5 accumulator fields (written by the first sweep, z)
 //   gobj : objective gradient g (5 fields) or null; added by the x sweep
-// The x sweep (LAST) completes the stage: mode 0..3 RK4 update with step dt
-// (negative for the backward integration), mode 4 writes the RHS.
-template <typename T, typename Q, int DIR, typename Lines>
+// The x sweep (LAST) completes the stage: RK4 update RK (RkForm) with step
+// rk.dt (negative for the backward integration).
+template <typename T, typename Q, int DIR, int RK, typename Lines>
 __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
                                             const double *const *__restrict__ q0p, T *__restrict__ rhs,
                                             const double *__restrict__ gobj, const Op<T> &op,
-                                            const SweepGeom &g, double gamma, double inv_h, long N, int mode,
-                                            double *__restrict__ qn, T *__restrict__ acc, T *qs_out,
-                                            double dt, Lines &ln) {
+                                            const SweepGeom &g, double gamma, double inv_h, long N,
+                                            const RkArgs<T> &rk, Lines &ln) {
   constexpr bool FIRST = DIR == 2, LAST = DIR == 0;
   const double *__restrict__ q = *q0p;
   const long B = tp.base, PS = g.PS;
@@ -123,7 +129,7 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
       R5[m] = R5[m] + gm1 * Bd;
       r[m] = FIRST ? -R5[m] : r[m] - R5[m];
     }
-    finish<DIR, T, LAST>(4, r, B, PS, N, rhs, gobj, mode, qn, acc, qs_out, dt);
+    finish<DIR, T, LAST, RK>(4, r, B, PS, N, rhs, gobj, rk);
   }
   // A = D qs1; A + u_d B_d waits in LDS (the thread's own slots) until the
   // end, which keeps the x sweep within 256 registers without spilling
@@ -150,7 +156,7 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
       S[m] = S[m] + (um[m] * irho[m]) * Bm;
       r[m] = FIRST ? -(ud[m] * Bm) : r[m] - ud[m] * Bm;
     }
-    finish<DIR, T, LAST>(1 + i, r, B, PS, N, rhs, gobj, mode, qn, acc, qs_out, dt);
+    finish<DIR, T, LAST, RK>(1 + i, r, B, PS, N, rhs, gobj, rk);
   }
   // r1 += u_d S, r_{d+2} -= A + u_d B_d + S
 #pragma unroll
@@ -163,19 +169,18 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
       const T c = v == 0 ? ud[m] * S[m] : -(stash[m][threadIdx.x] + S[m]);
       r[m] = FIRST ? c : r[m] + c;
     }
-    finish<DIR, T, LAST>(var, r, B, PS, N, rhs, gobj, mode, qn, acc, qs_out, dt);
+    finish<DIR, T, LAST, RK>(var, r, B, PS, N, rhs, gobj, rk);
   }
 }
 
-template <typename T, typename Q, int DIR, bool PER>
+template <typename T, typename Q, int DIR, bool PER, int RK>
 __global__ __launch_bounds__(NT) void k_asweep(const Q *qs, const double *const *__restrict__ q0p,
                                                T *__restrict__ rhs, const double *__restrict__ gobj,
                                                Op<T> op, SweepGeom g, double gamma, double inv_h, long N,
-                                               int mode, double *__restrict__ qn, T *__restrict__ acc,
-                                               T *qs_out, double dt) {
+                                               RkArgs<T> rk) {
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER>(op, tp);
-  asweep_body<T, Q, DIR>(tp, qs, q0p, rhs, gobj, op, g, gamma, inv_h, N, mode, qn, acc, qs_out, dt, ln);
+  asweep_body<T, Q, DIR, RK>(tp, qs, q0p, rhs, gobj, op, g, gamma, inv_h, N, rk, ln);
 }
 
 // characteristic_qs_k1d (src/boundaries/nonreflecting.f90:453-554) on the

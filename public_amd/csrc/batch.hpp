@@ -22,7 +22,8 @@ constexpr int BATCH_MAX = 64;
 
 // The arguments the per-member kernels take, for one member.
 struct BatchMember {
-  double *qn, *acc, *qs, *rhs, *G;  // direct state, RK accumulator, stage input, RHS, gradients
+  double *qn, *rhs, *G;             // direct state, RHS, gradients
+  double *y[3];                     // stage inputs y2, y3, y4
   double *qa;                       // adjoint state
   const double **q0p;               // adjoint: cell with the forward state of the step
   int *ntp;                         // adjoint: backward step counter
@@ -56,42 +57,52 @@ __device__ __forceinline__ int batch_entry(const BatchList *__restrict__ L) {
   return lo;
 }
 
-// first-derivative sweep; stage input q^n (from_qs = 0) or qs
+// input of RK stage `stage` (0: q0 itself) and the update's arguments
+__device__ __forceinline__ const double *stage_in(const BatchMember &b, const double *q0, int stage) {
+  return stage == 0 ? q0 : b.y[stage - 1];
+}
+__device__ __forceinline__ RkArgs<double> stage_rk(const BatchMember &b, double *q0, double dt, int stage) {
+  return RkArgs<double>{q0, nullptr, stage < 3 ? b.y[stage] : nullptr, b.y[0], b.y[1], b.y[2], dt,
+                        stage == 2 ? dt : 0.5 * dt};
+}
+
+// first-derivative sweep of RK stage `stage`
 template <int DIR, bool PER>
 __global__ __launch_bounds__(NT) void kb_sweep1(const BatchMember *__restrict__ M, const BatchList *__restrict__ L,
-                                                int from_qs) {
+                                                int stage) {
   const int e = batch_entry(L);
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.geom[DIR], blockIdx.x - L->start[e]);
   auto ln = make_lines<double, PER>(b.op[DIR], tp);
-  sweep1_body<double, double, DIR, RHS_CART>(tp, from_qs ? b.qs : b.qn, b.rhs, b.G, b.op[DIR], b.geom[DIR], b.ph, b.N,
+  sweep1_body<double, double, DIR, RHS_CART>(tp, stage_in(b, b.qn, stage), b.rhs, b.G, b.op[DIR], b.geom[DIR], b.ph, b.N,
                                              Metric<double>{}, Penal<double>{}, ln);
 }
 
-// viscous sweep; the x sweep finishes RK4 stage `mode` (FF: the last stage
+// viscous sweep; the x sweep finishes RK stage `stage` (FF: the last stage
 // with the fused x filter)
-template <int DIR, bool PER, bool FF>
+template <int DIR, bool PER, int RK, bool FF>
 __global__ __launch_bounds__(NT) void kb_sweep2(const BatchMember *__restrict__ M, const BatchList *__restrict__ L,
-                                                int mode) {
+                                                int stage) {
   const int e = batch_entry(L);
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.geom[DIR], blockIdx.x - L->start[e]);
   auto ln = make_lines<double, PER>(b.op[DIR], tp);
-  sweep2_body<double, DIR, RHS_CART, FF>(tp, b.rhs, b.G, b.op[DIR], b.fop[DIR], b.geom[DIR], b.ph, b.N, mode, b.qn,
-                                         b.acc, b.qs, b.dt, Metric<double>{}, nullptr, Penal<double>{}, ln);
+  sweep2_body<double, DIR, RHS_CART, RK, FF>(tp, b.rhs, b.G, b.op[DIR], b.fop[DIR], b.geom[DIR], b.ph, b.N,
+                                             stage_rk(b, b.qn, b.dt, stage), Metric<double>{}, nullptr,
+                                             Penal<double>{}, ln);
 }
 
 // the z first-derivative and viscous sweeps as one kernel (k_sweep12_z)
 template <bool PER>
 __global__ __launch_bounds__(NT) void kb_sweep12_z(const BatchMember *__restrict__ M,
-                                                   const BatchList *__restrict__ L, int from_qs) {
+                                                   const BatchList *__restrict__ L, int stage) {
   const int e = batch_entry(L);
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<2, true>(b.geom[2], blockIdx.x - L->start[e]);
   auto ln = make_lines<double, PER>(b.op[2], tp);
   ZCarry<double> zc;
   z_carry_slots(zc);
-  sweep1_body<double, double, 2, RHS_CART, true>(tp, from_qs ? b.qs : b.qn, b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N,
+  sweep1_body<double, double, 2, RHS_CART, true>(tp, stage_in(b, b.qn, stage), b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N,
                                                  Metric<double>{}, Penal<double>{}, ln, &zc);
   viscous_z_carry<double>(tp, b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N, ln, zc);
 }
@@ -108,16 +119,17 @@ __global__ __launch_bounds__(NT) void kb_filter(const BatchMember *__restrict__ 
   filter_body<double, DIR, double>(tp, q, q, b.fop[DIR], b.fgeom[DIR], b.N, 5, (double *)nullptr, ln);
 }
 
-// adjoint sweep (backward in time: dt -> -dt); stage input qs^n (from_qs = 0) or qs
-template <int DIR, bool PER>
+// adjoint sweep of RK stage `stage` (backward in time: dt -> -dt)
+template <int DIR, bool PER, int RK>
 __global__ __launch_bounds__(NT) void kb_asweep(const BatchMember *__restrict__ M, const BatchList *__restrict__ L,
-                                                int mode, int from_qs) {
+                                                int stage) {
   const int e = batch_entry(L);
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.geom[DIR], blockIdx.x - L->start[e]);
   auto ln = make_lines<double, PER>(b.op[DIR], tp);
-  asweep_body<double, double, DIR>(tp, from_qs ? b.qs : b.qa, (const double *const *)b.q0p, b.rhs, nullptr, b.op[DIR],
-                                   b.geom[DIR], b.gamma, b.ph.inv_h[DIR], b.N, mode, b.qa, b.acc, b.qs, -b.dt, ln);
+  asweep_body<double, double, DIR, RK>(tp, stage_in(b, b.qa, stage), (const double *const *)b.q0p, b.rhs, nullptr,
+                                       b.op[DIR], b.geom[DIR], b.gamma, b.ph.inv_h[DIR], b.N,
+                                       stage_rk(b, b.qa, -b.dt, stage), ln);
 }
 
 // Per-member bookkeeping of a batched step, one work-group row per member

@@ -29,6 +29,7 @@
 // defined in sweeps_*.hip
 INST_GROUP_PERIODIC64(extern)
 INST_GROUP_OPEN64(extern)
+INST_GROUP_OPEN64B(extern)
 INST_GROUP_CURV64(extern)
 INST_GROUP_CURV64O(extern)
 INST_GROUP_FP32(extern)
@@ -203,6 +204,10 @@ struct cruna_hip_ctx {
   int ckpt_n = 0;
   int sub_steps = 0;  // steps per subset (cruna_hip_subsets_alloc)
   void *qs = nullptr, *rhs = nullptr, *G = nullptr;  // compute precision
+  // FP64 without boundary rows that change the stage inputs or act on the
+  // complete RHS: the RK4 steps keep their stage inputs y2, y3, y4 (in qs, acc
+  // and y4) instead of an accumulator (RkForm)
+  double *y4 = nullptr;
   // learned closure added to the direct RHS (cruna_hip_set_closure)
   cruna_hip_cnn *cnn = nullptr;
   void *force = nullptr;  // its term, 5 fields in the compute precision
@@ -551,6 +556,37 @@ __global__ __launch_bounds__(256) void k_rk_stage(int mode, const T *__restrict_
 template <typename T, typename Q>
 int closure_term(cruna_hip_ctx *c, const Q *in);
 
+// The RK4 update of stage `mode` (0..3; 4: a single RHS evaluation) on the
+// state q0, with the step dt; y: the form without an accumulator.
+int rk_form(int mode, bool y) {
+  if (mode == 4) return RK_RHS;
+  if (y) return mode == 3 ? RK_YLAST : RK_Y;
+  return mode == 0 ? RK_FIRST : (mode == 3 ? RK_LAST : RK_MID);
+}
+template <typename T>
+RkArgs<T> rk_args(cruna_hip_ctx *c, double *q0, double dt, int mode, bool y) {
+  RkArgs<T> a{};
+  a.qn = q0;
+  a.acc = (T *)c->acc;
+  a.y2 = (const T *)c->qs;
+  a.y3 = (const T *)c->acc;
+  a.y4 = (const T *)c->y4;
+  a.out = (T *)(y && mode == 1 ? (void *)c->acc : (y && mode == 2 ? (void *)c->y4 : c->qs));
+  a.dt = dt;
+  a.c = mode == 2 ? dt : dt * 0.5;
+  return a;
+}
+// the input of stage `mode` >= 1
+template <typename T>
+const T *stage_input(cruna_hip_ctx *c, int mode, bool y) {
+  return (const T *)(y && mode == 2 ? (void *)c->acc : (y && mode == 3 ? (void *)c->y4 : c->qs));
+}
+bool direct_yform(const cruna_hip_ctx *c) { return c->y4 != nullptr; }
+// the adjoint also runs its sponge rows of the Euler equations on the complete RHS
+bool adjoint_yform(const cruna_hip_ctx *c) {
+  return c->y4 != nullptr && !(c->cfg.equations == CRUNA_HIP_EQ_EULER && c->has_bcrhs);
+}
+
 template <typename T, typename Q, int DIR, int FORM>
 void launch_sweep1_form(cruna_hip_ctx *c, const Q *in) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
@@ -630,74 +666,94 @@ int launch_sweep1(cruna_hip_ctx *c, const Q *in) {
   return check_launch();
 }
 
-template <typename T, int DIR, int FORM>
-void launch_sweep2_form(cruna_hip_ctx *c, int mode, bool fuse_filter) {
+template <typename T, int DIR, int FORM, int RK, bool FF>
+void launch_sweep2_k(cruna_hip_ctx *c, int mode) {
   const dim3 grid(c->sgeom[DIR].ntiles), block(c->swg[DIR]);
   const size_t lds = line_lds_bytes<T>(c->swg[DIR]);
-  T *rhs = (T *)c->rhs, *qs = (T *)c->qs;
+  T *rhs = (T *)c->rhs;
   const T *G = (const T *)c->G;
   const Op<T> &op = dops<T>(c)[DIR].op, &fop = fops<T>(c)[DIR].op;
   const T *force = (const T *)(DIR == 0 && c->cnn ? c->force : nullptr);
-  const bool per = c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC;
-  // the fused x filter exists on the last stage of the x sweep only
-  if constexpr (DIR == 0) {
-    if (fuse_filter && mode == 3) {
-      if (per)
-        hipLaunchKernelGGL((k_sweep2<T, DIR, true, FORM, true>), grid, block, lds, c->stream, rhs, G, op, fop,
-                           c->sgeom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, qs, c->cfg.dt, metric<T>(c), force,
-                           penal<T>(c));
-      else
-        hipLaunchKernelGGL((k_sweep2<T, DIR, false, FORM, true>), grid, block, lds, c->stream, rhs, G, op, fop,
-                           c->sgeom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, qs, c->cfg.dt, metric<T>(c), force,
-                           penal<T>(c));
-      return;
-    }
-  }
-  if (per) {
-    hipLaunchKernelGGL((k_sweep2<T, DIR, true, FORM, false>), grid, block, lds, c->stream, rhs, G, op, fop,
-                       c->sgeom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, qs, c->cfg.dt, metric<T>(c), force,
-                           penal<T>(c));
+  const RkArgs<T> rk = rk_args<T>(c, c->qn, c->cfg.dt, mode, direct_yform(c));
+  if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC)
+    hipLaunchKernelGGL((k_sweep2<T, DIR, true, FORM, RK, FF>), grid, block, lds, c->stream, rhs, G, op, fop,
+                       c->sgeom[DIR], c->phys, c->N, rk, metric<T>(c), force, penal<T>(c));
+  else
+    hipLaunchKernelGGL((k_sweep2<T, DIR, false, FORM, RK, FF>), grid, block, lds, c->stream, rhs, G, op, fop,
+                       c->sgeom[DIR], c->phys, c->N, rk, metric<T>(c), force, penal<T>(c));
+}
+
+template <typename T, int DIR, int FORM>
+void launch_sweep2_form(cruna_hip_ctx *c, int mode, bool fuse_filter) {
+  if constexpr (DIR != 0) {
+    launch_sweep2_k<T, DIR, FORM, RK_RHS, false>(c, mode);
   } else {
-    hipLaunchKernelGGL((k_sweep2<T, DIR, false, FORM, false>), grid, block, lds, c->stream, rhs, G, op, fop,
-                       c->sgeom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, qs, c->cfg.dt, metric<T>(c), force,
-                           penal<T>(c));
+    const int form = rk_form(mode, direct_yform(c));
+    // the fused x filter exists on the last stage only (in FP64 without an
+    // accumulator: contexts with boundary rows never fuse it)
+    if (form == RK_RHS) {
+      launch_sweep2_k<T, 0, FORM, RK_RHS, false>(c, mode);
+    } else if (form == RK_FIRST) {
+      launch_sweep2_k<T, 0, FORM, RK_FIRST, false>(c, mode);
+    } else if (form == RK_MID) {
+      launch_sweep2_k<T, 0, FORM, RK_MID, false>(c, mode);
+    } else if (form == RK_LAST) {
+      if constexpr (sizeof(T) == 4) {
+        if (fuse_filter) {
+          launch_sweep2_k<T, 0, FORM, RK_LAST, true>(c, mode);
+          return;
+        }
+      }
+      launch_sweep2_k<T, 0, FORM, RK_LAST, false>(c, mode);
+    } else if constexpr (sizeof(T) == 8) {
+      if (form == RK_Y) launch_sweep2_k<T, 0, FORM, RK_Y, false>(c, mode);
+      else if (fuse_filter) launch_sweep2_k<T, 0, FORM, RK_YLAST, true>(c, mode);
+      else launch_sweep2_k<T, 0, FORM, RK_YLAST, false>(c, mode);
+    }
   }
 }
 
-template <typename T, int DIR, bool PER, bool FF>
+template <typename T, int DIR, bool PER, bool FF, bool Y>
 void launch_curv_sweep2_k(cruna_hip_ctx *c, int mode) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
   const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
   const T *force = (const T *)(DIR == 0 && c->cnn ? c->force : nullptr);
+  const int form = DIR == 0 ? rk_form(mode, direct_yform(c)) : RK_RHS;
+  const RkArgs<T> rk = rk_args<T>(c, c->qn, c->cfg.dt, mode, direct_yform(c));
   if (c->ev)
-    hipLaunchKernelGGL((k_curv_sweep2<T, DIR, PER, FF, true>), grid, block, lds, c->stream, (T *)c->rhs,
+    hipLaunchKernelGGL((k_curv_sweep2<T, DIR, PER, FF, true, Y>), grid, block, lds, c->stream, (T *)c->rhs,
                        (const T *)c->G, (const T *)c->tg, dops<T>(c)[DIR].op, fops<T>(c)[DIR].op,
-                       c->geom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, (T *)c->qs, c->cfg.dt,
-                       curv_metric<T>(c), force, penal<T>(c));
+                       c->geom[DIR], c->phys, c->N, form, rk, curv_metric<T>(c), force, penal<T>(c));
   else
-    hipLaunchKernelGGL((k_curv_sweep2<T, DIR, PER, FF, false>), grid, block, lds, c->stream, (T *)c->rhs,
+    hipLaunchKernelGGL((k_curv_sweep2<T, DIR, PER, FF, false, Y>), grid, block, lds, c->stream, (T *)c->rhs,
                        (const T *)c->G, (const T *)c->tg, dops<T>(c)[DIR].op, fops<T>(c)[DIR].op,
-                       c->geom[DIR], c->phys, c->N, mode, c->qn, (T *)c->acc, (T *)c->qs, c->cfg.dt,
-                       curv_metric<T>(c), force, penal<T>(c));
+                       c->geom[DIR], c->phys, c->N, form, rk, curv_metric<T>(c), force, penal<T>(c));
+}
+
+template <typename T, int DIR, bool PER>
+void launch_curv_sweep2_per(cruna_hip_ctx *c, int mode, bool fuse_filter) {
+  // the fused x filter exists on the last stage of the x sweep only (FP64: of
+  // the form without an accumulator, as the Cartesian sweeps)
+  if constexpr (DIR == 0 && sizeof(T) == 8) {
+    if (direct_yform(c)) {
+      if (fuse_filter && mode == 3) launch_curv_sweep2_k<T, DIR, PER, true, true>(c, mode);
+      else launch_curv_sweep2_k<T, DIR, PER, false, true>(c, mode);
+      return;
+    }
+  }
+  if constexpr (DIR == 0 && sizeof(T) == 4) {
+    if (fuse_filter && mode == 3) {
+      launch_curv_sweep2_k<T, DIR, PER, true, false>(c, mode);
+      return;
+    }
+  }
+  launch_curv_sweep2_k<T, DIR, PER, false, false>(c, mode);
 }
 
 template <typename T, int DIR>
 void launch_curv_sweep2(cruna_hip_ctx *c, int mode, bool fuse_filter) {
-  const bool per = c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC;
-  // the fused x filter exists on the last stage of the x sweep only
-  if constexpr (DIR == 0) {
-    if (fuse_filter && mode == 3) {
-      if (per)
-        launch_curv_sweep2_k<T, DIR, true, true>(c, mode);
-      else
-        launch_curv_sweep2_k<T, DIR, false, true>(c, mode);
-      return;
-    }
-  }
-  if (per)
-    launch_curv_sweep2_k<T, DIR, true, false>(c, mode);
-  else
-    launch_curv_sweep2_k<T, DIR, false, false>(c, mode);
+  if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC) launch_curv_sweep2_per<T, DIR, true>(c, mode, fuse_filter);
+  else launch_curv_sweep2_per<T, DIR, false>(c, mode, fuse_filter);
 }
 
 template <typename T, int DIR>
@@ -763,7 +819,7 @@ int run_stage(cruna_hip_ctx *c, const double *from, int mode, bool fuse_filter =
   }
   if (c->has_bcq)
     if (int rc = bc_q<T>(c, qs)) return rc;
-  return rhs_stage<T, T>(c, (const T *)qs, mode, fuse_filter);
+  return rhs_stage<T, T>(c, stage_input<T>(c, mode, direct_yform(c)), mode, fuse_filter);
 }
 
 // RK4 step on qn; with fuse_filter the last stage also applies filter_i1.
@@ -1054,23 +1110,48 @@ int bc_qs(cruna_hip_ctx *c, Q *qs, bool outside = false) {
   return CRUNA_HIP_OK;
 }
 
+template <typename T, typename Q, int DIR, int RK>
+void launch_asweep_k(cruna_hip_ctx *c, const Q *in, const double *g, int mode) {
+  const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
+  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
+  // backward in time (rk_o4_e.f90:62-105)
+  const RkArgs<T> rk = rk_args<T>(c, c->qa, -c->cfg.dt, mode, adjoint_yform(c));
+  if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC)
+    hipLaunchKernelGGL((k_asweep<T, Q, DIR, true, RK>), grid, block, lds, c->stream, in, (const double *const *)c->q0p,
+                       (T *)c->rhs, g, dops<T>(c)[DIR].op, c->geom[DIR], c->cfg.gamma, c->phys.inv_h[DIR], c->N, rk);
+  else
+    hipLaunchKernelGGL((k_asweep<T, Q, DIR, false, RK>), grid, block, lds, c->stream, in, (const double *const *)c->q0p,
+                       (T *)c->rhs, g, dops<T>(c)[DIR].op, c->geom[DIR], c->cfg.gamma, c->phys.inv_h[DIR], c->N, rk);
+}
+
 template <typename T, typename Q, int DIR>
 int launch_asweep(cruna_hip_ctx *c, const Q *in, const double *g, int mode) {
   ProfScope p(c, DIR == 0 ? KID_AX : (DIR == 1 ? KID_AY : KID_AZ));
-  const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
-  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
-  T *rhs = (T *)c->rhs, *qs = (T *)c->qs;
-  const double dt = -c->cfg.dt;  // backward in time (rk_o4_e.f90:62-105)
-  if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC)
-    hipLaunchKernelGGL((k_asweep<T, Q, DIR, true>), grid, block, lds, c->stream, in,
-                       (const double *const *)c->q0p, rhs, g,
-                       dops<T>(c)[DIR].op, c->geom[DIR], c->cfg.gamma, c->phys.inv_h[DIR], c->N,
-                       mode, c->qa, (T *)c->acc, qs, dt);
-  else
-    hipLaunchKernelGGL((k_asweep<T, Q, DIR, false>), grid, block, lds, c->stream, in,
-                       (const double *const *)c->q0p, rhs, g,
-                       dops<T>(c)[DIR].op, c->geom[DIR], c->cfg.gamma, c->phys.inv_h[DIR], c->N,
-                       mode, c->qa, (T *)c->acc, qs, dt);
+  const int form = DIR == 0 ? rk_form(mode, adjoint_yform(c)) : RK_RHS;
+  if constexpr (DIR == 0) {
+    if (form == RK_FIRST) {
+      launch_asweep_k<T, Q, 0, RK_FIRST>(c, in, g, mode);
+      return check_launch();
+    }
+    if constexpr (sizeof(T) == sizeof(Q)) {  // later stages read the stage input
+      if (form == RK_MID) {
+        launch_asweep_k<T, Q, 0, RK_MID>(c, in, g, mode);
+        return check_launch();
+      }
+      if (form == RK_LAST) {
+        launch_asweep_k<T, Q, 0, RK_LAST>(c, in, g, mode);
+        return check_launch();
+      }
+      if constexpr (sizeof(T) == 8) {
+        if (form == RK_Y || form == RK_YLAST) {
+          if (form == RK_Y) launch_asweep_k<T, Q, 0, RK_Y>(c, in, g, mode);
+          else launch_asweep_k<T, Q, 0, RK_YLAST>(c, in, g, mode);
+          return check_launch();
+        }
+      }
+    }
+  }
+  launch_asweep_k<T, Q, DIR, RK_RHS>(c, in, g, mode);
   return check_launch();
 }
 
@@ -1129,7 +1210,7 @@ int arun_stage(cruna_hip_ctx *c, const double *from, const double *g, int mode) 
   }
   if (c->has_bcq)
     if (int rc = bc_qs<T>(c, qs)) return rc;
-  return arhs_stage<T, T>(c, (const T *)qs, g, mode);
+  return arhs_stage<T, T>(c, stage_input<T>(c, mode, adjoint_yform(c)), g, mode);
 }
 
 // time_stepper_adjoint (rk_o4_e.f90:62-105) on the device adjoint state qa.
@@ -1420,6 +1501,8 @@ int cruna_hip_create(const cruna_hip_cfg *cfg, cruna_hip_ctx **out) {
       hipMalloc(&c->acc, 5 * N * sizeof(double)) != hipSuccess ||
       hipMalloc(&c->qs, 5 * N * ts) != hipSuccess || hipMalloc(&c->rhs, 5 * N * ts) != hipSuccess ||
       hipMalloc(&c->G, 7 * N * ts) != hipSuccess ||
+      (cfg->precision == CRUNA_HIP_FP64 && !c->has_bcq && !c->has_bclate &&
+       hipMalloc(&c->y4, 5 * N * sizeof(double)) != hipSuccess) ||
       // the weighted filter's output buffer, allocated here so that a step
       // loop under graph capture allocates nothing
       ((cfg->wfilter_freq[0] > 0 || cfg->wfilter_freq[1] > 0 || cfg->wfilter_freq[2] > 0) &&
@@ -1446,7 +1529,7 @@ int cruna_hip_destroy(cruna_hip_ctx *c) {
   for (void *p : {(void *)c->qn, (void *)c->acc, (void *)c->qref, (void *)c->shape, (void *)c->tmp,
                   (void *)c->qa, (void *)c->traj, (void *)c->gobj, c->met, (void *)c->q0p, c->force,
                   (void *)c->ckpt, c->tg, c->pen, (void *)c->wphi, (void *)c->wtmp, (void *)c->wbuf,
-                  (void *)c->kvec, (void *)c->q0copy, (void *)c->res_buf,
+                  (void *)c->kvec, (void *)c->y4, (void *)c->q0copy, (void *)c->res_buf,
                   c->qs, c->rhs, c->G})
     if (p) (void)hipFree(p);
   for (auto &p : c->pending) {
@@ -2267,8 +2350,9 @@ int batch_upload(cruna_hip_ensemble *e, bool subsets, int nb) {
     cruna_hip_ctx *c = e->m[i];
     BatchMember &b = hm[i];
     b.qn = c->qn;
-    b.acc = c->acc;
-    b.qs = (double *)c->qs;
+    b.y[0] = (double *)c->qs;
+    b.y[1] = c->acc;
+    b.y[2] = c->y4;
     b.rhs = (double *)c->rhs;
     b.G = (double *)c->G;
     b.qa = c->qa;
@@ -2386,20 +2470,20 @@ struct BatchSlot {
 inline size_t batch_z_lds(int threads) { return z_lds_bytes<double>(threads, true); }
 
 template <int DIR>
-void batch_sweep1(const BatchSlot &S, int from_qs) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep1<DIR, true>), from_qs);
-  else BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep1<DIR, false>), from_qs);
+void batch_sweep1(const BatchSlot &S, int stage) {
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep1<DIR, true>), stage);
+  else BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep1<DIR, false>), stage);
 }
 
-void batch_sweep12z(const BatchSlot &S, int from_qs) {
-  if (S.e->bper[2]) BATCH_LAUNCH(S, 0, 0, 2, batch_z_lds, (kb_sweep12_z<true>), from_qs);
-  else BATCH_LAUNCH(S, 0, 0, 2, batch_z_lds, (kb_sweep12_z<false>), from_qs);
+void batch_sweep12z(const BatchSlot &S, int stage) {
+  if (S.e->bper[2]) BATCH_LAUNCH(S, 0, 0, 2, batch_z_lds, (kb_sweep12_z<true>), stage);
+  else BATCH_LAUNCH(S, 0, 0, 2, batch_z_lds, (kb_sweep12_z<false>), stage);
 }
 
-template <int DIR, bool FF>
-void batch_sweep2(const BatchSlot &S, int mode) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep2<DIR, true, FF>), mode);
-  else BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep2<DIR, false, FF>), mode);
+template <int DIR, int RK, bool FF>
+void batch_sweep2(const BatchSlot &S, int stage) {
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep2<DIR, true, RK, FF>), stage);
+  else BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep2<DIR, false, RK, FF>), stage);
 }
 
 template <int DIR>
@@ -2408,10 +2492,10 @@ void batch_filter(const BatchSlot &S, int grp) {
   else BATCH_LAUNCH(S, grp, 1, DIR, rec_lds_bytes, (kb_filter<DIR, false>), grp);
 }
 
-template <int DIR>
-void batch_asweep(const BatchSlot &S, int mode, int from_qs) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 1, 0, DIR, rec_lds_bytes, (kb_asweep<DIR, true>), mode, from_qs);
-  else BATCH_LAUNCH(S, 1, 0, DIR, rec_lds_bytes, (kb_asweep<DIR, false>), mode, from_qs);
+template <int DIR, int RK>
+void batch_asweep(const BatchSlot &S, int stage) {
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 1, 0, DIR, rec_lds_bytes, (kb_asweep<DIR, true, RK>), stage);
+  else BATCH_LAUNCH(S, 1, 0, DIR, rec_lds_bytes, (kb_asweep<DIR, false, RK>), stage);
 }
 
 // One forward step of the bin's group 0 (step_once of each member: RK4 with
@@ -2421,12 +2505,13 @@ int batch_forward_step(const BatchSlot &S, int record, int slot) {
   const cruna_hip_cfg &cf = S.e->m[0]->cfg;
   const bool fuse = cf.filter_freq[0] > 0;
   for (int st = 0; st < 4; ++st) {
-    batch_sweep1<0>(S, st > 0);
-    batch_sweep1<1>(S, st > 0);
-    batch_sweep12z(S, st > 0);
-    batch_sweep2<1, false>(S, st);
-    if (st == 3 && fuse) batch_sweep2<0, true>(S, st);
-    else batch_sweep2<0, false>(S, st);
+    batch_sweep1<0>(S, st);
+    batch_sweep1<1>(S, st);
+    batch_sweep12z(S, st);
+    batch_sweep2<1, RK_RHS, false>(S, st);
+    if (st < 3) batch_sweep2<0, RK_Y, false>(S, st);
+    else if (fuse) batch_sweep2<0, RK_YLAST, true>(S, st);
+    else batch_sweep2<0, RK_YLAST, false>(S, st);
   }
   if (cf.filter_freq[1] > 0) batch_filter<1>(S, 0);
   if (cf.filter_freq[2] > 0) batch_filter<2>(S, 0);
@@ -2440,9 +2525,10 @@ int batch_adjoint_step(const BatchSlot &S) {
   const BatchBin &B = S.bb();
   hipLaunchKernelGGL(kb_adjoint_slot, dim3(1, B.nadj), dim3(64), 0, S.s, S.mem(), S.list(1, 0, 0));
   for (int st = 0; st < 4; ++st) {
-    batch_asweep<2>(S, st, st > 0);
-    batch_asweep<1>(S, st, st > 0);
-    batch_asweep<0>(S, st, st > 0);
+    batch_asweep<2, RK_RHS>(S, st);
+    batch_asweep<1, RK_RHS>(S, st);
+    if (st < 3) batch_asweep<0, RK_Y>(S, st);
+    else batch_asweep<0, RK_YLAST>(S, st);
   }
   if (B.afreq[0] > 0) batch_filter<0>(S, 1);
   if (B.afreq[1] > 0) batch_filter<1>(S, 1);

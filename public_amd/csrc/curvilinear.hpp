@@ -192,15 +192,12 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
   acc(rhs + 4 * N, x);
 }
 
-template <typename T, int DIR, bool PER, bool FF, bool EV>
+template <typename T, int DIR, bool PER, bool FF, bool EV, bool Y>
 __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T *__restrict__ G,
                                                     const T *__restrict__ TG, Op<T> op,
                                                     Op<T> fop, SweepGeom g, Phys ph, long N,
-                                                    int mode, double *__restrict__ qn,
-                                                    T *__restrict__ acc,
-                                                    T *__restrict__ qs_out, double dt,
-                                                    CurvMetric<T> mt, const T *__restrict__ force,
-                                                    Penal<T> pe) {
+                                                    int form, RkArgs<T> rk, CurvMetric<T> mt,
+                                                    const T *__restrict__ force, Penal<T> pe) {
   constexpr bool LAST = DIR == 0;
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER>(op, tp);
@@ -306,16 +303,16 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
     }
     if constexpr (FF) {
       double a[PPT];
-      rk_new_state<DIR, T>(v, k, B, PS, N, qn, acc, dt, a);
+      rk_final<DIR, T, Y>(rk, v, k, B, PS, N, a);
       T f[PPT], x[PPT];
 #pragma unroll
       for (int m = 0; m < PPT; ++m) f[m] = T(a[m]);
       ln.bind(fop);
       ln.template solve<true>(fop, f, x);
       ln.bind(op);
-      st<DIR>(qn + v * N, B, PS, x);
+      st<DIR>(rk.qn + v * N, B, PS, x);
     } else {
-      rk_update<DIR, T>(mode, v, k, B, PS, N, rhs, qn, acc, qs_out, dt);
+      rk_update<DIR, T, Y>(form, rk, v, k, B, PS, N, rhs);
     }
   };
   if (EV) {  // phi tau_proj inside the derivative

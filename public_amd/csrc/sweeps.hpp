@@ -420,73 +420,167 @@ __global__ __launch_bounds__(NT) void k_sweep1(const Q *__restrict__ qs, T *__re
   sweep1_body<T, Q, DIR, FORM>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln);
 }
 
-// RK4 stage update of variable v from its complete RHS k (rk_o4_e.f90:45-50,
-// and :90-95 for the adjoint with dt -> -dt): stage inputs q0 + dt/2 k1,
-// q0 + dt/2 k2, q0 + dt k3, and q1 = q0 + dt/6 (k1 + 2 k2 + 2 k3 + k4).
-// The accumulator has the arithmetic type T.  FP64: it carries the partial
-// new state q0 + dt/6 k1 + dt/3 k2 + dt/3 k3, so the last stage reads it
-// alone (not q0 as well).  FP32-mixed: it carries the increment
-// dt/6 k1 + dt/3 k2 + dt/3 k3 alone, in FP32 (half the bytes of an FP64
-// accumulator in three stages out of four), and the last stage adds q0 in
-// FP64; the increment is a step's change of the state, so its FP32 rounding
-// is far below that of the FP32 stage inputs.  Either sum is associated
-// differently from the reference's, a rounding-level change.
-// mode 4 writes k into rhs instead (a single RHS evaluation).
-template <int DIR, typename T>
-__device__ __forceinline__ void rk_new_state(int v, const T (&k)[PPT], long B, long PS, long N,
-                                             const double *__restrict__ qn, const T *__restrict__ acc,
-                                             double dt, double (&q1)[PPT]) {
-  if constexpr (sizeof(T) == 8) {
-    ld<DIR>(acc + v * N, B, PS, q1);
-#pragma unroll
-    for (int m = 0; m < PPT; ++m) q1[m] = q1[m] + dt / 6.0 * double(k[m]);
-  } else {
-    T a[PPT];
-    ld<DIR>(qn + v * N, B, PS, q1);
-    ld<DIR>(acc + v * N, B, PS, a);
-#pragma unroll
-    for (int m = 0; m < PPT; ++m) q1[m] = q1[m] + (double(a[m]) + dt / 6.0 * double(k[m]));
+// RK4 stage update of a variable from its complete RHS k (rk_o4_e.f90:45-50,
+// and :90-95 for the adjoint with dt -> -dt): stage inputs y2 = q0 + dt/2 k1,
+// y3 = q0 + dt/2 k2, y4 = q0 + dt k3, and q1 = q0 + dt/6 (k1 + 2 k2 + 2 k3 + k4).
+// Two forms:
+//  * RK_Y, RK_YLAST (FP64 without boundary rows): no accumulator.  The stage
+//    inputs are kept, each in its own buffer, and the last stage forms
+//    q1 = q0 + ((y2 - q0) + 2 (y3 - q0) + (y4 - q0)) / 3 + dt/6 k4: 10 + 10 +
+//    10 + 25 words per point and step instead of 15 + 20 + 20 + 10, and three
+//    roundings at the size of q0 that enter q1 by 1/3, 2/3, 1/3 plus one, where
+//    the accumulator takes four.
+//  * RK_FIRST, RK_MID, RK_LAST: an accumulator of the arithmetic type T.
+//    FP64 (contexts with boundary rows, which change the stage inputs or need
+//    the complete RHS): the partial new state q0 + dt/6 k1 + dt/3 k2 + dt/3 k3.
+//    FP32-mixed: the increment dt/6 k1 + dt/3 k2 + dt/3 k3 alone, in FP32, and
+//    the last stage adds q0 in FP64; the increment is a step's change of the
+//    state, so its FP32 rounding is far below that of the FP32 stage inputs.
+// RK_RHS writes k into rhs instead (a single RHS evaluation).
+// The form is a template parameter: its loads then stand in one block with the
+// RHS's and are in flight together (as a runtime switch each was waited for
+// before the next was issued).
+enum RkForm { RK_FIRST = 0, RK_MID = 1, RK_LAST = 3, RK_RHS = 4, RK_Y = 5, RK_YLAST = 6 };
+
+template <typename T>
+struct RkArgs {
+  double *qn;             // q0, and q1 after the last stage
+  T *acc;                 // accumulator
+  T *out;                 // next stage input
+  const T *y2, *y3, *y4;  // RK_YLAST: the kept stage inputs
+  double dt, c;           // step, and the stage's c dt
+};
+
+// What the update of one variable reads besides k.
+template <int RK, typename T>
+struct RkIn {
+  double q0[PPT];
+  T a[PPT], b[PPT], c[PPT];
+};
+
+template <int DIR, int RK, typename T>
+__device__ __forceinline__ void rk_load(const RkArgs<T> &rk, int v, long B, long PS, long N, RkIn<RK, T> &in) {
+  if constexpr (RK == RK_RHS) return;
+  if constexpr (!(RK == RK_LAST && sizeof(T) == 8)) ld<DIR>(rk.qn + v * N, B, PS, in.q0);
+  if constexpr (RK == RK_MID || RK == RK_LAST) ld<DIR>(rk.acc + v * N, B, PS, in.a);
+  if constexpr (RK == RK_YLAST) {
+    ld<DIR>(rk.y2 + v * N, B, PS, in.a);
+    ld<DIR>(rk.y3 + v * N, B, PS, in.b);
+    ld<DIR>(rk.y4 + v * N, B, PS, in.c);
   }
 }
 
-template <int DIR, typename T>
-__device__ __forceinline__ void rk_update(int mode, int v, const T (&k)[PPT], long B, long PS,
-                                          long N, T *rhs, double *__restrict__ qn,
-                                          T *__restrict__ acc, T *qs_out, double dt) {
-  if (mode == 4) {
+// the new state q1 of the last stage
+template <int RK, typename T>
+__device__ __forceinline__ void rk_new_state(const RkArgs<T> &rk, const T (&k)[PPT], const RkIn<RK, T> &in,
+                                             double (&q1)[PPT]) {
+  const double dt = rk.dt;
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    if constexpr (RK == RK_YLAST) {
+      const double d = (in.a[m] - in.q0[m]) + __builtin_fma(2.0, in.b[m] - in.q0[m], in.c[m] - in.q0[m]);
+      q1[m] = in.q0[m] + __builtin_fma(d, 1.0 / 3.0, dt / 6.0 * k[m]);
+    } else if constexpr (sizeof(T) == 8) {
+      q1[m] = in.a[m] + dt / 6.0 * double(k[m]);
+    } else {
+      q1[m] = in.q0[m] + (double(in.a[m]) + dt / 6.0 * double(k[m]));
+    }
+  }
+}
+
+template <int DIR, int RK, typename T>
+__device__ __forceinline__ void rk_store(const RkArgs<T> &rk, int v, const T (&k)[PPT], const RkIn<RK, T> &in, long B,
+                                         long PS, long N, T *rhs) {
+  if constexpr (RK == RK_RHS) {
     st<DIR>(rhs + v * N, B, PS, k);
-    return;
-  }
-  double a[PPT];
-  if (mode == 3) {
-    rk_new_state<DIR, T>(v, k, B, PS, N, qn, acc, dt, a);
-    st<DIR>(qn + v * N, B, PS, a);
-    return;
-  }
-  double q0[PPT];
-  ld<DIR>(qn + v * N, B, PS, q0);
-  // the accumulator's value after this stage
-  const double base = sizeof(T) == 8 ? 1.0 : 0.0;  // FP32: the increment alone
-  if (mode == 0) {
-#pragma unroll
-    for (int m = 0; m < PPT; ++m) a[m] = base * q0[m] + dt / 6.0 * double(k[m]);
+  } else if constexpr (RK == RK_LAST || RK == RK_YLAST) {
+    double q1[PPT];
+    rk_new_state<RK, T>(rk, k, in, q1);
+    st<DIR>(rk.qn + v * N, B, PS, q1);
   } else {
-    ld<DIR>(acc + v * N, B, PS, a);
+    double a[PPT];
+    if constexpr (RK != RK_Y) {
+      // the accumulator's value after this stage
+      const double base = sizeof(T) == 8 ? 1.0 : 0.0;  // FP32: the increment alone
+      const double dt = rk.dt;
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) a[m] = a[m] + dt / 3.0 * double(k[m]);
+      for (int m = 0; m < PPT; ++m)
+        a[m] = RK == RK_FIRST ? base * in.q0[m] + dt / 6.0 * double(k[m]) : in.a[m] + dt / 3.0 * double(k[m]);
+      st<DIR>(rk.acc + v * N, B, PS, a);
+    }
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) a[m] = in.q0[m] + rk.c * double(k[m]);
+    st<DIR>(rk.out + v * N, B, PS, a);
   }
-  st<DIR>(acc + v * N, B, PS, a);
-  const double c_stage = mode == 2 ? dt : dt * 0.5;
+}
+
+// RK_YLAST's new state with one kept stage input live at a time, for the
+// sweeps that have no registers for three
+template <int DIR>
+__device__ __forceinline__ void rk_ylast(const RkArgs<double> &rk, int v, const double (&k)[PPT], long B, long PS,
+                                         long N, double (&q1)[PPT]) {
+  double q0[PPT], d[PPT];
+  asm volatile("" ::: "memory");
+  ld<DIR>(rk.qn + v * N, B, PS, q0);
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) a[m] = q0[m] + c_stage * double(k[m]);
-  st<DIR>(qs_out + v * N, B, PS, a);
+  for (int j = 0; j < 3; ++j) {
+    double y[PPT];
+    ld<DIR>((j == 0 ? rk.y2 : (j == 1 ? rk.y3 : rk.y4)) + v * N, B, PS, y);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      const double e = y[m] - q0[m];
+      d[m] = j == 0 ? e : __builtin_fma(j == 1 ? 2.0 : 1.0, e, d[m]);
+    }
+    asm volatile("" ::: "memory");
+  }
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) q1[m] = q0[m] + __builtin_fma(d[m], 1.0 / 3.0, rk.dt / 6.0 * k[m]);
+}
+
+// the form chosen at run time (uniform), for the sweeps whose instances are
+// not worth one per form; Y: the forms without an accumulator
+template <int DIR, typename T, bool Y>
+__device__ __forceinline__ void rk_update(int form, const RkArgs<T> &rk, int v, const T (&k)[PPT], long B, long PS,
+                                          long N, T *rhs) {
+#define CRUNA_RK(F)                                 \
+  {                                                 \
+    RkIn<F, T> in;                                  \
+    rk_load<DIR, F, T>(rk, v, B, PS, N, in);        \
+    rk_store<DIR, F, T>(rk, v, k, in, B, PS, N, rhs); \
+  }
+  if (form == RK_RHS) CRUNA_RK(RK_RHS)
+  else if constexpr (Y) {
+    if (form == RK_Y) {
+      CRUNA_RK(RK_Y)
+    } else {
+      double q1[PPT];
+      rk_ylast<DIR>(rk, v, k, B, PS, N, q1);
+      st<DIR>(rk.qn + v * N, B, PS, q1);
+    }
+  } else {
+    if (form == RK_FIRST) CRUNA_RK(RK_FIRST)
+    else if (form == RK_MID) CRUNA_RK(RK_MID)
+    else CRUNA_RK(RK_LAST)
+  }
+#undef CRUNA_RK
+}
+template <int DIR, typename T, bool Y>
+__device__ __forceinline__ void rk_final(const RkArgs<T> &rk, int v, const T (&k)[PPT], long B, long PS, long N,
+                                         double (&q1)[PPT]) {
+  if constexpr (Y) {
+    rk_ylast<DIR>(rk, v, k, B, PS, N, q1);
+  } else {
+    RkIn<RK_LAST, T> in;
+    rk_load<DIR, RK_LAST, T>(rk, v, B, PS, N, in);
+    rk_new_state<RK_LAST, T>(rk, k, in, q1);
+  }
 }
 
 // ----------------------------------------------------------------------------
 // S4 (z) / S5 (y) / S6 (x): viscous fluxes d/dx_d tau_{i d}; the x sweep also
 // adds tau:grad(u) (ns_rho_rhou_p.f90:202-205) and finishes the stage.
-// mode 0..3: RK4 stage update; mode 4: write the complete RHS into rhs.
-// FF (x sweep of the last stage, mode 3, only): also apply filter_i1 to
+// RK: the x sweep's stage update (RkForm).
+// FF (x sweep of the last stage only): also apply filter_i1 to
 // the new state before storing it (the x filter of the step loop, fused
 // because the x sweep holds complete x-lines); fop is that filter.  A
 // separate instance, so that the other stages do not carry the filter
@@ -497,13 +591,12 @@ __device__ __forceinline__ void rk_update(int mode, int v, const T (&k)[PPT], lo
 // last sweep multiplies every equation by X_jacobian and the dissipation once
 // more (ns_rho_rhou_p_grid_transform.f90:190-276).
 // EV: d/dx_d (phi tau_id), times the stored 1/phi (ns_rho_rhou_p_ev_phi.f90:161-201).
-template <typename T, int DIR, int FORM, bool FF, typename Lines>
+template <typename T, int DIR, int FORM, int RK, bool FF, typename Lines>
 __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__ rhs, const T *__restrict__ G,
                                             const Op<T> &op, const Op<T> &fop, const SweepGeom &g,
-                                            const Phys &ph, long N, int mode, double *__restrict__ qn,
-                                            T *__restrict__ acc, T *__restrict__ qs_out, double dt,
-                                            const Metric<T> &mt, const T *__restrict__ force,
-                                            const Penal<T> &pe, Lines &ln) {
+                                            const Phys &ph, long N, const RkArgs<T> &rk, const Metric<T> &mt,
+                                            const T *__restrict__ force, const Penal<T> &pe, Lines &ln) {
+  static_assert(!FF || RK == RK_LAST || RK == RK_YLAST, "the x filter follows the last stage");
   constexpr bool GT = FORM == RHS_GT, EV = FORM == RHS_EV;
   constexpr bool LAST = DIR == 0;
   const long B = tp.base, PS = g.PS;
@@ -553,60 +646,64 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
   }
   T Jv[PPT];
   if (LAST && GT) ld<DIR>(mt.J, B, PS, Jv);
-  // the last sweep's complete RHS of variable v: RK4 update, and on the
-  // final stage optionally the x filter of the new state
-  auto finish = [&](int v, T(&k)[PPT]) {
+  // the last sweep's complete RHS of variable v: what its RK4 update reads is
+  // loaded together with the RHS; on the final stage optionally the x filter
+  // of the new state
+  auto finish = [&](int v, T(&k)[PPT], const RkIn<RK, T> &in) {
+    // force (apply_force, ns_rho_rhou_p.f90:212): an additive term of the
+    // complete RHS, here the learned closure; null when there is none
+    if (force) {
+      T fv[PPT];
+      ld<DIR>(force + v * N, B, PS, fv);
+#pragma unroll
+      for (int m = 0; m < PPT; ++m) k[m] = k[m] + fv[m];
+    }
     if constexpr (FF) {
       double a[PPT];
-      rk_new_state<DIR, T>(v, k, B, PS, N, qn, acc, dt, a);
+      rk_new_state<RK, T>(rk, k, in, a);
       T f[PPT], x[PPT];
 #pragma unroll
       for (int m = 0; m < PPT; ++m) f[m] = T(a[m]);
       ln.bind(fop);
       ln.template solve<true>(fop, f, x);
       ln.bind(op);
-      st<DIR>(qn + v * N, B, PS, x);
+      st<DIR>(rk.qn + v * N, B, PS, x);
     } else {
-      rk_update<DIR, T>(mode, v, k, B, PS, N, rhs, qn, acc, qs_out, dt);
+      rk_store<DIR, RK, T>(rk, v, k, in, B, PS, N, rhs);
     }
   };
-  // each solve's result is consumed at once (z/y: read-modify-write of the
-  // momentum accumulators; x: the complete RHS of that variable and its RK4
-  // update), so only the remaining stress fields stay live across a solve;
-  // the fences keep that traffic below the solve it depends on
-  // force (apply_force, ns_rho_rhou_p.f90:212): an additive term of the
-  // complete RHS, here the learned closure; null when there is none
-  auto add_force = [&](int v, T(&k)[PPT]) {
-    if (LAST && force) {
-      T fv[PPT];
-      ld<DIR>(force + v * N, B, PS, fv);
-#pragma unroll
-      for (int m = 0; m < PPT; ++m) k[m] = k[m] + fv[m];
-    }
-  };
-  if (LAST && (mode != 4 || GT || force)) {
-    // k_1 = rhs_1 (times J) is complete already: its stage update goes first
-    T k[PPT];
+  if constexpr (LAST) {
+    // k_1 = rhs_1 (times J) and the pressure's (gamma - 1) (bracket +
+    // tau:grad(u)) (ns_rho_rhou_p.f90:200-209) are complete already: their
+    // updates go first, which frees the dissipation's registers for the solves
+    // (the last stage of the form without an accumulator reads four more
+    // fields per variable: it takes the two one after the other)
+    constexpr bool BOTH = RK != RK_YLAST;
+    T k[PPT], e[PPT];
+    RkIn<RK, T> in, ie;
     ld<DIR>(rhs, B, PS, k);
-    if (GT) {
-#pragma unroll
-      for (int m = 0; m < PPT; ++m) k[m] = Jv[m] * k[m];
+    rk_load<DIR, RK, T>(rk, 0, B, PS, N, in);
+    if (BOTH) {
+      ld<DIR>(rhs + 4 * N, B, PS, e);
+      rk_load<DIR, RK, T>(rk, 4, B, PS, N, ie);
     }
-    add_force(0, k);
-    finish(0, k);
-  }
-  if (LAST) {
-    // pressure: (gamma - 1) (bracket + tau:grad(u)) (ns_rho_rhou_p.f90:200-209),
-    // complete before the momentum solves: finishing it here frees the
-    // dissipation's registers for them
-    asm volatile("" ::: "memory");
-    T k[PPT];
-    ld<DIR>(rhs + 4 * N, B, PS, k);
+    issue_loads();
+    if (RK != RK_RHS || GT || force) {
+      if (GT) {
+#pragma unroll
+        for (int m = 0; m < PPT; ++m) k[m] = Jv[m] * k[m];
+      }
+      finish(0, k, in);
+    }
+    if (!BOTH) {
+      asm volatile("" ::: "memory");
+      ld<DIR>(rhs + 4 * N, B, PS, e);
+      rk_load<DIR, RK, T>(rk, 4, B, PS, N, ie);
+    }
 #pragma unroll
     for (int m = 0; m < PPT; ++m)
-      k[m] = GT ? (Jv[m] * T(ph.gm1)) * (k[m] + Jv[m] * diss[m]) : T(ph.gm1) * (k[m] + diss[m]);
-    add_force(4, k);
-    finish(4, k);
+      e[m] = GT ? (Jv[m] * T(ph.gm1)) * (e[m] + Jv[m] * diss[m]) : T(ph.gm1) * (e[m] + diss[m]);
+    finish(4, e, ie);
     asm volatile("" ::: "memory");
   }
   T IP[PPT];
@@ -621,37 +718,66 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
       t3[m] = PH[m] * t3[m];
     }
   }
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    T x[PPT];
-    ln.solve(op, i == 0 ? t1 : (i == 1 ? t2 : t3), x);
-    asm volatile("" ::: "memory");
-    T k[PPT];
-    ld<DIR>(rhs + (1 + i) * N, B, PS, k);
+  // z/y: read-modify-write of the momentum accumulators; x: the complete RHS
+  // of that variable and its RK4 update
+  auto complete = [&](int v, const T(&x)[PPT], T(&k)[PPT], const RkIn<RK, T> &in) {
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       k[m] = k[m] + (EV ? IP[m] * (x[m] * ih) : x[m] * ih);
       if (LAST && GT) k[m] = Jv[m] * k[m];
     }
-    if (!LAST) {
-      st<DIR>(rhs + (1 + i) * N, B, PS, k);
-    } else {
-      add_force(1 + i, k);
-      finish(1 + i, k);
+    if constexpr (LAST)
+      finish(v, k, in);
+    else
+      st<DIR>(rhs + v * N, B, PS, k);
+  };
+  {
+    // two stresses at once, the first accumulator in flight meanwhile
+    T x[PPT], y[PPT], k[PPT];
+    RkIn<RK, T> in;
+    constexpr bool EARLY = RK != RK_YLAST;
+    if (EARLY) {
+      ld<DIR>(rhs + N, B, PS, k);
+      if constexpr (LAST) rk_load<DIR, RK, T>(rk, 1, B, PS, N, in);
     }
+    ln.solve2(op, t1, x, t2, y);
+    asm volatile("" ::: "memory");
+    if (!EARLY) {
+      ld<DIR>(rhs + N, B, PS, k);
+      if constexpr (LAST) rk_load<DIR, RK, T>(rk, 1, B, PS, N, in);
+    }
+    complete(1, x, k, in);
+    asm volatile("" ::: "memory");
+    ld<DIR>(rhs + 2 * N, B, PS, k);
+    if constexpr (LAST) rk_load<DIR, RK, T>(rk, 2, B, PS, N, in);
+    complete(2, y, k, in);
+  }
+  {
+    T x[PPT], k[PPT];
+    RkIn<RK, T> in;
+    asm volatile("" ::: "memory");
+    if (RK != RK_YLAST) {
+      ld<DIR>(rhs + 3 * N, B, PS, k);
+      if constexpr (LAST) rk_load<DIR, RK, T>(rk, 3, B, PS, N, in);
+    }
+    ln.solve(op, t3, x);
+    if (RK == RK_YLAST) {
+      asm volatile("" ::: "memory");
+      ld<DIR>(rhs + 3 * N, B, PS, k);
+      if constexpr (LAST) rk_load<DIR, RK, T>(rk, 3, B, PS, N, in);
+    }
+    complete(3, x, k, in);
   }
 }
 
-template <typename T, int DIR, bool PER, int FORM, bool FF>
+template <typename T, int DIR, bool PER, int FORM, int RK, bool FF>
 __global__ __launch_bounds__(sweep_nt<T>()) void k_sweep2(T *__restrict__ rhs, const T *__restrict__ G,
                                                           Op<T> op, Op<T> fop, SweepGeom g, Phys ph,
-                                                          long N, int mode, double *__restrict__ qn,
-                                                          T *__restrict__ acc, T *__restrict__ qs_out,
-                                                          double dt, Metric<T> mt, const T *__restrict__ force,
-                                                          Penal<T> pe) {
+                                                          long N, RkArgs<T> rk, Metric<T> mt,
+                                                          const T *__restrict__ force, Penal<T> pe) {
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER, sweep_nt<T>()>(op, tp);
-  sweep2_body<T, DIR, FORM, FF>(tp, rhs, G, op, fop, g, ph, N, mode, qn, acc, qs_out, dt, mt, force, pe, ln);
+  sweep2_body<T, DIR, FORM, RK, FF>(tp, rhs, G, op, fop, g, ph, N, rk, mt, force, pe, ln);
 }
 
 // S3 + S4: the z first-derivative sweep and the z viscous sweep as one
@@ -711,8 +837,7 @@ __global__ __launch_bounds__(NT) void k_sweep12_z(const Q *__restrict__ qs, T *_
   } else {
     sweep1_body<T, Q, 2, FORM>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln);
     asm volatile("" ::: "memory");
-    sweep2_body<T, 2, FORM, false>(tp, rhs, G, op, op, g, ph, N, 0, nullptr, nullptr, nullptr, 0.0, mt, nullptr, pe,
-                                   ln);
+    sweep2_body<T, 2, FORM, RK_RHS, false>(tp, rhs, G, op, op, g, ph, N, RkArgs<T>{}, mt, nullptr, pe, ln);
   }
 }
 
