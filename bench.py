@@ -42,35 +42,32 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0
 # closure network: multiply-adds per point of its four 3x3x3 convolutions
 # over the real channels (5 -> 32 -> 32 -> 32 -> 5)
 CLOSURE_MACS_PER_POINT = 27 * (5 * 32 + 32 * 32 + 32 * 32 + 32 * 5)
-# Algorithmic FP64-equivalent words per grid point and launch (compulsory
-# reads + writes of each sweep; FP32-mixed fields count as half words).
+# Algorithmic words per grid point and launch (compulsory reads + writes of
+# each sweep), FP64 step: the y and z sweeps leave the stresses, so that the
+# viscous sweeps read two (y) and three (x) fields, and the stage inputs are
+# kept instead of an accumulator.
 SWEEP_WORDS = {
     "sweep1_x": 14.0,
     "sweep1_y": 20.0,
-    "sweep1_z": 21.0,
-    "sweep2_z": 12.0,
-    "sweep2_y": 12.0,
-    "sweep2_x_rk": 28.25,  # mean over the four stages: 27, 32, 32, 22
-    # sweep1_z and sweep2_z fused (k_sweep12_z): sweep1_z's 21 words and the
-    # two velocity gradients (u_x, v_y) that only the viscous part reads; the
-    # other gradients, the viscosity and the momentum RHS pass between the
-    # parts in registers and LDS
-    "sweep12_z": 23.0,
+    "sweep12_z": 24.0,
+    "sweep2_y": 6.0,
+    "sweep2_x_rk": 21.75,  # mean over the four stages: 18, 18, 18, 33
     "filter_x": 10.0,
     "filter_y": 10.0,
     "filter_z": 10.0,
     # adjoint sweeps: q and qs read, rhs written (z) or read-modify-written;
-    # the x sweep also carries the RK4 tail (30, 35, 35, 25 words)
+    # the x sweep also carries the RK4 tail (25, 25, 25, 40 words)
     "asweep_z": 15.0,
     "asweep_y": 20.0,
-    "asweep_x_rk": 31.25,
+    "asweep_x_rk": 28.75,
 }
-# words of each sweep that are stage-state / RHS / gradient fields held in the
-# compute precision (the rest are FP64 state or accumulator words)
-SWEEP_COMPUTE_WORDS = {
-    "sweep1_x": 14.0, "sweep1_y": 20.0, "sweep1_z": 21.0, "sweep2_z": 12.0, "sweep2_y": 12.0,
-    "sweep12_z": 23.0, "sweep2_x_rk": 15.75, "filter_x": 0.0, "filter_y": 0.0, "filter_z": 0.0,
-    "asweep_z": 5.0, "asweep_y": 10.0, "asweep_x_rk": 12.5,
+# FP32-mixed step: words, and those of them in the compute precision
+# (stage-state, RHS and gradient fields, accumulator; the rest are FP64 state).
+# The z sweeps pass the gradients, the viscosity and the momentum RHS between
+# their two parts in registers and LDS.
+SWEEP_WORDS_32 = {
+    "sweep1_x": (14.0, 14.0), "sweep1_y": (20.0, 20.0), "sweep12_z": (23.0, 23.0), "sweep2_y": (12.0, 12.0),
+    "sweep2_x_rk": (28.25, 15.75), "filter_x": (10.0, 0.0), "filter_y": (10.0, 0.0), "filter_z": (10.0, 0.0),
 }
 # The step-level byte model of the reference's dependency graph (4624 B per
 # point per FP64 RK4 step incl. filtering; 2672 B in FP32-mixed).
@@ -81,19 +78,18 @@ MODEL_BYTES = {"f64": 4624.0, "fp32-mixed": 2672.0}
 # fields written (x, also mu) or read-modify-written (y, z); viscous z/y:
 # metric row 3 + J + mu + 3 temperature gradients + 6 velocity gradients, 4
 # RHS fields read-modify-written; viscous x: the same 14 + 5 RHS read + the
-# RK4 tail (mean of 15, 20, 20, 10 words over the stages).
+# RK4 tail (mean of 10, 10, 10, 25 words over the stages).
 CURV_WORDS = {"sweep1_x": 23.0, "sweep1_y": 36.0, "sweep1_z": 36.0, "sweep2_z": 22.0,
-              "sweep2_y": 22.0, "sweep2_x_rk": 35.25, "filter_x": 10.0, "filter_y": 10.0,
+              "sweep2_y": 22.0, "sweep2_x_rk": 32.75, "filter_x": 10.0, "filter_y": 10.0,
               "filter_z": 10.0}
 # per point and FP64 step: four stages of the six sweeps and three filter passes
-CURV_MODEL_BYTES = 8.0 * (4 * (23 + 36 + 36 + 22 + 22 + 35.25) + 30)
+CURV_MODEL_BYTES = 8.0 * (4 * (23 + 36 + 36 + 22 + 22 + 32.75) + 30)
 
 
 def kernel_bytes_per_point(name, mixed):
-    words = SWEEP_WORDS[name]
     if not mixed:
-        return 8.0 * words
-    cw = SWEEP_COMPUTE_WORDS[name]
+        return 8.0 * SWEEP_WORDS[name]
+    words, cw = SWEEP_WORDS_32[name]
     return 4.0 * cw + 8.0 * (words - cw)
 
 

@@ -74,8 +74,12 @@ __global__ __launch_bounds__(NT) void kb_sweep1(const BatchMember *__restrict__ 
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.geom[DIR], blockIdx.x - L->start[e]);
   auto ln = make_lines<double, PER>(b.op[DIR], tp);
-  sweep1_body<double, double, DIR, RHS_CART>(tp, stage_in(b, b.qn, stage), b.rhs, b.G, b.op[DIR], b.geom[DIR], b.ph, b.N,
-                                             Metric<double>{}, Penal<double>{}, ln);
+  const double *qs = stage_in(b, b.qn, stage);
+  if constexpr (DIR == 1)
+    sweep1_y_stress(tp, qs, b.rhs, b.G, b.op[1], b.geom[1], b.ph, b.N, ln);
+  else
+    sweep1_body<double, double, DIR, RHS_CART>(tp, qs, b.rhs, b.G, b.op[DIR], b.geom[DIR], b.ph, b.N, Metric<double>{},
+                                               Penal<double>{}, ln);
 }
 
 // viscous sweep; the x sweep finishes RK stage `stage` (FF: the last stage
@@ -100,11 +104,7 @@ __global__ __launch_bounds__(NT) void kb_sweep12_z(const BatchMember *__restrict
   const BatchMember &b = M[L->mem[e]];
   const ThreadPos tp = thread_pos_tile<2, true>(b.geom[2], blockIdx.x - L->start[e]);
   auto ln = make_lines<double, PER>(b.op[2], tp);
-  ZCarry<double> zc;
-  z_carry_slots(zc);
-  sweep1_body<double, double, 2, RHS_CART, true>(tp, stage_in(b, b.qn, stage), b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N,
-                                                 Metric<double>{}, Penal<double>{}, ln, &zc);
-  viscous_z_carry<double>(tp, b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N, ln, zc);
+  sweep12_z_stress(tp, stage_in(b, b.qn, stage), b.rhs, b.G, b.op[2], b.geom[2], b.ph, b.N, ln);
 }
 
 // filter of the direct (adj = 0) or adjoint state in place

@@ -627,7 +627,7 @@ void launch_curv_sweep1(cruna_hip_ctx *c, const Q *in) {
 template <typename T, typename Q, int FORM>
 void launch_sweep12z_form(cruna_hip_ctx *c, const Q *in) {
   const dim3 grid(c->geom[2].ntiles), block(c->wg[2]);
-  const size_t lds = z_lds_bytes<T>(c->wg[2], FORM == RHS_CART);
+  const size_t lds = stress_form<T, FORM>() ? z_stress_lds_bytes(c->wg[2]) : line_lds_bytes<T>(c->wg[2]);
   T *rhs = (T *)c->rhs, *G = (T *)c->G;
   const Op<T> &op = dops<T>(c)[2].op;
   if (c->cfg.scheme[2] == CRUNA_HIP_PERIODIC)
@@ -2467,7 +2467,6 @@ struct BatchSlot {
                          LDS((S).bb().wg[grp][kind][d]), (S).s, (S).mem(), (S).list(grp, kind, d),       \
                          __VA_ARGS__);                                                                   \
   } while (0)
-inline size_t batch_z_lds(int threads) { return z_lds_bytes<double>(threads, true); }
 
 template <int DIR>
 void batch_sweep1(const BatchSlot &S, int stage) {
@@ -2476,8 +2475,8 @@ void batch_sweep1(const BatchSlot &S, int stage) {
 }
 
 void batch_sweep12z(const BatchSlot &S, int stage) {
-  if (S.e->bper[2]) BATCH_LAUNCH(S, 0, 0, 2, batch_z_lds, (kb_sweep12_z<true>), stage);
-  else BATCH_LAUNCH(S, 0, 0, 2, batch_z_lds, (kb_sweep12_z<false>), stage);
+  if (S.e->bper[2]) BATCH_LAUNCH(S, 0, 0, 2, z_stress_lds_bytes, (kb_sweep12_z<true>), stage);
+  else BATCH_LAUNCH(S, 0, 0, 2, z_stress_lds_bytes, (kb_sweep12_z<false>), stage);
 }
 
 template <int DIR, int RK, bool FF>

@@ -110,6 +110,7 @@ inline HostRecOp build_rec_op(OpKind kind, bool per, int n_real, double alpha) {
   op.M = 1;
   for (double r = op.rho; r > 0x1p-55; r *= op.rho) ++op.M;
   op.slow = op.M > REC_WIN ? 1 : 0;
+  if (op.slow && kind != OP_FILTER) throw std::runtime_error("a derivative that decays too slowly");
   if (op.slow) {
     const int most = per ? op.NB : op.NB - 1;
     if (op.M > most) {

@@ -428,13 +428,15 @@ struct RecLines {
   }
   __device__ __forceinline__ void sync() const { line_sync(wave_line); }
 
-  // sum_m rho^m value(block b -+ (1 + m)) of cell
+  // sum_m rho^m value(block b -+ (1 + m)) of cell (the derivatives' mu never
+  // needs more than REC_WIN terms)
+  template <bool FILT>
   __device__ __forceinline__ double window(const RecOp &op, const int (&at)[REC_WIN], int dir, int cell) const {
 #pragma clang fp contract(off)
     double v[REC_WIN];
 #pragma unroll
     for (int m = 0; m < REC_WIN; ++m) v[m] = get(at[m], cell);
-    if (!op.slow) {
+    if (!FILT || !op.slow) {
       double s = v[REC_WIN - 1];
 #pragma unroll
       for (int m = REC_WIN - 2; m >= 0; --m) s = __builtin_fma(s, op.rho, v[m]);
@@ -515,7 +517,7 @@ struct RecLines {
     sync();
 #pragma unroll
     for (int v = 0; v < NF; ++v) {
-      const double U = window(op, lf, -1, REC_UL + v);
+      const double U = window<FILT>(op, lf, -1, REC_UL + v);
 #pragma unroll
       for (int i = 0; i < PPT; ++i) x[v][i] = __builtin_fma(op.lp[i], U, x[v][i]);
       if (!PER && op.zrow[1] != 0) {  // nothing comes back from behind the last point
@@ -532,7 +534,7 @@ struct RecLines {
     sync();
 #pragma unroll
     for (int v = 0; v < NF; ++v) {
-      const double X = window(op, rt, +1, REC_XF + v);
+      const double X = window<FILT>(op, rt, +1, REC_XF + v);
 #pragma unroll
       for (int i = 0; i < PPT; ++i) x[v][i] = __builtin_fma(op.lp[PPT - 1 - i], X, x[v][i]);
     }

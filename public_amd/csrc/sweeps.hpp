@@ -24,6 +24,17 @@
 // (each sum is completed by the second sweep that contributes to it; the
 // result equals the reference's u_y + v_x etc. bit for bit).  S1 x evaluates
 // the viscosity law once per point and stage; S2, S3 and S4-S6 read it.
+//
+// FP64 Cartesian form (sweep1_y_stress, sweep12_z_stress): the later sweeps need the
+// stresses, not the gradients, so a gradient field turns into a stress where
+// it is complete: S2 y stores tau_12 (G3) and takes its y derivative at once, S3
+// z stores tau_11, tau_22, tau_13, tau_23 (G0, G1, G4, G5), and each adds its part of
+// tau:grad(u) to the pressure bracket.  S5 y then reads two fields and S6 x
+// three, without the viscosity: 20 + 24 + 6 + 8 words per point and stage in
+// S2, S3+S4, S5, S6 (before the RK update) instead of 20 + 23 + 12 + 12 (256^3, per
+// stage: S5 0.327 -> 0.158 ms, S6 with the shorter update 0.836 -> 0.478, S3+S4
+// 0.664 -> 0.688; the step 11.4 -> 10.3 ms).  Not in FP32, whose bits depend on the order of these sums, nor in the deformed-grid
+// and penalised forms.
 #pragma once
 
 #include "line_solve.hpp"
@@ -229,35 +240,12 @@ constexpr int sweep_nt() { return sizeof(T) == 4 ? NT_SWEEP32 : NT; }
 // z sweep completes (s13 = u_z + w_x, s23 = v_z + w_y, w_z) and the
 // viscosity in registers; the momentum RHS of the block in LDS (the thread's
 // own slots) instead of a store and a reload through HBM.
-// In FP64 the slots are thread-major with a stride of 25 values (odd: no bank
-// conflicts) in the dynamic LDS behind the line engine's; in FP32 a static
-// array.
-constexpr int ZC_STRIDE = 3 * PPT + 1;
 template <typename T>
 struct ZCarry {
   T s13[PPT], s23[PPT], wz[PPT], mu[PPT];
-  T *slots;   // LDS: momentum RHS (x, y, z) of the block
-  int tid;
-  __device__ __forceinline__ T &mom(int i, int m) const {
-    return sizeof(T) == 8 ? slots[i * PPT + m] : slots[(i * PPT + m) * NT + tid];
-  }
+  T (*slots)[PPT][NT];  // LDS: [3][PPT][NT] momentum RHS (x, y, z)
+  __device__ __forceinline__ T &mom(int i, int m) const { return slots[i][m][threadIdx.x]; }
 };
-template <typename T>
-__device__ __forceinline__ void z_carry_slots(ZCarry<T> &zc) {
-  zc.tid = threadIdx.x;
-  if constexpr (sizeof(T) == 8) {
-    zc.slots = reinterpret_cast<double *>(line_dyn) + (blockDim.x + 1) * REC_STRIDE + threadIdx.x * ZC_STRIDE;
-  } else {
-    __shared__ T mom[3 * PPT * NT];
-    zc.slots = mom;
-  }
-}
-// dynamic LDS of the fused z kernel in a work-group of `threads`
-template <typename T>
-size_t z_lds_bytes(int threads, bool carry) {
-  return line_lds_bytes<T>(threads) + (sizeof(T) == 8 && carry ? (size_t)threads * ZC_STRIDE * sizeof(double) : 0);
-}
-
 
 template <typename T, typename Q, int DIR, int FORM, bool FUSE = false, typename Lines>
 __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__restrict__ qs, T *__restrict__ rhs,
@@ -411,13 +399,245 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
   st<DIR>(rhs + 4 * N, B, PS, e);
 }
 
+template <typename T, int FORM>
+constexpr bool stress_form() { return sizeof(T) == 8 && FORM == RHS_CART; }
+
+// S2 y in the stress form: the first-derivative sweep along y with tau_12.
+template <typename Lines>
+__device__ __forceinline__ void sweep1_y_stress(const ThreadPos &tp, const double *__restrict__ qs,
+                                                double *__restrict__ rhs, double *__restrict__ G, const RecOp &op,
+                                                const SweepGeom &g, const Phys &ph, long N, Lines &ln) {
+  const long B = tp.base, PS = g.PS;
+  const double ih = ph.inv_h[1], hh = ph.heat_inv_h[1];
+  double irho[PPT], mom[PPT], p[PPT], mu[PPT], f[PPT], u[PPT], x[PPT], y[PPT], r[PPT], e[PPT], lt[PPT];
+  ld<1>(qs, B, PS, irho);
+  ld<1>(qs + 2 * N, B, PS, mom);
+  ld<1>(qs + 4 * N, B, PS, p);
+  ld<1>(qs + N, B, PS, u);
+  ld<1>(G + 3 * N, B, PS, r);  // v_x
+  ld<1>(G + 6 * N, B, PS, mu);
+  issue_loads();
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    irho[m] = 1.0 / irho[m];
+    u[m] = u[m] * irho[m];
+    f[m] = temperature(ph, irho[m], p[m]);
+  }
+  // u_y, which completes tau_12, and the inner derivative of the heat flux
+  ln.solve2(op, u, x, f, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    const double s12 = __builtin_fma(x[m], ih, r[m]);
+    x[m] = mu[m] * s12;  // tau_12
+    e[m] = x[m] * s12;   // its part of tau:grad(u)
+    lt[m] = lambda_of(ph, mu[m]) * (y[m] * hh);
+    f[m] = mom[m] * u[m];
+  }
+  materialize(e);
+  materialize(lt);
+  st<1>(G + 3 * N, B, PS, x);
+  ld<1>(rhs + N, B, PS, r);
+  // rho u: -d(rho v u)/dy + d(tau_12)/dy
+  ln.solve2(op, x, u, f, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) r[m] = r[m] + (u[m] - y[m]) * ih;
+  st<1>(rhs + N, B, PS, r);
+  asm volatile("" ::: "memory");
+  // w_y and rho w
+  ld<1>(qs + 3 * N, B, PS, u);
+  ld<1>(rhs + 3 * N, B, PS, r);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    u[m] = u[m] * irho[m];
+    f[m] = mom[m] * u[m];
+  }
+  ln.solve2(op, u, x, f, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    x[m] = x[m] * ih;
+    r[m] = __builtin_fma(-y[m], ih, r[m]);
+  }
+  st<1>(G + 5 * N, B, PS, x);
+  st<1>(rhs + 3 * N, B, PS, r);
+  asm volatile("" ::: "memory");
+  // v_y and mass
+  ld<1>(rhs, B, PS, r);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) u[m] = mom[m] * irho[m];
+  ln.solve2(op, u, x, mom, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    x[m] = x[m] * ih;
+    r[m] = __builtin_fma(-y[m], ih, r[m]);
+  }
+  st<1>(G + N, B, PS, x);
+  st<1>(rhs, B, PS, r);
+  asm volatile("" ::: "memory");
+  // p_y and rho v
+  ld<1>(rhs + 2 * N, B, PS, r);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) f[m] = mom[m] * u[m];
+  ln.solve2(op, p, x, f, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    r[m] = r[m] - (x[m] + y[m]) * ih;
+    e[m] = __builtin_fma(u[m], x[m] * ih, e[m]);  // u.grad(p)
+    f[m] = p[m] * u[m];
+  }
+  st<1>(rhs + 2 * N, B, PS, r);
+  asm volatile("" ::: "memory");
+  // pressure bracket
+  ld<1>(rhs + 4 * N, B, PS, r);
+  ln.solve2(op, f, x, lt, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    e[m] = __builtin_fma(-ph.gt, x[m] * ih, e[m]);
+    r[m] = r[m] + __builtin_fma(y[m], hh, e[m]);
+  }
+  st<1>(rhs + 4 * N, B, PS, r);
+}
+
+// S3 + S4 z in the stress form: the first-derivative sweep along z, the stresses
+// and their z derivatives.  The z sweep is the last first-derivative sweep of a
+// stage, so the gradients of the thread's block are complete in it.  The
+// momentum RHS of x and y wait in LDS (the thread's own slots, stride 17: odd,
+// no bank conflicts) for the last two solves.
+constexpr int ZS_STRIDE = 2 * PPT + 1;
+inline size_t z_stress_lds_bytes(int threads) {
+  return rec_lds_bytes(threads) + (size_t)threads * ZS_STRIDE * sizeof(double);
+}
+template <typename Lines>
+__device__ __forceinline__ void sweep12_z_stress(const ThreadPos &tp, const double *__restrict__ qs,
+                                                 double *__restrict__ rhs, double *__restrict__ G, const RecOp &op,
+                                                 const SweepGeom &g, const Phys &ph, long N, Lines &ln) {
+  const long B = tp.base, PS = g.PS;
+  const double ih = ph.inv_h[2], hh = ph.heat_inv_h[2];
+  double *slot = reinterpret_cast<double *>(line_dyn) + (blockDim.x + 1) * REC_STRIDE + threadIdx.x * ZS_STRIDE;
+  double mom[PPT], w[PPT], p[PPT], t1[PPT], t2[PPT], t3[PPT], e[PPT], lt[PPT];
+  {
+    double irho[PPT], f[PPT], u[PPT], x[PPT], y[PPT], r[PPT], sx[PPT];
+    ld<2>(qs, B, PS, irho);
+    ld<2>(qs + 3 * N, B, PS, mom);
+    // u_z (+ w_x), v_z (+ w_y) and the momentum fluxes rho w u, rho w v
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      ld<2>(qs + (1 + i) * N, B, PS, u);
+      ld<2>(G + (4 + i) * N, B, PS, sx);
+      ld<2>(rhs + (1 + i) * N, B, PS, r);
+      issue_loads();
+#pragma unroll
+      for (int m = 0; m < PPT; ++m) {
+        if (i == 0) irho[m] = 1.0 / irho[m];
+        u[m] = u[m] * irho[m];
+        f[m] = mom[m] * u[m];
+      }
+      ln.solve2(op, u, x, f, y);
+#pragma unroll
+      for (int m = 0; m < PPT; ++m) {
+        (i == 0 ? t1 : t2)[m] = __builtin_fma(x[m], ih, sx[m]);
+        slot[i * PPT + m] = __builtin_fma(-y[m], ih, r[m]);
+      }
+      asm volatile("" ::: "memory");
+    }
+    // w_z and the inner derivative of the heat flux
+    ld<2>(qs + 4 * N, B, PS, p);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      w[m] = mom[m] * irho[m];
+      f[m] = temperature(ph, irho[m], p[m]);
+    }
+    ln.solve2(op, w, t3, f, lt);
+  }
+  asm volatile("" ::: "memory");
+  {
+    // the stresses (ns_rho_rhou_p.f90:115-128) and tau:grad(u) without tau_12
+    double ux[PPT], vy[PPT], mu[PPT];
+    ld<2>(G + 6 * N, B, PS, mu);
+    ld<2>(G, B, PS, ux);
+    ld<2>(G + N, B, PS, vy);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      const double s13 = t1[m], s23 = t2[m], wz = t3[m] * ih;
+      const double md = -2.0 / 3.0 * mu[m] * (ux[m] + vy[m] + wz);
+      const double m2 = 2.0 * mu[m];
+      const double t11 = __builtin_fma(m2, ux[m], md), t22 = __builtin_fma(m2, vy[m], md);
+      t1[m] = mu[m] * s13;
+      t2[m] = mu[m] * s23;
+      t3[m] = __builtin_fma(m2, wz, md);
+      e[m] = __builtin_fma(
+          t11, ux[m], __builtin_fma(t22, vy[m], __builtin_fma(t3[m], wz, __builtin_fma(t1[m], s13, t2[m] * s23))));
+      lt[m] = lambda_of(ph, mu[m]) * (lt[m] * hh);
+      ux[m] = t11;
+      vy[m] = t22;
+    }
+    materialize(e);
+    materialize(lt);
+    materialize(t3);
+    st<2>(G, B, PS, ux);
+    st<2>(G + N, B, PS, vy);
+    st<2>(G + 4 * N, B, PS, t1);
+    st<2>(G + 5 * N, B, PS, t2);
+  }
+  {
+    // z derivatives of tau_13 and tau_23 complete the x and y momentum
+    double x[PPT], y[PPT];
+    ln.solve2(op, t1, x, t2, y);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      x[m] = __builtin_fma(x[m], ih, slot[m]);
+      y[m] = __builtin_fma(y[m], ih, slot[PPT + m]);
+    }
+    st<2>(rhs + N, B, PS, x);
+    st<2>(rhs + 2 * N, B, PS, y);
+  }
+  asm volatile("" ::: "memory");
+  {
+    // mass and the heat flux
+    double x[PPT], r[PPT];
+    ld<2>(rhs, B, PS, r);
+    ln.solve2(op, mom, x, lt, t1);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      r[m] = __builtin_fma(-x[m], ih, r[m]);
+      e[m] = __builtin_fma(t1[m], hh, e[m]);
+    }
+    st<2>(rhs, B, PS, r);
+  }
+  asm volatile("" ::: "memory");
+  {
+    // rho w: p_z, d(tau_33)/dz, the flux; and the pressure bracket
+    double f[PPT], x[PPT], y[PPT], r[PPT], q[PPT];
+    ld<2>(rhs + 3 * N, B, PS, r);
+    ln.solve2(op, p, x, t3, y);
+    ld<2>(rhs + 4 * N, B, PS, q);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      e[m] = __builtin_fma(w[m], x[m] * ih, e[m]);
+      r[m] = __builtin_fma(y[m] - x[m], ih, r[m]);
+      f[m] = mom[m] * w[m];
+      p[m] = p[m] * w[m];
+    }
+    ln.solve2(op, f, x, p, y);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      r[m] = __builtin_fma(-x[m], ih, r[m]);
+      q[m] = q[m] + __builtin_fma(-ph.gt, y[m] * ih, e[m]);
+    }
+    st<2>(rhs + 3 * N, B, PS, r);
+    st<2>(rhs + 4 * N, B, PS, q);
+  }
+}
+
 template <typename T, typename Q, int DIR, bool PER, int FORM>
 __global__ __launch_bounds__(NT) void k_sweep1(const Q *__restrict__ qs, T *__restrict__ rhs,
                                                           T *__restrict__ G, Op<T> op, SweepGeom g,
                                                           Phys ph, long N, Metric<T> mt, Penal<T> pe) {
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER>(op, tp);
-  sweep1_body<T, Q, DIR, FORM>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln);
+  if constexpr (DIR == 1 && stress_form<T, FORM>())
+    sweep1_y_stress(tp, qs, rhs, G, op, g, ph, N, ln);
+  else
+    sweep1_body<T, Q, DIR, FORM>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln);
 }
 
 // RK4 stage update of a variable from its complete RHS k (rk_o4_e.f90:45-50,
@@ -601,8 +821,14 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
   constexpr bool LAST = DIR == 0;
   const long B = tp.base, PS = g.PS;
   const T ih = GT ? T(ph.inv_h[DIR]) * mt.m[DIR][tp.lidx] : T(ph.inv_h[DIR]);
+  constexpr bool ST = stress_form<T, FORM>();
   T t1[PPT], t2[PPT], t3[PPT], diss[PPT];
-  {
+  if constexpr (ST) {
+    // tau_11, tau_12, tau_13 (x) or tau_22, tau_23 (y)
+    if (LAST) ld<DIR>(G, B, PS, t1);
+    ld<DIR>(G + (LAST ? 3 : 1) * N, B, PS, t2);
+    ld<DIR>(G + (LAST ? 4 : 5) * N, B, PS, t3);
+  } else {
     T mu[PPT], ux[PPT], vy[PPT], wz[PPT], sa[PPT], sb[PPT];
     ld<DIR>(G + 6 * N, B, PS, mu);
     ld<DIR>(G + 0 * N, B, PS, ux);
@@ -702,7 +928,7 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     }
 #pragma unroll
     for (int m = 0; m < PPT; ++m)
-      e[m] = GT ? (Jv[m] * T(ph.gm1)) * (e[m] + Jv[m] * diss[m]) : T(ph.gm1) * (e[m] + diss[m]);
+      e[m] = GT ? (Jv[m] * T(ph.gm1)) * (e[m] + Jv[m] * diss[m]) : T(ph.gm1) * (ST ? e[m] : e[m] + diss[m]);
     finish(4, e, ie);
     asm volatile("" ::: "memory");
   }
@@ -731,6 +957,16 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     else
       st<DIR>(rhs + v * N, B, PS, k);
   };
+  if constexpr (ST && !LAST) {
+    T x[PPT], y[PPT], k[PPT], l[PPT];
+    const RkIn<RK, T> none{};
+    ld<DIR>(rhs + 2 * N, B, PS, k);
+    ld<DIR>(rhs + 3 * N, B, PS, l);
+    ln.solve2(op, t2, x, t3, y);
+    complete(2, x, k, none);
+    complete(3, y, l, none);
+    return;
+  }
   {
     // two stresses at once, the first accumulator in flight meanwhile
     T x[PPT], y[PPT], k[PPT];
@@ -785,10 +1021,11 @@ __global__ __launch_bounds__(sweep_nt<T>()) void k_sweep2(T *__restrict__ rhs, c
 // first-derivative sweep of a stage, so once a thread has completed the
 // velocity gradients of its block (w_z, u_z + w_x, v_z + w_y) the stresses
 // of the block are known and the viscous z derivatives can follow at once.
-// Cartesian form: the gradients and the viscosity stay in registers and the
-// momentum RHS in LDS between the two parts (ZCarry), so the viscous part
-// reads only u_x and v_y and writes the momentum RHS once; the deformed-grid
-// and penalised forms run the two sweep bodies one after the other.
+// FP64 Cartesian form: sweep12_z_stress.  FP32 Cartesian form: the gradients and
+// the viscosity stay in registers and the momentum RHS in LDS between the two
+// parts (ZCarry), so the viscous part reads only u_x and v_y and writes the
+// momentum RHS once.  The deformed-grid and penalised forms run the two sweep
+// bodies one after the other.
 template <typename T, typename Lines>
 __device__ __forceinline__ void viscous_z_carry(const ThreadPos &tp, T *__restrict__ rhs, const T *__restrict__ G,
                                                 const Op<T> &op, const SweepGeom &g, const Phys &ph, long N,
@@ -829,9 +1066,12 @@ __global__ __launch_bounds__(NT) void k_sweep12_z(const Q *__restrict__ qs, T *_
                                                    long N, Metric<T> mt, Penal<T> pe) {
   const ThreadPos tp = thread_pos<2>(g);
   auto ln = make_lines<T, PER>(op, tp);
-  if constexpr (FORM == RHS_CART) {
+  if constexpr (stress_form<T, FORM>()) {
+    sweep12_z_stress(tp, qs, rhs, G, op, g, ph, N, ln);
+  } else if constexpr (FORM == RHS_CART) {
+    __shared__ T mom[3][PPT][NT];
     ZCarry<T> zc;
-    z_carry_slots(zc);
+    zc.slots = mom;
     sweep1_body<T, Q, 2, FORM, true>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln, &zc);
     viscous_z_carry<T>(tp, rhs, G, op, g, ph, N, ln, zc);
   } else {
