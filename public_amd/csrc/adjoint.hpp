@@ -29,29 +29,39 @@
 
 namespace cruna {
 
+// In FP64, a product that is about to be added to another product: which of the
+// two a compiler fuses into the addition may differ between the kernels that
+// this sweep is inlined into (the batched ones give the same bits).
+template <typename T>
+__device__ __forceinline__ void pin(T (&a)[PPT]) {
+  if constexpr (sizeof(T) == 8) materialize(a);
+}
+
 // Hand the accumulated variable v on: intermediate sweeps store it; the last
 // sweep adds g and applies the RK4 stage update.
-template <int DIR, typename T, bool LAST, int RK>
-__device__ __forceinline__ void finish(int v, T (&r)[PPT], long B, long PS, long N, T *__restrict__ rhs,
+template <bool LAST, int RK, typename T, typename IO>
+__device__ __forceinline__ void finish(int v, T (&r)[PPT], const IO &io, long N, T *__restrict__ rhs,
                                        const double *__restrict__ gobj, const RkArgs<T> &rk) {
   if constexpr (!LAST) {
-    st<DIR>(rhs + v * N, B, PS, r);
+    io.st(rhs + v * N, r);
   } else {
     RkIn<RK, T> in;
-    if constexpr (RK != RK_YLAST) rk_load<DIR, RK, T>(rk, v, B, PS, N, in);
+    if constexpr (RK != RK_YLAST) rk_load<RK, T>(rk, v, io, N, in);
     if (gobj) {
       double gg[PPT];
-      ld<DIR>(gobj + v * N, B, PS, gg);
+      io.ld(gobj + v * N, gg);
+      io.got(gg);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) r[m] = r[m] + T(gg[m]);
     }
     if constexpr (RK == RK_YLAST) {
       double q1[PPT];
       materialize(r);
-      rk_ylast<DIR>(rk, v, r, B, PS, N, q1);
-      st<DIR>(rk.qn + v * N, B, PS, q1);
+      rk_ylast(rk, v, r, io, N, q1);
+      io.st(rk.qn + v * N, q1);
     } else {
-      rk_store<DIR, RK, T>(rk, v, r, in, B, PS, N, rhs);
+      rk_got<RK, T>(io, in);
+      rk_store<RK, T>(rk, v, r, in, io, N, rhs);
     }
   }
 }
@@ -73,18 +83,22 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
                                             const RkArgs<T> &rk, Lines &ln) {
   constexpr bool FIRST = DIR == 2, LAST = DIR == 0;
   const double *__restrict__ q = *q0p;
-  const long B = tp.base, PS = g.PS;
+  const FieldIO<DIR, T> io(tp, g);
   const T ih = T(inv_h), gam = T(gamma), gm1 = T(gamma - 1.0), ggm = T(gamma / (gamma - 1.0));
   T ud[PPT], irho[PPT], S[PPT], R5[PPT], f[PPT], x[PPT], r[PPT];
   {
     T gdp[PPT], qs5[PPT];
     {
       T rho[PPT], md[PPT];
-      ld<DIR>(q, B, PS, rho);
-      ld<DIR>(q + (1 + DIR) * N, B, PS, md);
-      ld<DIR>(q + 4 * N, B, PS, f);  // p
-      ld<DIR>(qs + 4 * N, B, PS, qs5);
+      io.ld(q, rho);
+      io.ld(q + (1 + DIR) * N, md);
+      io.ld(q + 4 * N, f);  // p
+      io.ld(qs + 4 * N, qs5);
       issue_loads();
+      io.got(rho);
+      io.got(md);
+      io.got(f);
+      io.got(qs5);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) {
         irho[m] = T(1) / rho[m];
@@ -96,6 +110,7 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
     ln.solve(op, f, x);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) S[m] = qs5[m] * irho[m] * (x[m] * ih);
+    pin(S);
     // E = D qs5
     ln.solve(op, qs5, x);
 #pragma unroll
@@ -105,6 +120,7 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
       R5[m] = gam * ud[m] * E;
       f[m] = -ud[m] * qs5[m];
     }
+    pin(R5);
   }
   // F = D(-u_d qs5)
   ln.solve(op, f, x);
@@ -117,10 +133,14 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
   T Ta[PPT];
   {
     asm volatile("" ::: "memory");
-    ld<DIR>(qs + (1 + DIR) * N, B, PS, f);
+    io.ld(qs + (1 + DIR) * N, f);
+    io.got(f);
     ln.solve(op, f, x);
     asm volatile("" ::: "memory");
-    if (!FIRST) ld<DIR>(rhs + 4 * N, B, PS, r);
+    if (!FIRST) {
+      io.ld(rhs + 4 * N, r);
+      io.got(r);
+    }
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       const T Bd = x[m] * ih;
@@ -129,13 +149,15 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
       R5[m] = R5[m] + gm1 * Bd;
       r[m] = FIRST ? -R5[m] : r[m] - R5[m];
     }
-    finish<DIR, T, LAST, RK>(4, r, B, PS, N, rhs, gobj, rk);
+    pin(Ta);
+    finish<LAST, RK>(4, r, io, N, rhs, gobj, rk);
   }
   // A = D qs1; A + u_d B_d waits in LDS (the thread's own slots) until the
   // end, which keeps the x sweep within 256 registers without spilling
   __shared__ T stash[PPT][NT];
   asm volatile("" ::: "memory");
-  ld<DIR>(qs, B, PS, f);
+  io.ld(qs, f);
+  io.got(f);
   ln.solve(op, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) stash[m][threadIdx.x] = Ta[m] + x[m] * ih;
@@ -145,31 +167,37 @@ __device__ __forceinline__ void asweep_body(const ThreadPos &tp, const Q *qs,
     if (i == DIR) continue;
     T um[PPT];
     asm volatile("" ::: "memory");
-    ld<DIR>(qs + (1 + i) * N, B, PS, f);
+    io.ld(qs + (1 + i) * N, f);
+    io.got(f);
     ln.solve(op, f, x);
     asm volatile("" ::: "memory");
-    ld<DIR>(q + (1 + i) * N, B, PS, um);
-    if (!FIRST) ld<DIR>(rhs + (1 + i) * N, B, PS, r);
+    io.ld(q + (1 + i) * N, um);
+    if (!FIRST) io.ld(rhs + (1 + i) * N, r);
+    io.got(um);
+    if (!FIRST) io.got(r);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       const T Bm = x[m] * ih;
       S[m] = S[m] + (um[m] * irho[m]) * Bm;
       r[m] = FIRST ? -(ud[m] * Bm) : r[m] - ud[m] * Bm;
     }
-    finish<DIR, T, LAST, RK>(1 + i, r, B, PS, N, rhs, gobj, rk);
+    finish<LAST, RK>(1 + i, r, io, N, rhs, gobj, rk);
   }
   // r1 += u_d S, r_{d+2} -= A + u_d B_d + S
 #pragma unroll
   for (int v = 0; v < 2; ++v) {
     const int var = v == 0 ? 0 : 1 + DIR;
     asm volatile("" ::: "memory");
-    if (!FIRST) ld<DIR>(rhs + var * N, B, PS, r);
+    if (!FIRST) {
+      io.ld(rhs + var * N, r);
+      io.got(r);
+    }
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       const T c = v == 0 ? ud[m] * S[m] : -(stash[m][threadIdx.x] + S[m]);
       r[m] = FIRST ? c : r[m] + c;
     }
-    finish<DIR, T, LAST, RK>(var, r, B, PS, N, rhs, gobj, rk);
+    finish<LAST, RK>(var, r, io, N, rhs, gobj, rk);
   }
 }
 

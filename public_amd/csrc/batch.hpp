@@ -75,11 +75,10 @@ __global__ __launch_bounds__(NT) void kb_sweep1(const BatchMember *__restrict__ 
   const ThreadPos tp = thread_pos_tile<DIR, true>(b.geom[DIR], blockIdx.x - L->start[e]);
   auto ln = make_lines<double, PER>(b.op[DIR], tp);
   const double *qs = stage_in(b, b.qn, stage);
-  if constexpr (DIR == 1)
-    sweep1_y_stress(tp, qs, b.rhs, b.G, b.op[1], b.geom[1], b.ph, b.N, ln);
+  if constexpr (DIR == 0)
+    sweep1_x_cart(tp, qs, b.rhs, b.G, b.op[0], b.geom[0], b.ph, b.N, ln);
   else
-    sweep1_body<double, double, DIR, RHS_CART>(tp, qs, b.rhs, b.G, b.op[DIR], b.geom[DIR], b.ph, b.N, Metric<double>{},
-                                               Penal<double>{}, ln);
+    sweep1_y_stress(tp, qs, b.rhs, b.G, b.op[1], b.geom[1], b.ph, b.N, ln);
 }
 
 // viscous sweep; the x sweep finishes RK stage `stage` (FF: the last stage

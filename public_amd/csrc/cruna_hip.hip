@@ -352,7 +352,7 @@ int check_launch() {
 #define DISPATCH_DIR(c, d, KER, TARGS, ...)                                                 \
   do {                                                                                      \
     const dim3 grid_((c)->geom[d].ntiles), block_((c)->wg[d]);                              \
-    const size_t lds_ = line_lds_bytes<TARGS>((c)->wg[d]);                                  \
+    const size_t lds_ = sweep_lds_bytes<TARGS>(d, (c)->wg[d]);                                  \
     const bool per_ = (c)->cfg.scheme[d] == CRUNA_HIP_PERIODIC;                            \
     if (d == 0) {                                                                           \
       if (per_) hipLaunchKernelGGL((KER<TARGS, 0, true>), grid_, block_, lds_, (c)->stream, __VA_ARGS__); \
@@ -590,7 +590,7 @@ bool adjoint_yform(const cruna_hip_ctx *c) {
 template <typename T, typename Q, int DIR, int FORM>
 void launch_sweep1_form(cruna_hip_ctx *c, const Q *in) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
-  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
+  const size_t lds = sweep_lds_bytes<T>(DIR, c->wg[DIR]);
   T *rhs = (T *)c->rhs, *G = (T *)c->G;
   const Op<T> &op = dops<T>(c)[DIR].op;
   if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC)
@@ -604,7 +604,7 @@ void launch_sweep1_form(cruna_hip_ctx *c, const Q *in) {
 template <typename T, typename Q, int DIR>
 void launch_curv_sweep1(cruna_hip_ctx *c, const Q *in) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
-  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
+  const size_t lds = sweep_lds_bytes<T>(DIR, c->wg[DIR]);
   T *rhs = (T *)c->rhs, *G = (T *)c->G, *TG = (T *)c->tg;
   const Op<T> &op = dops<T>(c)[DIR].op;
   const bool per = c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC;
@@ -669,7 +669,7 @@ int launch_sweep1(cruna_hip_ctx *c, const Q *in) {
 template <typename T, int DIR, int FORM, int RK, bool FF>
 void launch_sweep2_k(cruna_hip_ctx *c, int mode) {
   const dim3 grid(c->sgeom[DIR].ntiles), block(c->swg[DIR]);
-  const size_t lds = line_lds_bytes<T>(c->swg[DIR]);
+  const size_t lds = sweep_lds_bytes<T>(DIR, c->swg[DIR]);
   T *rhs = (T *)c->rhs;
   const T *G = (const T *)c->G;
   const Op<T> &op = dops<T>(c)[DIR].op, &fop = fops<T>(c)[DIR].op;
@@ -716,7 +716,7 @@ void launch_sweep2_form(cruna_hip_ctx *c, int mode, bool fuse_filter) {
 template <typename T, int DIR, bool PER, bool FF, bool Y>
 void launch_curv_sweep2_k(cruna_hip_ctx *c, int mode) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
-  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
+  const size_t lds = sweep_lds_bytes<T>(DIR, c->wg[DIR]);
   const T *force = (const T *)(DIR == 0 && c->cnn ? c->force : nullptr);
   const int form = DIR == 0 ? rk_form(mode, direct_yform(c)) : RK_RHS;
   const RkArgs<T> rk = rk_args<T>(c, c->qn, c->cfg.dt, mode, direct_yform(c));
@@ -839,14 +839,16 @@ void launch_filter(cruna_hip_ctx *c, const S *src, double *q64, int nv, T *copy)
   if constexpr (sizeof(T) == 8) {
     if (!c->fop64[DIR].rec) {
       const LineOp<double> &op = c->fcr64[DIR].op;
+      // the field exchange lies behind the (here unused) recursion cells
+      const size_t cr_lds = sweep_lds_bytes<double>(DIR, c->fwg[DIR]);
       if (per)
-        hipLaunchKernelGGL((k_filter_cr<DIR, true>), grid, block, 0, c->stream, src, q64, op, c->fgeom[DIR], c->N, nv);
+        hipLaunchKernelGGL((k_filter_cr<DIR, true>), grid, block, cr_lds, c->stream, src, q64, op, c->fgeom[DIR], c->N, nv);
       else
-        hipLaunchKernelGGL((k_filter_cr<DIR, false>), grid, block, 0, c->stream, src, q64, op, c->fgeom[DIR], c->N, nv);
+        hipLaunchKernelGGL((k_filter_cr<DIR, false>), grid, block, cr_lds, c->stream, src, q64, op, c->fgeom[DIR], c->N, nv);
       return;
     }
   }
-  const size_t lds = line_lds_bytes<T>(c->fwg[DIR]);
+  const size_t lds = sweep_lds_bytes<T>(DIR, c->fwg[DIR]);
   const Op<T> &op = fops<T>(c)[DIR].op;
   if (per)
     hipLaunchKernelGGL((k_filter<T, DIR, true, S>), grid, block, lds, c->stream, src, q64, op, c->fgeom[DIR],
@@ -1113,7 +1115,7 @@ int bc_qs(cruna_hip_ctx *c, Q *qs, bool outside = false) {
 template <typename T, typename Q, int DIR, int RK>
 void launch_asweep_k(cruna_hip_ctx *c, const Q *in, const double *g, int mode) {
   const dim3 grid(c->geom[DIR].ntiles), block(c->wg[DIR]);
-  const size_t lds = line_lds_bytes<T>(c->wg[DIR]);
+  const size_t lds = sweep_lds_bytes<T>(DIR, c->wg[DIR]);
   // backward in time (rk_o4_e.f90:62-105)
   const RkArgs<T> rk = rk_args<T>(c, c->qa, -c->cfg.dt, mode, adjoint_yform(c));
   if (c->cfg.scheme[DIR] == CRUNA_HIP_PERIODIC)
@@ -1470,8 +1472,10 @@ int cruna_hip_create(const cruna_hip_cfg *cfg, cruna_hip_ctx **out) {
       if (int rc = c->fop64[d].upload(build_rec_op(OP_FILTER, per, cfg->n[d], cfg->filter_alpha))) return rc;
       if (!c->fop64[d].rec)
         if (int rc = c->fcr64[d].upload(ff)) return rc;
-      if (int rc = c->dop32[d].upload(dd)) return rc;
-      if (int rc = c->fop32[d].upload(ff)) return rc;
+      if (cfg->precision == CRUNA_HIP_FP32_MIXED) {
+        if (int rc = c->dop32[d].upload(dd)) return rc;
+        if (int rc = c->fop32[d].upload(ff)) return rc;
+      }
     } catch (const std::exception &e) {
       return fail(CRUNA_HIP_EINVAL, e.what());
     }
@@ -2469,9 +2473,12 @@ struct BatchSlot {
   } while (0)
 
 template <int DIR>
+size_t batch_lds(int threads) { return sweep_lds_bytes<double>(DIR, threads); }
+
+template <int DIR>
 void batch_sweep1(const BatchSlot &S, int stage) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep1<DIR, true>), stage);
-  else BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep1<DIR, false>), stage);
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, batch_lds<DIR>, (kb_sweep1<DIR, true>), stage);
+  else BATCH_LAUNCH(S, 0, 0, DIR, batch_lds<DIR>, (kb_sweep1<DIR, false>), stage);
 }
 
 void batch_sweep12z(const BatchSlot &S, int stage) {
@@ -2481,20 +2488,20 @@ void batch_sweep12z(const BatchSlot &S, int stage) {
 
 template <int DIR, int RK, bool FF>
 void batch_sweep2(const BatchSlot &S, int stage) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep2<DIR, true, RK, FF>), stage);
-  else BATCH_LAUNCH(S, 0, 0, DIR, rec_lds_bytes, (kb_sweep2<DIR, false, RK, FF>), stage);
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 0, 0, DIR, batch_lds<DIR>, (kb_sweep2<DIR, true, RK, FF>), stage);
+  else BATCH_LAUNCH(S, 0, 0, DIR, batch_lds<DIR>, (kb_sweep2<DIR, false, RK, FF>), stage);
 }
 
 template <int DIR>
 void batch_filter(const BatchSlot &S, int grp) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, grp, 1, DIR, rec_lds_bytes, (kb_filter<DIR, true>), grp);
-  else BATCH_LAUNCH(S, grp, 1, DIR, rec_lds_bytes, (kb_filter<DIR, false>), grp);
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, grp, 1, DIR, batch_lds<DIR>, (kb_filter<DIR, true>), grp);
+  else BATCH_LAUNCH(S, grp, 1, DIR, batch_lds<DIR>, (kb_filter<DIR, false>), grp);
 }
 
 template <int DIR, int RK>
 void batch_asweep(const BatchSlot &S, int stage) {
-  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 1, 0, DIR, rec_lds_bytes, (kb_asweep<DIR, true, RK>), stage);
-  else BATCH_LAUNCH(S, 1, 0, DIR, rec_lds_bytes, (kb_asweep<DIR, false, RK>), stage);
+  if (S.e->bper[DIR]) BATCH_LAUNCH(S, 1, 0, DIR, batch_lds<DIR>, (kb_asweep<DIR, true, RK>), stage);
+  else BATCH_LAUNCH(S, 1, 0, DIR, batch_lds<DIR>, (kb_asweep<DIR, false, RK>), stage);
 }
 
 // One forward step of the bin's group 0 (step_once of each member: RK4 with

@@ -42,7 +42,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
   constexpr bool FIRST = DIR == 0;
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER>(op, tp);
-  const long B = tp.base, PS = g.PS;
+  const FieldIO<DIR, T> io(tp, g);
   const T ih = T(ph.inv_h[DIR]);
   // In FP64, rho, and in the periodic x sweep the momenta, stay in
   // registers from their first read to the convective fluxes: those sweeps
@@ -52,21 +52,26 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
   constexpr bool KEEPR = sizeof(T) == 8, KEEPM = KEEPR && DIR == 0 && PER;
   T M0[PPT], M1[PPT], M2[PPT], rho[PPT], irho[PPT], uh[PPT], x[PPT], f[PPT];
   T mk[KEEPM ? 3 : 1][PPT];
-  ld<DIR>(mt.M + (DIR + 0) * N, B, PS, M0);
-  ld<DIR>(mt.M + (DIR + 3) * N, B, PS, M1);
-  ld<DIR>(mt.M + (DIR + 6) * N, B, PS, M2);
-  ld<DIR>(qs, B, PS, rho);
+  io.ld(mt.M + (DIR + 0) * N, M0);
+  io.ld(mt.M + (DIR + 3) * N, M1);
+  io.ld(mt.M + (DIR + 6) * N, M2);
+  io.ld(qs, rho);
+  io.got(M0);
+  io.got(M1);
+  io.got(M2);
+  io.got(rho);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) irho[m] = T(1) / rho[m];
   // accumulate a value into field slot `fld` (the first sweep writes it)
   auto acc = [&](T *fld, T(&v)[PPT]) {
     if (!FIRST) {
       T o[PPT];
-      ld<DIR>(fld, B, PS, o);
+      io.ld(fld, o);
+      io.got(o);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) v[m] = o[m] + v[m];
     }
-    st<DIR>(fld, B, PS, v);
+    io.st(fld, v);
   };
 
   // physical velocity gradients (:114-135) and the contravariant velocity
@@ -75,7 +80,8 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     T ui[PPT];
-    ld<DIR>(qs + (1 + i) * N, B, PS, ui);
+    io.ld(qs + (1 + i) * N, ui);
+    io.got(ui);
     if constexpr (KEEPM) {
 #pragma unroll
       for (int m = 0; m < PPT; ++m) mk[i][m] = ui[m];
@@ -123,14 +129,15 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
   // temperature, its physical gradient (:168-175) and, in the first sweep,
   // the viscosity of the stage input
   T p[PPT];
-  ld<DIR>(qs + 4 * N, B, PS, p);
+  io.ld(qs + 4 * N, p);
+  io.got(p);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) f[m] = temperature(ph, irho[m], p[m]);
   if (FIRST) {
     T mu[PPT];
 #pragma unroll
     for (int m = 0; m < PPT; ++m) mu[m] = viscosity(ph, f[m]);
-    st<DIR>(G + 6 * N, B, PS, mu);
+    io.st(G + 6 * N, mu);
   }
   ln.solve(op, f, x);
 #pragma unroll
@@ -151,12 +158,15 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
   // convective fluxes with the contravariant velocity (:184-247)
   T PH[PPT], IP[PPT];
   if (EV) {
-    ld<DIR>(pe.phi, B, PS, PH);
-    ld<DIR>(pe.inv_phi, B, PS, IP);
+    io.ld(pe.phi, PH);
+    io.ld(pe.inv_phi, IP);
+    io.got(PH);
+    io.got(IP);
   }
   auto div = [&](int m, T v) -> T { return EV ? IP[m] * v : v; };
   {  // mass
-    if constexpr (!KEEPR) ld<DIR>(qs, B, PS, rho);
+    if constexpr (!KEEPR) io.ld(qs, rho);
+    if constexpr (!KEEPR) io.got(rho);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * rho[m]) * uh[m] : rho[m] * uh[m];
     ln.solve(op, f, x);
@@ -171,7 +181,8 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
 #pragma unroll
       for (int m = 0; m < PPT; ++m) mom[m] = mk[i][m];
     } else {
-      ld<DIR>(qs + (1 + i) * N, B, PS, mom);
+      io.ld(qs + (1 + i) * N, mom);
+      io.got(mom);
     }
 #pragma unroll
     for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * mom[m]) * uh[m] : mom[m] * uh[m];
@@ -201,13 +212,17 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
   constexpr bool LAST = DIR == 0;
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER>(op, tp);
-  const long B = tp.base, PS = g.PS;
+  const StridedIO<DIR> io(tp, g);  // (the exchange through LDS would spill)
   const T ih = T(ph.inv_h[DIR]);
   T M0[PPT], M1[PPT], M2[PPT], mu[PPT];
-  ld<DIR>(mt.M + (DIR + 0) * N, B, PS, M0);
-  ld<DIR>(mt.M + (DIR + 3) * N, B, PS, M1);
-  ld<DIR>(mt.M + (DIR + 6) * N, B, PS, M2);
-  ld<DIR>(G + 6 * N, B, PS, mu);
+  io.ld(mt.M + (DIR + 0) * N, M0);
+  io.ld(mt.M + (DIR + 3) * N, M1);
+  io.ld(mt.M + (DIR + 6) * N, M2);
+  io.ld(G + 6 * N, mu);
+  io.got(M0);
+  io.got(M1);
+  io.got(M2);
+  io.got(mu);
   // heat flux along DIR first (the metric row and mu are live for it and the
   // stresses only): sum_j M(DIR,j) D_DIR(lambda J T_j), no h (:252-268).
   // J, phi and 1/phi are read where they are used (again later in the
@@ -216,10 +231,12 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
   T hs[PPT];
   {
     T lj[PPT];  // (phi) lambda J
-    ld<DIR>(mt.J, B, PS, lj);
+    io.ld(mt.J, lj);
+    io.got(lj);
     if (EV) {
       T PH[PPT];
-      ld<DIR>(pe.phi, B, PS, PH);
+      io.ld(pe.phi, PH);
+      io.got(PH);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) lj[m] = (PH[m] * lambda_of(ph, mu[m])) * lj[m];
     } else {
@@ -229,7 +246,8 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       T f[PPT], x[PPT];
-      ld<DIR>(TG + j * N, B, PS, f);
+      io.ld(TG + j * N, f);
+      io.got(f);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) f[m] = lj[m] * f[m];
       ln.solve(op, f, x);
@@ -242,16 +260,18 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
   }
   if (EV) {
     T IP[PPT];
-    ld<DIR>(pe.inv_phi, B, PS, IP);
+    io.ld(pe.inv_phi, IP);
+    io.got(IP);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) hs[m] = IP[m] * hs[m];
   }
   if (!LAST) {
     T k[PPT];
-    ld<DIR>(rhs + 4 * N, B, PS, k);
+    io.ld(rhs + 4 * N, k);
+    io.got(k);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) k[m] = k[m] + hs[m];
-    st<DIR>(rhs + 4 * N, B, PS, k);
+    io.st(rhs + 4 * N, k);
   }
   // projected stresses tau_proj_{i,DIR} = sum_j M(DIR,j) tau_ij (:195-238)
   // (the diagonal first, then one symmetric pair at a time, so that only
@@ -259,9 +279,12 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
   T t1[PPT], t2[PPT], t3[PPT], diss[PPT];
   {
     T ux[PPT], vy[PPT], wz[PPT];
-    ld<DIR>(G + 0 * N, B, PS, ux);
-    ld<DIR>(G + 1 * N, B, PS, vy);
-    ld<DIR>(G + 2 * N, B, PS, wz);
+    io.ld(G + 0 * N, ux);
+    io.ld(G + 1 * N, vy);
+    io.ld(G + 2 * N, wz);
+    io.got(ux);
+    io.got(vy);
+    io.got(wz);
     issue_loads();
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
@@ -277,7 +300,8 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
 #pragma unroll
   for (int s = 0; s < 3; ++s) {  // s12 = u_y + v_x, s13 = u_z + w_x, s23 = v_z + w_y
     T sv[PPT];
-    ld<DIR>(G + (3 + s) * N, B, PS, sv);
+    io.ld(G + (3 + s) * N, sv);
+    io.got(sv);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       const T t = mu[m] * sv[m];
@@ -297,27 +321,29 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
   auto finish = [&](int v, T(&k)[PPT]) {
     if (LAST && force) {
       T fv[PPT];
-      ld<DIR>(force + v * N, B, PS, fv);
+      io.ld(force + v * N, fv);
+      io.got(fv);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) k[m] = k[m] + fv[m];
     }
     if constexpr (FF) {
       double a[PPT];
-      rk_final<DIR, T, Y>(rk, v, k, B, PS, N, a);
+      rk_final<Y>(rk, v, k, io, N, a);
       T f[PPT], x[PPT];
 #pragma unroll
       for (int m = 0; m < PPT; ++m) f[m] = T(a[m]);
       ln.bind(fop);
       ln.template solve<true>(fop, f, x);
       ln.bind(op);
-      st<DIR>(rk.qn + v * N, B, PS, x);
+      io.st(rk.qn + v * N, x);
     } else {
-      rk_update<DIR, T, Y>(form, rk, v, k, B, PS, N, rhs);
+      rk_update<Y>(form, rk, v, k, io, N, rhs);
     }
   };
   if (EV) {  // phi tau_proj inside the derivative
     T PH[PPT];
-    ld<DIR>(pe.phi, B, PS, PH);
+    io.ld(pe.phi, PH);
+    io.got(PH);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       t1[m] = PH[m] * t1[m];
@@ -326,10 +352,12 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
     }
   }
   T Jv[PPT];
-  if (LAST) ld<DIR>(mt.J, B, PS, Jv);
+  if (LAST) io.ld(mt.J, Jv);
+  if (LAST) io.got(Jv);
   if (LAST) {  // pressure: J (gamma - 1) (bracket + heat + J tau:grad(u)) (:270-276)
     T k[PPT];
-    ld<DIR>(rhs + 4 * N, B, PS, k);
+    io.ld(rhs + 4 * N, k);
+    io.got(k);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       k[m] = k[m] + hs[m];
@@ -339,7 +367,8 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
   }
   if (LAST) {  // mass (:189-190)
     T k[PPT];
-    ld<DIR>(rhs, B, PS, k);
+    io.ld(rhs, k);
+    io.got(k);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) k[m] = Jv[m] * k[m];
     finish(0, k);
@@ -350,10 +379,12 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
     ln.solve(op, i == 0 ? t1 : (i == 1 ? t2 : t3), x);
     asm volatile("" ::: "memory");
     T k[PPT];
-    ld<DIR>(rhs + (1 + i) * N, B, PS, k);
+    io.ld(rhs + (1 + i) * N, k);
+    io.got(k);
     if (EV) {
       T IP[PPT];
-      ld<DIR>(pe.inv_phi, B, PS, IP);
+      io.ld(pe.inv_phi, IP);
+      io.got(IP);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) x[m] = IP[m] * x[m];
     }
@@ -365,7 +396,7 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
     if (LAST)
       finish(1 + i, k);
     else
-      st<DIR>(rhs + (1 + i) * N, B, PS, k);
+      io.st(rhs + (1 + i) * N, k);
   }
 }
 

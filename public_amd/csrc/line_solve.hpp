@@ -332,7 +332,10 @@ __device__ __forceinline__ void line_solve(const LineOp<T> &op, LineLds<T, NTM> 
 // immediate offset away.  Dynamic LDS, so that a work-group takes what its own
 // size needs.
 constexpr int REC_STRIDE = 13, REC_HALO = 8, REC_UL = 8, REC_XF = 10;
-inline size_t rec_lds_bytes(int threads) { return (size_t)(threads + 1) * REC_STRIDE * sizeof(double); }
+// (a multiple of 16: what follows is accessed in 16-byte pieces)
+__host__ __device__ inline size_t rec_lds_bytes(int threads) {
+  return ((size_t)(threads + 1) * REC_STRIDE * sizeof(double) + 15) / 16 * 16;
+}
 
 template <typename T>
 struct OpOf {

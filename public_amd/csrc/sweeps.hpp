@@ -209,6 +209,116 @@ __device__ __forceinline__ void st(Q *__restrict__ p, long base, long PS, const 
   }
 }
 
+// Field access of a sweep along DIR.  ld issues the loads of the thread's block,
+// got (after all loads of a group are issued) makes the values the thread's
+// own; st stores.  Along y and z got does nothing.  Along x a thread's block is
+// 64 contiguous bytes (FP64), so thread-by-thread 16-byte accesses lie 64 bytes
+// apart and each instruction touches every cache line of the wavefront's 4 KB,
+// which makes the vector cache's request rate the limit.  In FP64 lane l moves
+// chunk l of each contiguous 1 KB instead, and the blocks are exchanged through
+// LDS within the wavefront (a lane's slot is 80 bytes, so that 8 lanes' 16-byte
+// pieces fall on different banks).  Measured at 256^3: the x first-derivative
+// sweep 456 -> 356 us (14 words per point: 4.1 -> 5.3 TB/s), at 128^3 59 -> 44 us,
+// the x filter 38 -> 30 us.  FP32 (32-byte blocks) gained nothing and keeps the
+// thread-by-thread form.
+template <int DIR>
+struct StridedIO {
+  long B, PS;
+  __device__ __forceinline__ StridedIO(const ThreadPos &tp, const SweepGeom &g) : B(tp.base), PS(g.PS) {}
+  template <typename Q, typename V>
+  __device__ __forceinline__ void ld(const Q *__restrict__ p, V (&v)[PPT]) const {
+    cruna::ld<DIR>(p, B, PS, v);
+  }
+  template <typename V>
+  __device__ __forceinline__ void got(V (&)[PPT]) const {}
+  template <typename Q, typename V>
+  __device__ __forceinline__ void st(Q *__restrict__ p, const V (&v)[PPT]) const {
+    cruna::st<DIR>(p, B, PS, v);
+  }
+};
+template <int DIR, typename T>
+struct FieldIO : StridedIO<DIR> {
+  using StridedIO<DIR>::StridedIO;
+};
+
+constexpr int X_STAGE = 80;  // bytes of LDS per thread of an FP64 x sweep
+// dynamic LDS of a sweep along dir in a work-group of `threads`
+template <typename T>
+size_t sweep_lds_bytes(int dir, int threads) {
+  return line_lds_bytes<T>(threads) + (dir == 0 && sizeof(T) == 8 ? (size_t)((threads + 63) / 64 * 64) * X_STAGE : 0);
+}
+
+template <>
+struct FieldIO<0, double> {
+  static constexpr int NCH = PPT / 2;  // 16-byte chunks of a block
+  char *own, *raw;     // LDS: the lane's slot; the place of the chunks it moves
+  unsigned off;        // byte offset of its first chunk in a field
+  unsigned gstep, lstep;  // distance of its chunks in the field, in LDS
+  __device__ __forceinline__ FieldIO(const ThreadPos &tp, const SweepGeom &) {
+    const unsigned lane = threadIdx.x & 63;
+    char *stage = line_dyn + rec_lds_bytes(blockDim.x) + (threadIdx.x >> 6) * (64 * X_STAGE);
+    const bool idle = tp.base == IDLE_BASE;
+    // lanes with a block: the first ones of the wavefront, their blocks one
+    // after the other in memory
+    const unsigned active = __popcll(__builtin_amdgcn_ballot_w64(!idle));
+    const unsigned first = __builtin_amdgcn_readfirstlane(unsigned(tp.base)) * 8u;
+    own = stage + lane * X_STAGE;
+    if (active % NCH == 0 && active != 0) {
+      // chunk k * active + lane of the wavefront, k = 0..3
+      raw = idle ? own : stage + (lane / NCH) * X_STAGE + (lane % NCH) * 16;
+      off = idle ? FIELD_EXTENT : first + lane * 16;
+      gstep = active * 16;
+      lstep = active / NCH * X_STAGE;
+    } else {  // the lane's own block
+      raw = own;
+      off = idle ? FIELD_EXTENT : first + lane * 64;
+      gstep = 16;
+      lstep = 16;
+    }
+  }
+  __device__ __forceinline__ static void order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+  }
+  __device__ __forceinline__ void ld(const double *__restrict__ p, double (&v)[PPT]) const {
+    const __amdgpu_buffer_rsrc_t r = rsrc(p);
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+      const bu4 t = __builtin_amdgcn_raw_buffer_load_b128(r, off, k * gstep, 0);
+      v[2 * k] = __builtin_bit_cast(double, bu2{t[0], t[1]});
+      v[2 * k + 1] = __builtin_bit_cast(double, bu2{t[2], t[3]});
+    }
+  }
+  // (an idle lane's chunk k >= 1 would fall outside its slot: it writes nothing)
+  __device__ __forceinline__ void got(double (&v)[PPT]) const {
+#pragma unroll
+    for (int k = 0; k < NCH; ++k)
+      if (off != FIELD_EXTENT) *reinterpret_cast<double2 *>(raw + k * lstep) = double2{v[2 * k], v[2 * k + 1]};
+    order();
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      const double2 c = *reinterpret_cast<const double2 *>(own + j * 16);
+      v[2 * j] = c.x;
+      v[2 * j + 1] = c.y;
+    }
+    order();
+  }
+  __device__ __forceinline__ void st(double *__restrict__ p, const double (&v)[PPT]) const {
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) *reinterpret_cast<double2 *>(own + j * 16) = double2{v[2 * j], v[2 * j + 1]};
+    order();
+    const __amdgpu_buffer_rsrc_t r = rsrc(p);
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+      // (an idle lane's store is dropped; it reads its own slot)
+      const bu4 t = *reinterpret_cast<const bu4 *>(off != FIELD_EXTENT ? raw + k * lstep : own + k * 16);
+      __builtin_amdgcn_raw_buffer_store_b128(t, r, off, k * gstep, 0);
+    }
+    order();
+  }
+};
+
 // Work-group size limit of the Cartesian viscous sweeps: FP32 tiles take up
 // to 32 y/z lines so that rows of floats are 128 bytes, as FP64 rows of 16.
 template <typename T>
@@ -254,7 +364,7 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
                                             Lines &ln, ZCarry<T> *zc = nullptr) {
   constexpr bool GT = FORM == RHS_GT, EV = FORM == RHS_EV;
   static_assert(!FUSE || (DIR == 2 && FORM == RHS_CART), "the fused z sweep is Cartesian");
-  const long B = tp.base, PS = g.PS;
+  const FieldIO<DIR, T> io(tp, g);
   const T mline = GT ? mt.m[DIR][tp.lidx] : T(1);
   const T ih = GT ? T(ph.inv_h[DIR]) * mline : T(ph.inv_h[DIR]);
   // heat flux: inner (temperature) and outer derivative scales
@@ -263,8 +373,10 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
   // penalisation: phi inside the fluxes, the stored 1/phi on their divergence
   T PH[PPT], IP[PPT];
   if (EV) {
-    ld<DIR>(pe.phi, B, PS, PH);
-    ld<DIR>(pe.inv_phi, B, PS, IP);
+    io.ld(pe.phi, PH);
+    io.ld(pe.inv_phi, IP);
+    io.got(PH);
+    io.got(IP);
   }
   auto div = [&](int m, T v) -> T { return EV ? IP[m] * v : v; };
   // G slot of d(u_i)/dx_DIR and whether it completes a symmetric sum begun by
@@ -276,8 +388,11 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
   };
   auto gsum = [](int i) -> bool { return (DIR == 1 && i == 0) || (DIR == 2 && i < 2); };
   T irho[PPT], mom[PPT], p[PPT], f[PPT], x[PPT], y[PPT], r[PPT];
-  ld<DIR>(qs, B, PS, f);
-  ld<DIR>(qs + (1 + DIR) * N, B, PS, mom);
+  io.ld(qs, f);
+  io.ld(qs + (1 + DIR) * N, mom);
+  if (DIR == 0) issue_loads();
+  io.got(f);
+  io.got(mom);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) irho[m] = T(1) / f[m];
 
@@ -288,23 +403,27 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
     const int i = k == 0 ? (DIR == 0 ? 1 : 0) : (DIR == 2 ? 1 : 2);
     T ui[PPT], gs[PPT];
     asm volatile("" ::: "memory");
-    ld<DIR>(qs + (1 + i) * N, B, PS, ui);
-    if (gsum(i)) ld<DIR>(G + gslot(i) * N, B, PS, gs);
+    io.ld(qs + (1 + i) * N, ui);
+    if (gsum(i)) io.ld(G + gslot(i) * N, gs);
     issue_loads();
+    io.got(ui);
+    if (gsum(i)) io.got(gs);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       ui[m] = ui[m] * irho[m];
       f[m] = EV ? (PH[m] * mom[m]) * ui[m] : mom[m] * ui[m];
     }
-    if (DIR != 0) ld<DIR>(rhs + (1 + i) * N, B, PS, r);
-    if (k == 1) ld<DIR>(qs + 4 * N, B, PS, p);  // in flight for the pressure terms
+    if (DIR != 0) io.ld(rhs + (1 + i) * N, r);
+    if (k == 1) io.ld(qs + 4 * N, p);  // in flight for the pressure terms
     ln.solve2(op, ui, y, f, x);
+    if (DIR != 0) io.got(r);
+    if (k == 1) io.got(p);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       y[m] = y[m] * ih;
       if (gsum(i)) y[m] = y[m] + gs[m];
     }
-    st<DIR>(G + gslot(i) * N, B, PS, y);
+    io.st(G + gslot(i) * N, y);
     if constexpr (FUSE) {
 #pragma unroll
       for (int m = 0; m < PPT; ++m) (k == 0 ? zc->s13 : zc->s23)[m] = y[m];
@@ -315,7 +434,7 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
 #pragma unroll
       for (int m = 0; m < PPT; ++m) zc->mom(i, m) = r[m];
     } else {
-      st<DIR>(rhs + (1 + i) * N, B, PS, r);
+      io.st(rhs + (1 + i) * N, r);
     }
   }
 
@@ -326,25 +445,27 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
     ud[m] = mom[m] * irho[m];
     f[m] = EV ? PH[m] * mom[m] : mom[m];
   }
-  if (DIR != 0) ld<DIR>(rhs, B, PS, r);
+  if (DIR != 0) io.ld(rhs, r);
   ln.solve2(op, ud, y, f, x);
+  if (DIR != 0) io.got(r);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) y[m] = y[m] * ih;
-  st<DIR>(G + DIR * N, B, PS, y);
+  io.st(G + DIR * N, y);
   if constexpr (FUSE) {
 #pragma unroll
     for (int m = 0; m < PPT; ++m) zc->wz[m] = y[m];
   }
 #pragma unroll
   for (int m = 0; m < PPT; ++m) r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
-  st<DIR>(rhs, B, PS, r);
+  io.st(rhs, r);
 
   // pressure gradient p_DIR, and momentum DIR: -d/dx_DIR (rho u_DIR u_DIR) - p_DIR
   T pd[PPT];
-  if (DIR != 0) ld<DIR>(rhs + (1 + DIR) * N, B, PS, r);
+  if (DIR != 0) io.ld(rhs + (1 + DIR) * N, r);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * mom[m]) * ud[m] : mom[m] * ud[m];
   ln.solve2(op, p, pd, f, x);
+  if (DIR != 0) io.got(r);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) {
     pd[m] = pd[m] * ih;
@@ -355,7 +476,7 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
 #pragma unroll
     for (int m = 0; m < PPT; ++m) zc->mom(DIR, m) = r[m];
   } else {
-    st<DIR>(rhs + (1 + DIR) * N, B, PS, r);
+    io.st(rhs + (1 + DIR) * N, r);
   }
 
   // pressure-equation bracket: gamma/(gamma-1) (-d(p u_DIR)) + u_DIR p_DIR
@@ -364,10 +485,15 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
   // mu in G6 for the later sweeps of the stage
   T e[PPT], tk[PPT], mu[PPT], Jv[PPT];
   if (DIR != 0) {
-    ld<DIR>(rhs + 4 * N, B, PS, r);
-    ld<DIR>(G + 6 * N, B, PS, mu);
+    io.ld(rhs + 4 * N, r);
+    io.ld(G + 6 * N, mu);
   }
-  if (GT) ld<DIR>(mt.J, B, PS, Jv);
+  if (GT) io.ld(mt.J, Jv);
+  if (DIR != 0) {
+    io.got(r);
+    io.got(mu);
+  }
+  if (GT) io.got(Jv);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) {
     f[m] = EV ? (PH[m] * p[m]) * ud[m] : p[m] * ud[m];
@@ -376,7 +502,7 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
   if (DIR == 0) {
 #pragma unroll
     for (int m = 0; m < PPT; ++m) mu[m] = viscosity(ph, tk[m]);
-    st<DIR>(G + 6 * N, B, PS, mu);
+    io.st(G + 6 * N, mu);
   }
   if constexpr (FUSE) {
 #pragma unroll
@@ -396,17 +522,104 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
     e[m] = e[m] + div(m, x[m] * hout);
     if (DIR != 0) e[m] = r[m] + e[m];
   }
-  st<DIR>(rhs + 4 * N, B, PS, e);
+  io.st(rhs + 4 * N, e);
 }
 
 template <typename T, int FORM>
 constexpr bool stress_form() { return sizeof(T) == 8 && FORM == RHS_CART; }
+
+// These FP64 sweeps write every fused multiply-add out and contract nothing, so
+// that the batched kernels, compiled apart, give the same bits.
+
+// S1 x in FP64 (Cartesian form): two independent solves per exchange, the
+// transverse momenta in flight while the solves before them run.
+template <typename Lines>
+__device__ __forceinline__ void sweep1_x_cart(const ThreadPos &tp, const double *__restrict__ qs,
+                                              double *__restrict__ rhs, double *__restrict__ G, const RecOp &op,
+                                              const SweepGeom &g, const Phys &ph, long N, Lines &ln) {
+#pragma clang fp contract(off)
+  const FieldIO<0, double> io(tp, g);
+  const double ih = ph.inv_h[0], hh = ph.heat_inv_h[0];
+  double irho[PPT], mom[PPT], u[PPT], p[PPT], lt[PPT], f[PPT], x[PPT], y[PPT];
+  io.ld(qs, irho);
+  io.ld(qs + N, mom);
+  io.ld(qs + 4 * N, p);
+  issue_loads();
+  io.got(irho);
+  io.got(mom);
+  io.got(p);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    irho[m] = 1.0 / irho[m];
+    f[m] = temperature(ph, irho[m], p[m]);
+  }
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) lt[m] = viscosity(ph, f[m]);
+  io.st(G + 6 * N, lt);
+  // p_x and the inner derivative of the heat flux
+  double pd[PPT];
+  ln.solve2(op, p, pd, f, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    u[m] = mom[m] * irho[m];
+    lt[m] = lambda_of(ph, lt[m]) * (y[m] * hh);
+    pd[m] = pd[m] * ih;
+    f[m] = mom[m] * u[m];
+    p[m] = p[m] * u[m];
+  }
+  // rho u, and the pressure bracket's flux with u p_x
+  ln.solve2(op, f, x, p, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    x[m] = __builtin_fma(-x[m], ih, -pd[m]);
+    p[m] = __builtin_fma(-ph.gt, y[m] * ih, u[m] * pd[m]);
+  }
+  io.st(rhs + N, x);
+  asm volatile("" ::: "memory");
+  // the heat flux completes the bracket; u_x
+  double v[PPT];
+  io.ld(qs + 2 * N, v);
+  ln.solve2(op, lt, x, u, y);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) {
+    p[m] = __builtin_fma(x[m], hh, p[m]);
+    y[m] = y[m] * ih;
+  }
+  io.st(rhs + 4 * N, p);
+  io.st(G, y);
+  // v_x, w_x and the fluxes rho u v, rho u w
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    io.got(v);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      u[m] = v[m] * irho[m];
+      f[m] = mom[m] * u[m];
+    }
+    asm volatile("" ::: "memory");
+    if (i == 0) io.ld(qs + 3 * N, v);
+    ln.solve2(op, u, x, f, y);
+#pragma unroll
+    for (int m = 0; m < PPT; ++m) {
+      x[m] = x[m] * ih;
+      y[m] = -(y[m] * ih);
+    }
+    io.st(G + (3 + i) * N, x);
+    io.st(rhs + (2 + i) * N, y);
+  }
+  // mass
+  ln.solve(op, mom, x);
+#pragma unroll
+  for (int m = 0; m < PPT; ++m) x[m] = -(x[m] * ih);
+  io.st(rhs, x);
+}
 
 // S2 y in the stress form: the first-derivative sweep along y with tau_12.
 template <typename Lines>
 __device__ __forceinline__ void sweep1_y_stress(const ThreadPos &tp, const double *__restrict__ qs,
                                                 double *__restrict__ rhs, double *__restrict__ G, const RecOp &op,
                                                 const SweepGeom &g, const Phys &ph, long N, Lines &ln) {
+#pragma clang fp contract(off)
   const long B = tp.base, PS = g.PS;
   const double ih = ph.inv_h[1], hh = ph.heat_inv_h[1];
   double irho[PPT], mom[PPT], p[PPT], mu[PPT], f[PPT], u[PPT], x[PPT], y[PPT], r[PPT], e[PPT], lt[PPT];
@@ -440,7 +653,7 @@ __device__ __forceinline__ void sweep1_y_stress(const ThreadPos &tp, const doubl
   // rho u: -d(rho v u)/dy + d(tau_12)/dy
   ln.solve2(op, x, u, f, y);
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) r[m] = r[m] + (u[m] - y[m]) * ih;
+  for (int m = 0; m < PPT; ++m) r[m] = __builtin_fma(u[m] - y[m], ih, r[m]);
   st<1>(rhs + N, B, PS, r);
   asm volatile("" ::: "memory");
   // w_y and rho w
@@ -480,7 +693,7 @@ __device__ __forceinline__ void sweep1_y_stress(const ThreadPos &tp, const doubl
   ln.solve2(op, p, x, f, y);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) {
-    r[m] = r[m] - (x[m] + y[m]) * ih;
+    r[m] = __builtin_fma(-(x[m] + y[m]), ih, r[m]);
     e[m] = __builtin_fma(u[m], x[m] * ih, e[m]);  // u.grad(p)
     f[m] = p[m] * u[m];
   }
@@ -510,9 +723,10 @@ template <typename Lines>
 __device__ __forceinline__ void sweep12_z_stress(const ThreadPos &tp, const double *__restrict__ qs,
                                                  double *__restrict__ rhs, double *__restrict__ G, const RecOp &op,
                                                  const SweepGeom &g, const Phys &ph, long N, Lines &ln) {
+#pragma clang fp contract(off)
   const long B = tp.base, PS = g.PS;
   const double ih = ph.inv_h[2], hh = ph.heat_inv_h[2];
-  double *slot = reinterpret_cast<double *>(line_dyn) + (blockDim.x + 1) * REC_STRIDE + threadIdx.x * ZS_STRIDE;
+  double *slot = reinterpret_cast<double *>(line_dyn) + rec_lds_bytes(blockDim.x) / sizeof(double) + threadIdx.x * ZS_STRIDE;
   double mom[PPT], w[PPT], p[PPT], t1[PPT], t2[PPT], t3[PPT], e[PPT], lt[PPT];
   {
     double irho[PPT], f[PPT], u[PPT], x[PPT], y[PPT], r[PPT], sx[PPT];
@@ -634,7 +848,9 @@ __global__ __launch_bounds__(NT) void k_sweep1(const Q *__restrict__ qs, T *__re
                                                           Phys ph, long N, Metric<T> mt, Penal<T> pe) {
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER>(op, tp);
-  if constexpr (DIR == 1 && stress_form<T, FORM>())
+  if constexpr (DIR == 0 && stress_form<T, FORM>())
+    sweep1_x_cart(tp, qs, rhs, G, op, g, ph, N, ln);
+  else if constexpr (DIR == 1 && stress_form<T, FORM>())
     sweep1_y_stress(tp, qs, rhs, G, op, g, ph, N, ln);
   else
     sweep1_body<T, Q, DIR, FORM>(tp, qs, rhs, G, op, g, ph, N, mt, pe, ln);
@@ -678,15 +894,26 @@ struct RkIn {
   T a[PPT], b[PPT], c[PPT];
 };
 
-template <int DIR, int RK, typename T>
-__device__ __forceinline__ void rk_load(const RkArgs<T> &rk, int v, long B, long PS, long N, RkIn<RK, T> &in) {
+// (issued; rk_got makes the values the thread's own)
+template <int RK, typename T, typename IO>
+__device__ __forceinline__ void rk_load(const RkArgs<T> &rk, int v, const IO &io, long N, RkIn<RK, T> &in) {
   if constexpr (RK == RK_RHS) return;
-  if constexpr (!(RK == RK_LAST && sizeof(T) == 8)) ld<DIR>(rk.qn + v * N, B, PS, in.q0);
-  if constexpr (RK == RK_MID || RK == RK_LAST) ld<DIR>(rk.acc + v * N, B, PS, in.a);
+  if constexpr (!(RK == RK_LAST && sizeof(T) == 8)) io.ld(rk.qn + v * N, in.q0);
+  if constexpr (RK == RK_MID || RK == RK_LAST) io.ld(rk.acc + v * N, in.a);
   if constexpr (RK == RK_YLAST) {
-    ld<DIR>(rk.y2 + v * N, B, PS, in.a);
-    ld<DIR>(rk.y3 + v * N, B, PS, in.b);
-    ld<DIR>(rk.y4 + v * N, B, PS, in.c);
+    io.ld(rk.y2 + v * N, in.a);
+    io.ld(rk.y3 + v * N, in.b);
+    io.ld(rk.y4 + v * N, in.c);
+  }
+}
+template <int RK, typename T, typename IO>
+__device__ __forceinline__ void rk_got(const IO &io, RkIn<RK, T> &in) {
+  if constexpr (RK == RK_RHS) return;
+  if constexpr (!(RK == RK_LAST && sizeof(T) == 8)) io.got(in.q0);
+  if constexpr (RK == RK_MID || RK == RK_LAST || RK == RK_YLAST) io.got(in.a);
+  if constexpr (RK == RK_YLAST) {
+    io.got(in.b);
+    io.got(in.c);
   }
 }
 
@@ -708,15 +935,15 @@ __device__ __forceinline__ void rk_new_state(const RkArgs<T> &rk, const T (&k)[P
   }
 }
 
-template <int DIR, int RK, typename T>
-__device__ __forceinline__ void rk_store(const RkArgs<T> &rk, int v, const T (&k)[PPT], const RkIn<RK, T> &in, long B,
-                                         long PS, long N, T *rhs) {
+template <int RK, typename T, typename IO>
+__device__ __forceinline__ void rk_store(const RkArgs<T> &rk, int v, const T (&k)[PPT], const RkIn<RK, T> &in,
+                                         const IO &io, long N, T *rhs) {
   if constexpr (RK == RK_RHS) {
-    st<DIR>(rhs + v * N, B, PS, k);
+    io.st(rhs + v * N, k);
   } else if constexpr (RK == RK_LAST || RK == RK_YLAST) {
     double q1[PPT];
     rk_new_state<RK, T>(rk, k, in, q1);
-    st<DIR>(rk.qn + v * N, B, PS, q1);
+    io.st(rk.qn + v * N, q1);
   } else {
     double a[PPT];
     if constexpr (RK != RK_Y) {
@@ -726,26 +953,28 @@ __device__ __forceinline__ void rk_store(const RkArgs<T> &rk, int v, const T (&k
 #pragma unroll
       for (int m = 0; m < PPT; ++m)
         a[m] = RK == RK_FIRST ? base * in.q0[m] + dt / 6.0 * double(k[m]) : in.a[m] + dt / 3.0 * double(k[m]);
-      st<DIR>(rk.acc + v * N, B, PS, a);
+      io.st(rk.acc + v * N, a);
     }
 #pragma unroll
     for (int m = 0; m < PPT; ++m) a[m] = in.q0[m] + rk.c * double(k[m]);
-    st<DIR>(rk.out + v * N, B, PS, a);
+    io.st(rk.out + v * N, a);
   }
 }
 
 // RK_YLAST's new state with one kept stage input live at a time, for the
 // sweeps that have no registers for three
-template <int DIR>
-__device__ __forceinline__ void rk_ylast(const RkArgs<double> &rk, int v, const double (&k)[PPT], long B, long PS,
-                                         long N, double (&q1)[PPT]) {
+template <typename IO>
+__device__ __forceinline__ void rk_ylast(const RkArgs<double> &rk, int v, const double (&k)[PPT], const IO &io, long N,
+                                         double (&q1)[PPT]) {
   double q0[PPT], d[PPT];
   asm volatile("" ::: "memory");
-  ld<DIR>(rk.qn + v * N, B, PS, q0);
+  io.ld(rk.qn + v * N, q0);
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     double y[PPT];
-    ld<DIR>((j == 0 ? rk.y2 : (j == 1 ? rk.y3 : rk.y4)) + v * N, B, PS, y);
+    io.ld((j == 0 ? rk.y2 : (j == 1 ? rk.y3 : rk.y4)) + v * N, y);
+    if (j == 0) io.got(q0);
+    io.got(y);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       const double e = y[m] - q0[m];
@@ -759,14 +988,15 @@ __device__ __forceinline__ void rk_ylast(const RkArgs<double> &rk, int v, const 
 
 // the form chosen at run time (uniform), for the sweeps whose instances are
 // not worth one per form; Y: the forms without an accumulator
-template <int DIR, typename T, bool Y>
-__device__ __forceinline__ void rk_update(int form, const RkArgs<T> &rk, int v, const T (&k)[PPT], long B, long PS,
+template <bool Y, typename T, typename IO>
+__device__ __forceinline__ void rk_update(int form, const RkArgs<T> &rk, int v, const T (&k)[PPT], const IO &io,
                                           long N, T *rhs) {
 #define CRUNA_RK(F)                                 \
   {                                                 \
     RkIn<F, T> in;                                  \
-    rk_load<DIR, F, T>(rk, v, B, PS, N, in);        \
-    rk_store<DIR, F, T>(rk, v, k, in, B, PS, N, rhs); \
+    rk_load<F, T>(rk, v, io, N, in);                \
+    rk_got<F, T>(io, in);                           \
+    rk_store<F, T>(rk, v, k, in, io, N, rhs);       \
   }
   if (form == RK_RHS) CRUNA_RK(RK_RHS)
   else if constexpr (Y) {
@@ -774,8 +1004,8 @@ __device__ __forceinline__ void rk_update(int form, const RkArgs<T> &rk, int v, 
       CRUNA_RK(RK_Y)
     } else {
       double q1[PPT];
-      rk_ylast<DIR>(rk, v, k, B, PS, N, q1);
-      st<DIR>(rk.qn + v * N, B, PS, q1);
+      rk_ylast(rk, v, k, io, N, q1);
+      io.st(rk.qn + v * N, q1);
     }
   } else {
     if (form == RK_FIRST) CRUNA_RK(RK_FIRST)
@@ -784,14 +1014,15 @@ __device__ __forceinline__ void rk_update(int form, const RkArgs<T> &rk, int v, 
   }
 #undef CRUNA_RK
 }
-template <int DIR, typename T, bool Y>
-__device__ __forceinline__ void rk_final(const RkArgs<T> &rk, int v, const T (&k)[PPT], long B, long PS, long N,
+template <bool Y, typename T, typename IO>
+__device__ __forceinline__ void rk_final(const RkArgs<T> &rk, int v, const T (&k)[PPT], const IO &io, long N,
                                          double (&q1)[PPT]) {
   if constexpr (Y) {
-    rk_ylast<DIR>(rk, v, k, B, PS, N, q1);
+    rk_ylast(rk, v, k, io, N, q1);
   } else {
     RkIn<RK_LAST, T> in;
-    rk_load<DIR, RK_LAST, T>(rk, v, B, PS, N, in);
+    rk_load<RK_LAST, T>(rk, v, io, N, in);
+    rk_got<RK_LAST, T>(io, in);
     rk_new_state<RK_LAST, T>(rk, k, in, q1);
   }
 }
@@ -819,25 +1050,37 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
   static_assert(!FF || RK == RK_LAST || RK == RK_YLAST, "the x filter follows the last stage");
   constexpr bool GT = FORM == RHS_GT, EV = FORM == RHS_EV;
   constexpr bool LAST = DIR == 0;
-  const long B = tp.base, PS = g.PS;
+  const FieldIO<DIR, T> io(tp, g);
   const T ih = GT ? T(ph.inv_h[DIR]) * mt.m[DIR][tp.lidx] : T(ph.inv_h[DIR]);
   constexpr bool ST = stress_form<T, FORM>();
   T t1[PPT], t2[PPT], t3[PPT], diss[PPT];
   if constexpr (ST) {
     // tau_11, tau_12, tau_13 (x) or tau_22, tau_23 (y)
-    if (LAST) ld<DIR>(G, B, PS, t1);
-    ld<DIR>(G + (LAST ? 3 : 1) * N, B, PS, t2);
-    ld<DIR>(G + (LAST ? 4 : 5) * N, B, PS, t3);
+    if (LAST) io.ld(G, t1);
+    io.ld(G + (LAST ? 3 : 1) * N, t2);
+    io.ld(G + (LAST ? 4 : 5) * N, t3);
+    if (LAST) {
+      issue_loads();
+      io.got(t1);
+      io.got(t2);
+      io.got(t3);
+    }
   } else {
     T mu[PPT], ux[PPT], vy[PPT], wz[PPT], sa[PPT], sb[PPT];
-    ld<DIR>(G + 6 * N, B, PS, mu);
-    ld<DIR>(G + 0 * N, B, PS, ux);
-    ld<DIR>(G + 1 * N, B, PS, vy);
-    ld<DIR>(G + 2 * N, B, PS, wz);
+    io.ld(G + 6 * N, mu);
+    io.ld(G + 0 * N, ux);
+    io.ld(G + 1 * N, vy);
+    io.ld(G + 2 * N, wz);
     // x: s12 = u_y + v_x, s13 = u_z + w_x;  y: s12, s23 = v_z + w_y;  z: s13, s23
-    ld<DIR>(G + (DIR == 2 ? 4 : 3) * N, B, PS, sa);
-    ld<DIR>(G + (DIR == 0 ? 4 : 5) * N, B, PS, sb);
+    io.ld(G + (DIR == 2 ? 4 : 3) * N, sa);
+    io.ld(G + (DIR == 0 ? 4 : 5) * N, sb);
     issue_loads();
+    io.got(mu);
+    io.got(ux);
+    io.got(vy);
+    io.got(wz);
+    io.got(sa);
+    io.got(sb);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       const T md = -2.0 / 3.0 * mu[m] * (ux[m] + vy[m] + wz[m]);
@@ -864,14 +1107,18 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     materialize(t2);
     materialize(t3);
     if (LAST) {
-      ld<DIR>(G + 5 * N, B, PS, sa);
+      io.ld(G + 5 * N, sa);
+      io.got(sa);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) diss[m] = diss[m] + (mu[m] * sa[m]) * sa[m];
       materialize(diss);
     }
   }
   T Jv[PPT];
-  if (LAST && GT) ld<DIR>(mt.J, B, PS, Jv);
+  if (LAST && GT) {
+    io.ld(mt.J, Jv);
+    io.got(Jv);
+  }
   // the last sweep's complete RHS of variable v: what its RK4 update reads is
   // loaded together with the RHS; on the final stage optionally the x filter
   // of the new state
@@ -880,7 +1127,8 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     // complete RHS, here the learned closure; null when there is none
     if (force) {
       T fv[PPT];
-      ld<DIR>(force + v * N, B, PS, fv);
+      io.ld(force + v * N, fv);
+      io.got(fv);
 #pragma unroll
       for (int m = 0; m < PPT; ++m) k[m] = k[m] + fv[m];
     }
@@ -893,9 +1141,9 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
       ln.bind(fop);
       ln.template solve<true>(fop, f, x);
       ln.bind(op);
-      st<DIR>(rk.qn + v * N, B, PS, x);
+      io.st(rk.qn + v * N, x);
     } else {
-      rk_store<DIR, RK, T>(rk, v, k, in, B, PS, N, rhs);
+      rk_store<RK, T>(rk, v, k, in, io, N, rhs);
     }
   };
   if constexpr (LAST) {
@@ -904,17 +1152,20 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     // updates go first, which frees the dissipation's registers for the solves
     // (the last stage of the form without an accumulator reads four more
     // fields per variable: it takes the two one after the other)
-    constexpr bool BOTH = RK != RK_YLAST;
+    // (FP32 keeps its registers for occupancy: 256^3 0.508 -> 0.478 ms)
+    constexpr bool BOTH = RK != RK_YLAST && sizeof(T) == 8;
     T k[PPT], e[PPT];
     RkIn<RK, T> in, ie;
-    ld<DIR>(rhs, B, PS, k);
-    rk_load<DIR, RK, T>(rk, 0, B, PS, N, in);
+    io.ld(rhs, k);
+    rk_load<RK, T>(rk, 0, io, N, in);
     if (BOTH) {
-      ld<DIR>(rhs + 4 * N, B, PS, e);
-      rk_load<DIR, RK, T>(rk, 4, B, PS, N, ie);
+      io.ld(rhs + 4 * N, e);
+      rk_load<RK, T>(rk, 4, io, N, ie);
     }
     issue_loads();
     if (RK != RK_RHS || GT || force) {
+      io.got(k);
+      rk_got<RK, T>(io, in);
       if (GT) {
 #pragma unroll
         for (int m = 0; m < PPT; ++m) k[m] = Jv[m] * k[m];
@@ -923,9 +1174,11 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     }
     if (!BOTH) {
       asm volatile("" ::: "memory");
-      ld<DIR>(rhs + 4 * N, B, PS, e);
-      rk_load<DIR, RK, T>(rk, 4, B, PS, N, ie);
+      io.ld(rhs + 4 * N, e);
+      rk_load<RK, T>(rk, 4, io, N, ie);
     }
+    io.got(e);
+    rk_got<RK, T>(io, ie);
 #pragma unroll
     for (int m = 0; m < PPT; ++m)
       e[m] = GT ? (Jv[m] * T(ph.gm1)) * (e[m] + Jv[m] * diss[m]) : T(ph.gm1) * (ST ? e[m] : e[m] + diss[m]);
@@ -935,8 +1188,10 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
   T IP[PPT];
   if (EV) {  // phi tau_id inside the derivative, 1/phi on it
     T PH[PPT];
-    ld<DIR>(pe.phi, B, PS, PH);
-    ld<DIR>(pe.inv_phi, B, PS, IP);
+    io.ld(pe.phi, PH);
+    io.ld(pe.inv_phi, IP);
+    io.got(PH);
+    io.got(IP);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       t1[m] = PH[m] * t1[m];
@@ -946,7 +1201,9 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
   }
   // z/y: read-modify-write of the momentum accumulators; x: the complete RHS
   // of that variable and its RK4 update
-  auto complete = [&](int v, const T(&x)[PPT], T(&k)[PPT], const RkIn<RK, T> &in) {
+  auto complete = [&](int v, const T(&x)[PPT], T(&k)[PPT], RkIn<RK, T> &in) {
+    io.got(k);
+    if constexpr (LAST) rk_got<RK, T>(io, in);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) {
       k[m] = k[m] + (EV ? IP[m] * (x[m] * ih) : x[m] * ih);
@@ -955,13 +1212,13 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     if constexpr (LAST)
       finish(v, k, in);
     else
-      st<DIR>(rhs + v * N, B, PS, k);
+      io.st(rhs + v * N, k);
   };
   if constexpr (ST && !LAST) {
     T x[PPT], y[PPT], k[PPT], l[PPT];
-    const RkIn<RK, T> none{};
-    ld<DIR>(rhs + 2 * N, B, PS, k);
-    ld<DIR>(rhs + 3 * N, B, PS, l);
+    RkIn<RK, T> none{};
+    io.ld(rhs + 2 * N, k);
+    io.ld(rhs + 3 * N, l);
     ln.solve2(op, t2, x, t3, y);
     complete(2, x, k, none);
     complete(3, y, l, none);
@@ -971,36 +1228,37 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     // two stresses at once, the first accumulator in flight meanwhile
     T x[PPT], y[PPT], k[PPT];
     RkIn<RK, T> in;
-    constexpr bool EARLY = RK != RK_YLAST;
+    constexpr bool EARLY = RK != RK_YLAST && sizeof(T) == 8;
     if (EARLY) {
-      ld<DIR>(rhs + N, B, PS, k);
-      if constexpr (LAST) rk_load<DIR, RK, T>(rk, 1, B, PS, N, in);
+      io.ld(rhs + N, k);
+      if constexpr (LAST) rk_load<RK, T>(rk, 1, io, N, in);
     }
     ln.solve2(op, t1, x, t2, y);
     asm volatile("" ::: "memory");
     if (!EARLY) {
-      ld<DIR>(rhs + N, B, PS, k);
-      if constexpr (LAST) rk_load<DIR, RK, T>(rk, 1, B, PS, N, in);
+      io.ld(rhs + N, k);
+      if constexpr (LAST) rk_load<RK, T>(rk, 1, io, N, in);
     }
     complete(1, x, k, in);
     asm volatile("" ::: "memory");
-    ld<DIR>(rhs + 2 * N, B, PS, k);
-    if constexpr (LAST) rk_load<DIR, RK, T>(rk, 2, B, PS, N, in);
+    io.ld(rhs + 2 * N, k);
+    if constexpr (LAST) rk_load<RK, T>(rk, 2, io, N, in);
     complete(2, y, k, in);
   }
   {
     T x[PPT], k[PPT];
     RkIn<RK, T> in;
     asm volatile("" ::: "memory");
-    if (RK != RK_YLAST) {
-      ld<DIR>(rhs + 3 * N, B, PS, k);
-      if constexpr (LAST) rk_load<DIR, RK, T>(rk, 3, B, PS, N, in);
+    constexpr bool EARLY = RK != RK_YLAST && sizeof(T) == 8;
+    if (EARLY) {
+      io.ld(rhs + 3 * N, k);
+      if constexpr (LAST) rk_load<RK, T>(rk, 3, io, N, in);
     }
     ln.solve(op, t3, x);
-    if (RK == RK_YLAST) {
+    if (!EARLY) {
       asm volatile("" ::: "memory");
-      ld<DIR>(rhs + 3 * N, B, PS, k);
-      if constexpr (LAST) rk_load<DIR, RK, T>(rk, 3, B, PS, N, in);
+      io.ld(rhs + 3 * N, k);
+      if constexpr (LAST) rk_load<RK, T>(rk, 3, io, N, in);
     }
     complete(3, x, k, in);
   }
@@ -1089,12 +1347,14 @@ __global__ __launch_bounds__(NT) void k_diff(const T *__restrict__ in, T *__rest
                                              Op<T> op, SweepGeom g, double inv_h) {
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER>(op, tp);
+  const FieldIO<DIR, T> io(tp, g);
   T f[PPT], x[PPT];
-  ld<DIR>(in, tp.base, g.PS, f);
+  io.ld(in, f);
+  io.got(f);
   ln.solve(op, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) x[m] = x[m] * T(inv_h);
-  st<DIR>(out, tp.base, g.PS, x);
+  io.st(out, x);
 }
 
 // Filter of nv fields in place (filter_4d): q = B_f^-1 A_f q per field.
@@ -1108,19 +1368,21 @@ constexpr int filter_nt() { return sizeof(T) == 4 ? NT_FILTER32 : NT; }
 template <typename T, int DIR, typename S, typename LOp, typename Lines>
 __device__ __forceinline__ void filter_body(const ThreadPos &tp, const S *src, double *q64, const LOp &op,
                                             const SweepGeom &g, long N, int nv, T *copy, Lines &ln) {
+  const FieldIO<DIR, T> io(tp, g);
   double a[PPT];
-  ld<DIR>(src, tp.base, g.PS, a);
+  io.ld(src, a);
   for (int v = 0; v < nv; ++v) {
     T f[PPT], x[PPT];
+    io.got(a);
 #pragma unroll
     for (int m = 0; m < PPT; ++m) f[m] = T(a[m]);
     // the next field's loads fly while this one is filtered
-    if (v + 1 < nv) ld<DIR>(src + (v + 1) * N, tp.base, g.PS, a);
+    if (v + 1 < nv) io.ld(src + (v + 1) * N, a);
     ln.template solve<true>(op, f, x);
-    if (q64) st<DIR>(q64 + v * N, tp.base, g.PS, x);
+    if (q64) io.st(q64 + v * N, x);
     // the filtered state in the compute precision, when the next RK stage
     // or filter pass reads it (it equals the FP64 value converted back)
-    if (copy) st<DIR>(copy + v * N, tp.base, g.PS, x);
+    if (copy) io.st(copy + v * N, x);
   }
 }
 
