@@ -21,6 +21,7 @@
 #include "weighted_filter.hpp"
 #include "adjoint.hpp"
 #include "counters.hpp"
+#include "host_copy.hpp"
 #include "closure.hpp"
 #include "residual.hpp"
 #include "batch.hpp"
@@ -127,6 +128,7 @@ struct cruna_hip_cnn;
 // count of the contexts a closure is attached to (cruna_hip_set_closure)
 static void cnn_user(cruna_hip_cnn *n, int delta);
 struct cruna_hip_ctx {
+  HostCopyUser copies;
   cruna_hip_cfg cfg{};
   int device = 0;
   hipStream_t stream = nullptr;
@@ -148,6 +150,7 @@ struct cruna_hip_ctx {
   Phys phys{};
   // device state
   double *qn = nullptr, *acc = nullptr, *qref = nullptr, *shape = nullptr, *tmp = nullptr;
+  double *real = nullptr;  // padded layout: the real points of up to 5 fields
   // boundary_conditions.dat rows in file order (types 201, 400, 401)
   std::vector<std::pair<int, BoxRow>> bc;
   bool has_bcq = false, has_bcrhs = false;
@@ -1011,43 +1014,46 @@ std::vector<double> pad_host(const cruna_hip_ctx *c, const double *h, int nv, co
   return out;
 }
 
-// the real points of nv padded device-layout fields into a host array
-void unpad_host(const cruna_hip_ctx *c, const std::vector<double> &d, double *h, int nv) {
-  const long n1 = c->cfg.n[0], n2 = c->cfg.n[1], n3 = c->cfg.n[2];
-  const long p1 = c->np[0], p2 = c->np[1], N = c->N, Nr = n1 * n2 * n3;
-  for (int v = 0; v < nv; ++v)
-    for (long k = 0; k < n3; ++k)
-      for (long j = 0; j < n2; ++j)
-        for (long i = 0; i < n1; ++i)
-          h[v * Nr + i + n1 * (j + n2 * k)] =
-              d[(size_t)v * N + (i + c->pf[0]) + p1 * ((j + c->pf[1]) + p2 * (k + c->pf[2]))];
+PadLayout pad_layout(const cruna_hip_ctx *c) {
+  return PadLayout{c->cfg.n[0], c->cfg.n[1], c->cfg.n[2], c->np[0], c->np[1], c->np[2], c->pf[0], c->pf[1], c->pf[2]};
 }
+long real_points(const cruna_hip_ctx *c) { return (long)c->cfg.n[0] * c->cfg.n[1] * c->cfg.n[2]; }
+unsigned grid_for(long n) { return (unsigned)std::min<long>(8192, (n + 255) / 256); }
 
-// host -> device fields (asynchronous on the context stream when unpadded,
-// as the plain copies were; waits for the staging copy when padded)
-int put_fields(cruna_hip_ctx *c, double *dev, const double *host, int nv, const double *fill) {
-  const size_t bytes = (size_t)nv * c->N * sizeof(double);
-  if (!c->padded) {
-    HIP_TRY(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, c->stream));
-    return CRUNA_HIP_OK;
-  }
-  std::vector<double> v = pad_host(c, host, nv, fill);
-  HIP_TRY(hipMemcpyAsync(dev, v.data(), bytes, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+int ensure_real(cruna_hip_ctx *c) {
+  if (!c->real) HIP_TRY(hipMalloc(&c->real, 5 * real_points(c) * sizeof(double)));
   return CRUNA_HIP_OK;
 }
 
-// device -> host fields (the real points)
-int get_fields(cruna_hip_ctx *c, double *host, const double *dev, int nv) {
-  const size_t bytes = (size_t)nv * c->N * sizeof(double);
+// host -> device fields (padding points fill[v], fill null: 0)
+int put_fields(cruna_hip_ctx *c, double *dev, const double *host, int nv, const double *fill) {
+  HostCopyPool &pool = HostCopyPool::get();
   if (!c->padded) {
-    HIP_TRY(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(pool.copy(dev, host, (size_t)nv * c->N * sizeof(double), true, c->device, c->stream));
     return CRUNA_HIP_OK;
   }
-  std::vector<double> v((size_t)nv * c->N);
-  HIP_TRY(hipMemcpyAsync(v.data(), dev, bytes, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  unpad_host(c, v, host, nv);
+  if (int rc = ensure_real(c)) return rc;
+  HIP_TRY(pool.copy(c->real, host, (size_t)nv * real_points(c) * sizeof(double), true, c->device, c->stream));
+  PadFill f{};
+  for (int v = 0; fill && v < nv; ++v) f.v[v] = fill[v];
+  hipLaunchKernelGGL(k_scatter_real, dim3(grid_for(nv * c->N)), dim3(256), 0, c->stream, (const double *)c->real, dev,
+                     nv, pad_layout(c), f);
+  return check_launch();
+}
+
+// device -> host fields (the real points); done when it returns
+int get_fields(cruna_hip_ctx *c, double *host, const double *dev, int nv) {
+  HostCopyPool &pool = HostCopyPool::get();
+  if (!c->padded) {
+    HIP_TRY(pool.copy(host, dev, (size_t)nv * c->N * sizeof(double), false, c->device, c->stream));
+    return CRUNA_HIP_OK;
+  }
+  if (int rc = ensure_real(c)) return rc;
+  const long n = nv * real_points(c);
+  hipLaunchKernelGGL((k_gather_real<double>), dim3(grid_for(n)), dim3(256), 0, c->stream, dev, c->real, nv,
+                     pad_layout(c));
+  if (int rc = check_launch()) return rc;
+  HIP_TRY(pool.copy(host, c->real, (size_t)n * sizeof(double), false, c->device, c->stream));
   return CRUNA_HIP_OK;
 }
 
@@ -1059,21 +1065,13 @@ int ensure_tmp(cruna_hip_ctx *c) {
 
 // The RHS (compute precision) back to a host FP64 array.
 int copy_rhs_out(cruna_hip_ctx *c, double *rhs) {
-  if (c->cfg.precision == CRUNA_HIP_FP32_MIXED) {
-    std::vector<float> h(5 * c->N);
-    HIP_TRY(hipMemcpyAsync(h.data(), c->rhs, 5 * c->N * sizeof(float), hipMemcpyDeviceToHost,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (!c->padded) {
-      for (long i = 0; i < 5 * c->N; ++i) rhs[i] = h[i];
-    } else {
-      std::vector<double> d(h.begin(), h.end());
-      unpad_host(c, d, rhs, 5);
-    }
-  } else {
-    if (int rc = get_fields(c, rhs, (const double *)c->rhs, 5)) return rc;
-    HIP_TRY(hipStreamSynchronize(c->stream));
-  }
+  if (c->cfg.precision != CRUNA_HIP_FP32_MIXED) return get_fields(c, rhs, (const double *)c->rhs, 5);
+  // the real points in FP64, in the first half of the staging area
+  const long n = 5 * real_points(c);
+  hipLaunchKernelGGL((k_gather_real<float>), dim3(grid_for(n)), dim3(256), 0, c->stream, (const float *)c->rhs, c->tmp,
+                     5, pad_layout(c));
+  if (int rc = check_launch()) return rc;
+  HIP_TRY(HostCopyPool::get().copy(rhs, c->tmp, (size_t)n * sizeof(double), false, c->device, c->stream));
   return CRUNA_HIP_OK;
 }
 
@@ -1533,7 +1531,7 @@ int cruna_hip_destroy(cruna_hip_ctx *c) {
   for (void *p : {(void *)c->qn, (void *)c->acc, (void *)c->qref, (void *)c->shape, (void *)c->tmp,
                   (void *)c->qa, (void *)c->traj, (void *)c->gobj, c->met, (void *)c->q0p, c->force,
                   (void *)c->ckpt, c->tg, c->pen, (void *)c->wphi, (void *)c->wtmp, (void *)c->wbuf,
-                  (void *)c->kvec, (void *)c->y4, (void *)c->q0copy, (void *)c->res_buf,
+                  (void *)c->kvec, (void *)c->y4, (void *)c->real, (void *)c->q0copy, (void *)c->res_buf,
                   c->qs, c->rhs, c->G})
     if (p) (void)hipFree(p);
   for (auto &p : c->pending) {
@@ -2842,6 +2840,8 @@ int cruna_hip_ensemble_autotune(cruna_hip_ensemble *e, int steps, int *tile_line
 // Learned subfilter closure (closure.hpp): a 3-D CNN on a periodic S^3 grid.
 
 struct cruna_hip_cnn {
+  HostCopyUser copies;
+  int device = 0;
   int S = 0;
   long N = 0;  // S^3
   hipStream_t stream = nullptr;
@@ -3064,8 +3064,9 @@ int cnn_stage(cruna_hip_cnn *n, const double *q, const double *target, StageWhat
   if (!n->stage) HIP_TRY(hipMalloc(&n->stage, 10 * n->N * sizeof(double)));
   const unsigned nb = (unsigned)((n->N + 255) / 256);
   double *qd = n->stage, *td = n->stage + 5 * n->N;
-  HIP_TRY(hipMemcpyAsync(qd, q, 5 * n->N * sizeof(double), hipMemcpyHostToDevice, n->stream));
-  if (target) HIP_TRY(hipMemcpyAsync(td, target, 5 * n->N * sizeof(double), hipMemcpyHostToDevice, n->stream));
+  HostCopyPool &pool = HostCopyPool::get();
+  HIP_TRY(pool.copy(qd, q, 5 * n->N * sizeof(double), true, n->device, n->stream));
+  if (target) HIP_TRY(pool.copy(td, target, 5 * n->N * sizeof(double), true, n->device, n->stream));
   if (what == STAGE_FORCE) {
     if (int rc = closure_eval<double, double>(n, n->stream, qd, td)) return rc;
   } else {
@@ -3094,6 +3095,7 @@ int cruna_hip_cnn_create(int S, cruna_hip_cnn **out) {
   *out = nullptr;
   if (S < 16 || S > 512 || (S & (S - 1)) != 0) return fail(CRUNA_HIP_EINVAL, "S must be a power of two in [16, 512]");
   std::unique_ptr<cruna_hip_cnn> n(new cruna_hip_cnn());
+  HIP_TRY(hipGetDevice(&n->device));
   n->S = S;
   n->N = (long)S * S * S;
   long o = 0, pk = 0;
@@ -3218,9 +3220,7 @@ int cruna_hip_cnn_set_gain(cruna_hip_cnn *n, const double gain[5]) {
 int cruna_hip_cnn_forward(cruna_hip_cnn *n, const double *q, double *closure) {
   if (!n || !q || !closure) return fail(CRUNA_HIP_EINVAL, "null argument");
   if (int rc = cnn_stage(n, q, nullptr, STAGE_FORCE)) return rc;
-  HIP_TRY(hipMemcpyAsync(closure, n->stage + 5 * n->N, 5 * n->N * sizeof(double), hipMemcpyDeviceToHost,
-                         n->stream));
-  HIP_TRY(hipStreamSynchronize(n->stream));
+  HIP_TRY(HostCopyPool::get().copy(closure, n->stage + 5 * n->N, 5 * n->N * sizeof(double), false, n->device, n->stream));
   return CRUNA_HIP_OK;
 }
 
@@ -3380,36 +3380,6 @@ int scratch_on(int dev, double **out) {
   return CRUNA_HIP_OK;
 }
 
-// Real points (n1, n2, n3; contiguous, Fortran order) of nv fields into the
-// padded device layout (np1, np2, np3, front padding pf), padding points set
-// to fill[v].
-__global__ void k_scatter_real(const double *__restrict__ src, double *__restrict__ dst, int nv, int n1, int n2,
-                               int n3, int p1, int p2, int p3, int f1, int f2, int f3, double fill0,
-                               double fill4) {
-  const long N = (long)p1 * p2 * p3, Nr = (long)n1 * n2 * n3;
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < nv * N; t += (long)gridDim.x * blockDim.x) {
-    const int v = (int)(t / N);
-    const long p = t - v * N;
-    const int i = (int)(p % p1) - f1, j = (int)((p / p1) % p2) - f2, k = (int)(p / ((long)p1 * p2)) - f3;
-    const bool real = i >= 0 && i < n1 && j >= 0 && j < n2 && k >= 0 && k < n3;
-    dst[t] = real ? src[v * Nr + i + (long)n1 * (j + (long)n2 * k)] : (v == 0 ? fill0 : (v == 4 ? fill4 : 0.0));
-  }
-}
-
-// The real points of nv padded device-layout fields (type T) into a
-// contiguous FP64 array.
-template <typename T>
-__global__ void k_gather_real(const T *__restrict__ src, double *__restrict__ dst, int nv, int n1, int n2, int n3,
-                              int p1, int p2, int p3, int f1, int f2, int f3) {
-  const long N = (long)p1 * p2 * p3, Nr = (long)n1 * n2 * n3;
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < nv * Nr; t += (long)gridDim.x * blockDim.x) {
-    const int v = (int)(t / Nr);
-    const long r = t - v * Nr;
-    const int i = (int)(r % n1), j = (int)((r / n1) % n2), k = (int)(r / ((long)n1 * n2));
-    dst[t] = double(src[v * N + (i + f1) + (long)p1 * ((j + f2) + (long)p2 * (k + f3))]);
-  }
-}
-
 }  // namespace
 
 extern "C" {
@@ -3427,23 +3397,22 @@ int cruna_hip_rhs_direct_noalloc(cruna_hip_ctx *c, double *rhs, const double *q,
   if (int rc = scratch_on(c->device, &s)) return rc;
   double *stage = s, *real = s + 5 * c->N;
   c->qs_fresh = false;
-  const int *np = c->np, *pf = c->pf;
-  const unsigned blocks = (unsigned)std::min<long>(8192, (5 * c->N + 255) / 256);
+  const unsigned blocks = grid_for(5 * c->N);
+  const PadLayout lay = pad_layout(c);
+  PadFill fill;
+  for (int v = 0; v < 5; ++v) fill.v[v] = kRestState[v];
   // the input state: contiguous host copy, then the device layout
   HIP_TRY(hipMemcpyAsync(real, q, 5 * Nr * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_scatter_real, dim3(blocks), dim3(256), 0, c->stream, (const double *)real, stage, 5, n[0],
-                     n[1], n[2], np[0], np[1], np[2], pf[0], pf[1], pf[2], kRestState[0], kRestState[4]);
+  hipLaunchKernelGGL(k_scatter_real, dim3(blocks), dim3(256), 0, c->stream, (const double *)real, stage, 5, lay, fill);
   if (int rc = check_launch()) return rc;
   const bool mixed = c->cfg.precision == CRUNA_HIP_FP32_MIXED;
   int rc = mixed ? run_stage<float>(c, stage, 4) : run_stage<double>(c, stage, 4);
   if (rc) return rc;
   // the RHS: real points in FP64, then to the host
   if (mixed)
-    hipLaunchKernelGGL((k_gather_real<float>), dim3(blocks), dim3(256), 0, c->stream, (const float *)c->rhs, real,
-                       5, n[0], n[1], n[2], np[0], np[1], np[2], pf[0], pf[1], pf[2]);
+    hipLaunchKernelGGL((k_gather_real<float>), dim3(blocks), dim3(256), 0, c->stream, (const float *)c->rhs, real, 5, lay);
   else
-    hipLaunchKernelGGL((k_gather_real<double>), dim3(blocks), dim3(256), 0, c->stream, (const double *)c->rhs,
-                       real, 5, n[0], n[1], n[2], np[0], np[1], np[2], pf[0], pf[1], pf[2]);
+    hipLaunchKernelGGL((k_gather_real<double>), dim3(blocks), dim3(256), 0, c->stream, (const double *)c->rhs, real, 5, lay);
   if (int rc2 = check_launch()) return rc2;
   HIP_TRY(hipMemcpyAsync(rhs, real, 5 * Nr * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
