@@ -77,54 +77,7 @@ __device__ __forceinline__ Coord coord_of(long p, const ConvGeom &g) {
   return Coord{(int)(r2 - (long)j * g.X), j, k, (long)b * XYZ};
 }
 
-// neighbour of a point at tap t (t = 9 (dz+1) + 3 (dy+1) + (dx+1)), sign -1
-// for the transposed operator; -1 when it falls outside a crop
-__device__ __forceinline__ long tap_neighbour(const Coord &c, int t, int sign, const ConvGeom &g) {
-  int i = c.i + sign * (t % 3 - 1), j = c.j + sign * ((t / 3) % 3 - 1), k = c.k + sign * (t / 9 - 1);
-  if (g.periodic) {
-    i = i < 0 ? i + g.X : (i >= g.X ? i - g.X : i);
-    j = j < 0 ? j + g.Y : (j >= g.Y ? j - g.Y : j);
-    k = k < 0 ? k + g.Z : (k >= g.Z ? k - g.Z : k);
-  } else if (i < 0 || i >= g.X || j < 0 || j >= g.Y || k < 0 || k >= g.Z) {
-    return -1;
-  }
-  return c.base + i + (long)g.X * (j + (long)g.Y * k);
-}
-
 enum ConvMode { CONV_GELU = 0, CONV_LINEAR = 1, CONV_BACKWARD = 2 };
-
-// Per-point neighbour offsets along one direction: off[0..2] for d = -1, 0,
-// +1 (wrapped on periodic boxes) and a validity bit per d (crops).
-struct AxisOffsets {
-  int off[3];
-  unsigned valid;  // bit d
-};
-__device__ __forceinline__ AxisOffsets axis_offsets(int i, int X, int stride, bool periodic, int sign) {
-  AxisOffsets a;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    int ii = i + sign * (d - 1);
-    bool ok = true;
-    if (ii < 0) {
-      ok = periodic;
-      ii += X;
-    } else if (ii >= X) {
-      ok = periodic;
-      ii -= X;
-    }
-    a.off[d] = (ii - i) * stride;
-  }
-  a.valid = 0;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int ii = i + sign * (d - 1);
-    if (periodic || (ii >= 0 && ii < X)) a.valid |= 1u << d;
-  }
-  return a;
-}
-
-// a[d] for a runtime d in 0..2 without indexing a register array
-__device__ __forceinline__ int pick3(const int (&a)[3], int d) { return d == 0 ? a[0] : (d == 1 ? a[1] : a[2]); }
 
 // One convolution as an implicit GEMM on BF16 MFMA: out[p][co] over the 27
 // taps and CK input channels of each point's neighbours.
@@ -320,93 +273,157 @@ __global__ __launch_bounds__(CT_THREADS) void k_conv_tile(const bf16 *__restrict
   }
 }
 
-// Weight gradient partials of one tap: block (chunk, t) sums
-// dz[p][co] in[p + o_t][ci] over the chunk's points into
-// part[chunk][t][co][ci], as an MFMA GEMM with the points as reduction
-// index: sub-chunks of WG_SUB points of dz and of the tap-shifted input are
-// staged transposed in LDS ([channel][point]), so that every lane reads
-// its 4 consecutive points of one channel as one 8-byte word.  Blocks of
-// tap 0 also sum dz over their points into bpart[chunk][co] (bias
-// gradient partials).  Wavefront w takes the (co, ci) tile w (at most 4).
-constexpr int WG_SUB = 256;
-template <int CI, int CO>
-__global__ __launch_bounds__(256) void k_conv_wgrad(const bf16 *__restrict__ in, const bf16 *__restrict__ dz,
-                                                    ConvGeom geo, long npts, int chunk,
-                                                    float *__restrict__ part, float *__restrict__ bpart) {
-  constexpr int LD = WG_SUB + 8;
-  __shared__ __align__(16) bf16 dzT[CO * LD];
-  __shared__ __align__(16) bf16 inT[CI * LD];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, kg = lane >> 4;
-  const int t = blockIdx.y;
-  const int tx = t % 3, ty = (t / 3) % 3, tz = t / 9;
-  const int c0 = blockIdx.x * chunk;
-  const int c1 = c0 + chunk < npts ? c0 + chunk : (int)npts;
-  constexpr int NT_CI = CI / 16, NTILE = (CO / 16) * NT_CI;
-  static_assert(NTILE <= 4, "one tile per wavefront");
-  const bool has_tile = wave < NTILE;
-  const int mb = wave / NT_CI, nbk = wave % NT_CI;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.f;
-  const bool per = geo.periodic != 0;
-  for (int sp = c0; sp < c1; sp += WG_SUB) {
-    const int np = c1 - sp < WG_SUB ? c1 - sp : WG_SUB;  // a multiple of 16
-    __syncthreads();
-    for (int e = threadIdx.x; e < np * (CO / 8); e += 256) {
-      const int q = e / (CO / 8), piece = e % (CO / 8);
-      const uint4 v = *reinterpret_cast<const uint4 *>(dz + (long)(sp + q) * CO + piece * 8);
-      const unsigned w4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        dzT[(piece * 8 + 2 * u) * LD + q] = (bf16)(w4[u] & 0xffffu);
-        dzT[(piece * 8 + 2 * u + 1) * LD + q] = (bf16)(w4[u] >> 16);
-      }
-    }
-    for (int e = threadIdx.x; e < np * (CI / 8); e += 256) {
-      const int q = e / (CI / 8), piece = e % (CI / 8);
-      const Coord cc = coord_of(sp + q, geo);
-      const AxisOffsets ax = axis_offsets(cc.i, geo.X, 1, per, 1);
-      const AxisOffsets ay = axis_offsets(cc.j, geo.Y, geo.X, per, 1);
-      const AxisOffsets az = axis_offsets(cc.k, geo.Z, geo.X * geo.Y, per, 1);
-      const bool ok = per || ((ax.valid >> tx) & (ay.valid >> ty) & (az.valid >> tz) & 1u);
-      const int nb = sp + q + pick3(ax.off, tx) + pick3(ay.off, ty) + pick3(az.off, tz);
-      uint4 v = {0u, 0u, 0u, 0u};
-      if (ok) v = *reinterpret_cast<const uint4 *>(in + (long)nb * CI + piece * 8);
-      const unsigned w4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        inT[(piece * 8 + 2 * u) * LD + q] = (bf16)(w4[u] & 0xffffu);
-        inT[(piece * 8 + 2 * u + 1) * LD + q] = (bf16)(w4[u] >> 16);
-      }
-    }
-    __syncthreads();
-    if (has_tile)
-      for (int k = 0; k < np; k += 16) {
-        const bf16x4 a = *reinterpret_cast<const bf16x4 *>(dzT + (mb * 16 + r) * LD + k + 4 * kg);
-        const bf16x4 b = *reinterpret_cast<const bf16x4 *>(inT + (nbk * 16 + r) * LD + k + 4 * kg);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-      }
-    if (t == 0 && (int)threadIdx.x < CO)
-      for (int k = 0; k < np; ++k) bsum += from_bf16(dzT[threadIdx.x * LD + k]);
-  }
-  if (has_tile) {
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const int co = mb * 16 + 4 * kg + rr, ci = nbk * 16 + r;
-      part[(((long)blockIdx.x * 27 + t) * CO + co) * CI + ci] = acc[rr];
-    }
-  }
-  if (t == 0 && (int)threadIdx.x < CO) bpart[(long)blockIdx.x * CO + threadIdx.x] = bsum;
+// Weight gradient partials: work-group g sums dz[p][co] in[p + o_t][ci] over
+// its tiles (16 x 4 x 8 points, as k_conv_tile's) into part[g][t][co][ci] for
+// all 27 taps, as MFMA GEMMs with the points as reduction index.  A tile's dz and
+// its input with a one-point halo are staged in LDS once, rows of channels as
+// they lie in memory; the matrix operands, which run over points, come from
+// the LDS transpose read (16 lanes read 4 rows of 16 channels and each gets the
+// four values of its channel), so that a tap is nothing but another first row.
+// Wavefront w takes the taps w, w + 8, ... and keeps their accumulators over all
+// its tiles; wavefront 7 also sums dz (times ones) for the bias gradient.
+// Bound by LDS reads (2 per channel block and 16 points) and by the staging of
+// the next tile.  At 64^3 the 32 -> 32 layers take 40 us each, 16 -> 32 28 and
+// 32 -> 16 30; a kernel that read and transposed every point once per tap took
+// 217, 170 and 198.
+constexpr int WG_MAX = 256;  // work-groups: one per CU (100 KB of LDS)
+
+__device__ __forceinline__ bf16x4 read_points(const bf16 *p) {
+  typedef __attribute__((address_space(3))) bf16x4 lds4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)p);
 }
 
-// dW[e] = sum over chunks of part[chunk][e] (e over nelem entries)
-__global__ void k_sum_chunks(const float *__restrict__ part, int nchunks, long nelem,
-                             float *__restrict__ dW) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nelem) return;
+template <int CI, int CO>
+__global__ __launch_bounds__(CT_THREADS) void k_conv_wgrad(const bf16 *__restrict__ in, const bf16 *__restrict__ dz,
+                                                          ConvGeom geo, long npts, float *__restrict__ part,
+                                                          float *__restrict__ bpart) {
+  constexpr int CT_PTS = CT_X * CT_Y * CT_Z, WAVES = CT_Z, TAPS = (27 + WAVES - 1) / WAVES;
+  __shared__ __align__(16) bf16 dt[CT_PTS * CO];
+  __shared__ __align__(16) bf16 xt[CT_HALO * CI];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, kg = lane >> 4;
+  const bool per = geo.periodic != 0;
+  const int X = geo.X, Y = geo.Y, Z = geo.Z;
+  const long XYZ = (long)X * Y * Z;
+  const int nbx = (X + CT_X - 1) / CT_X, nby = (Y + CT_Y - 1) / CT_Y, nbz = (Z + CT_Z - 1) / CT_Z;
+  const int per_box = nbx * nby * nbz;
+  const int ntiles = (int)(npts / XYZ) * per_box;
+  const int G = gridDim.x, chunk = (ntiles + G - 1) / G;
+  const int t0 = blockIdx.x * chunk, t1 = t0 + chunk < ntiles ? t0 + chunk : ntiles;
+  f32x4 acc[TAPS][CO / 16][CI / 16], bacc[CO / 16];
+#pragma unroll
+  for (int m = 0; m < CO / 16; ++m) {
+    bacc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k)
+#pragma unroll
+      for (int n = 0; n < CI / 16; ++n) acc[k][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const bf16x4 ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};  // 1 in BF16
+  // row of this lane's 8 bytes of a 4 x 16 block: point 4 kg + r / 4, channels 4 (r % 4)..+3
+  const int prow = 4 * kg + r / 4, pch = 4 * (r % 4);
+  for (int tile = t0; tile < t1; ++tile) {
+    const int b = tile / per_box, rem = tile % per_box;
+    const int i0 = (rem % nbx) * CT_X, j0 = ((rem / nbx) % nby) * CT_Y, k0 = (rem / (nbx * nby)) * CT_Z;
+    const long base = (long)b * XYZ;
+    __syncthreads();  // the previous tile's reads are done
+    for (int e = threadIdx.x; e < CT_PTS * (CO / 8); e += CT_THREADS) {
+      const int q = e / (CO / 8), c8 = e % (CO / 8);
+      const int gi = i0 + q % CT_X, gj = j0 + (q / CT_X) % CT_Y, gk = k0 + q / (CT_X * CT_Y);
+      uint4 v = {0u, 0u, 0u, 0u};  // points beyond the box's far faces add nothing
+      if (gi < X && gj < Y && gk < Z)
+        v = *reinterpret_cast<const uint4 *>(dz + (base + gi + X * ((long)gj + (long)Y * gk)) * CO + c8 * 8);
+      *reinterpret_cast<uint4 *>(dt + e * 8) = v;
+    }
+    for (int e = threadIdx.x; e < CT_HALO * (CI / 8); e += CT_THREADS) {
+      const int q = e / (CI / 8), c8 = e % (CI / 8);
+      int gi = i0 + q % CH_X - 1, gj = j0 + (q / CH_X) % CH_Y - 1, gk = k0 + q / (CH_X * CH_Y) - 1;
+      bool ok = true;
+      if (per) {
+        gi = gi < 0 ? gi + X : (gi >= X ? gi - X : gi);
+        gj = gj < 0 ? gj + Y : (gj >= Y ? gj - Y : gj);
+        gk = gk < 0 ? gk + Z : (gk >= Z ? gk - Z : gk);
+      } else {
+        ok = gi >= 0 && gj >= 0 && gk >= 0;
+      }
+      ok = ok && gi < X && gj < Y && gk < Z;  // (wrapped once: further points meet dz = 0)
+      uint4 v = {0u, 0u, 0u, 0u};
+      if (ok) v = *reinterpret_cast<const uint4 *>(in + (base + gi + X * ((long)gj + (long)Y * gk)) * CI + c8 * 8);
+      *reinterpret_cast<uint4 *>(xt + e * 8) = v;
+    }
+    __syncthreads();
+    // the tile's x-rows of 16 points, one reduction step each
+#pragma unroll 2
+    for (int s = 0; s < CT_Y * CT_Z; ++s) {
+      const int y = s % CT_Y, z = s / CT_Y;
+      bf16x4 a[CO / 16];
+#pragma unroll
+      for (int m = 0; m < CO / 16; ++m) a[m] = read_points(dt + (s * CT_X + prow) * CO + m * 16 + pch);
+      if (wave == WAVES - 1) {
+#pragma unroll
+        for (int m = 0; m < CO / 16; ++m)
+          bacc[m] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], ones, bacc[m], 0, 0, 0);
+      }
+#pragma unroll
+      for (int k = 0; k < TAPS; ++k) {
+        const int t = wave + WAVES * k;
+        if (t >= 27) continue;  // uniform in the wavefront
+        const int dx = t % 3, dy = (t / 3) % 3, dzt = t / 9;
+        const int row = ((z + dzt) * CH_Y + y + dy) * CH_X + dx + prow;
+#pragma unroll
+        for (int n = 0; n < CI / 16; ++n) {
+          const bf16x4 x = read_points(xt + row * CI + n * 16 + pch);
+#pragma unroll
+          for (int m = 0; m < CO / 16; ++m)
+            acc[k][m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], x, acc[k][m][n], 0, 0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < TAPS; ++k) {
+    const int t = wave + WAVES * k;
+    if (t >= 27) continue;
+#pragma unroll
+    for (int m = 0; m < CO / 16; ++m)
+#pragma unroll
+      for (int n = 0; n < CI / 16; ++n)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          part[(((long)blockIdx.x * 27 + t) * CO + m * 16 + 4 * kg + rr) * CI + n * 16 + r] = acc[k][m][n][rr];
+  }
+  if (wave == WAVES - 1 && r == 0) {
+#pragma unroll
+    for (int m = 0; m < CO / 16; ++m)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) bpart[(long)blockIdx.x * CO + m * 16 + 4 * kg + rr] = bacc[m][rr];
+  }
+}
+
+// Sums of the work-groups' partials: dW[e] over nw weights and, in the last
+// work-group, db[e] over nb <= 64 biases.  64 entries per work-group; its 16
+// wavefronts take a sixteenth of the chunks each, several loads in flight (four
+// wavefronts with one load at a time took 17 us for 256 chunks of 27648).
+__global__ __launch_bounds__(1024) void k_sum_chunks(const float *__restrict__ part, const float *__restrict__ bpart,
+                                                     int nchunks, int nw, int nb, float *__restrict__ dW,
+                                                     float *__restrict__ db) {
+  __shared__ float red[16][64];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const bool bias = blockIdx.x == gridDim.x - 1;
+  const float *src = bias ? bpart : part;
+  const int n = bias ? nb : nw, e = bias ? l : blockIdx.x * 64 + l;
   float s = 0.f;
-  for (int c = 0; c < nchunks; ++c) s += part[c * nelem + e];
-  dW[e] = s;
+  if (e < n) {
+#pragma unroll 8
+    for (int c = w; c < nchunks; c += 16) s += src[(long)c * n + e];
+  }
+  red[w][l] = s;
+  __syncthreads();
+  if (w == 0 && e < n) {
+#pragma unroll
+    for (int k = 1; k < 16; ++k) s += red[k][l];
+    (bias ? db : dW)[e] = s;
+  }
 }
 
 // Mean-square loss over the nout real channels of out[p][16] against

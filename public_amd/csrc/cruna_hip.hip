@@ -2861,7 +2861,6 @@ struct cruna_hip_cnn {
   long cap = 0;
   bf16 *act[L] = {}, *z[L - 1] = {}, *dz_a = nullptr, *dz_b = nullptr;
   float *out32 = nullptr, *tgt = nullptr, *lpart = nullptr, *part = nullptr, *bpart = nullptr;
-  long part_cap = 0;
   CropSpec *spec = nullptr;
   long spec_cap = 0;
   std::vector<bf16 *> ds_feat;
@@ -2875,19 +2874,21 @@ static void cnn_user(cruna_hip_cnn *n, int delta) { n->users += delta; }
 
 namespace {
 
-constexpr int WGRAD_CHUNK = 8192;
-
 // launch of a convolution (k_conv_tile): persistent work-groups, as many as
 // the LDS lets reside on the MI355X's 256 CUs (160 KB each), a multiple of
 // the XCD count
 constexpr long CONV_CUS = 256, CONV_LDS_PER_CU = 163840;
+// tiles of a batch of boxes
+long conv_tiles(const ConvGeom &geo, long npts) {
+  return npts / ((long)geo.X * geo.Y * geo.Z) * ((geo.X + CT_X - 1) / CT_X) * ((geo.Y + CT_Y - 1) / CT_Y) *
+         ((geo.Z + CT_Z - 1) / CT_Z);
+}
+
 template <int CK, int CN, int MODE>
 void launch_conv(hipStream_t s, const ConvGeom &geo, long npts, const bf16 *in, const bf16 *W, const float *bias,
                  float *out32, bf16 *out16, bf16 *zsave, const bf16 *zin) {
   constexpr long lds = 27L * CN * CK * 2 + (long)CT_HALO * CK * 2;
-  const long box = (long)geo.X * geo.Y * geo.Z;
-  const long ntiles = npts / box * ((geo.X + CT_X - 1) / CT_X) * ((geo.Y + CT_Y - 1) / CT_Y) *
-                      ((geo.Z + CT_Z - 1) / CT_Z);
+  const long ntiles = conv_tiles(geo, npts);
   long G = std::min(ntiles, CONV_CUS * std::max(1L, CONV_LDS_PER_CU / lds));
   G = (G + CONV_XCDS - 1) / CONV_XCDS * CONV_XCDS;
   hipLaunchKernelGGL((k_conv_tile<CK, CN, MODE>), dim3((unsigned)G), dim3(CT_THREADS), 0, s, in, W, bias, geo, npts, out32,
@@ -2926,7 +2927,6 @@ int cnn_reserve(cruna_hip_cnn *n, long npts) {
   for (void *q : n->work) (void)hipFree(q);
   n->work.clear();
   n->cap = 0;
-  n->part_cap = 0;
   int rc = CRUNA_HIP_OK;
   for (int l = 0; l < n->L && !rc; ++l) rc = cnn_alloc(n->work, &n->act[l], npts * n->ci[l]);
   for (int l = 0; l < n->L - 1 && !rc; ++l) rc = cnn_alloc(n->work, &n->z[l], npts * n->co[l]);
@@ -2935,16 +2935,14 @@ int cnn_reserve(cruna_hip_cnn *n, long npts) {
   if (!rc) rc = cnn_alloc(n->work, &n->out32, npts * 16);
   if (!rc) rc = cnn_alloc(n->work, &n->tgt, npts * 5);
   if (!rc) rc = cnn_alloc(n->work, &n->lpart, (npts + 255) / 256);
-  const long nch = (npts + WGRAD_CHUNK - 1) / WGRAD_CHUNK;
-  if (!rc) rc = cnn_alloc(n->work, &n->part, (size_t)nch * 27 * 32 * 32);
-  if (!rc) rc = cnn_alloc(n->work, &n->bpart, (size_t)nch * 32);
+  if (!rc) rc = cnn_alloc(n->work, &n->part, (size_t)WG_MAX * 27 * 32 * 32);
+  if (!rc) rc = cnn_alloc(n->work, &n->bpart, (size_t)WG_MAX * 32);
   if (rc) {
     for (void *q : n->work) (void)hipFree(q);
     n->work.clear();
     return rc;
   }
   n->cap = npts;
-  n->part_cap = nch;
   return CRUNA_HIP_OK;
 }
 
@@ -2976,14 +2974,11 @@ int cnn_forward(cruna_hip_cnn *n, hipStream_t s, const ConvGeom &geo, long npts,
 template <int CI, int CO>
 void cnn_wgrad(cruna_hip_cnn *n, hipStream_t s, int l, const ConvGeom &geo, long npts, const bf16 *in,
                const bf16 *dz) {
-  const int nch = (int)((npts + WGRAD_CHUNK - 1) / WGRAD_CHUNK);
-  hipLaunchKernelGGL((k_conv_wgrad<CI, CO>), dim3(nch, 27), dim3(256), 0, s, in, dz, geo, npts, WGRAD_CHUNK,
-                     n->part, n->bpart);
-  const long e = 27L * CO * CI;
-  hipLaunchKernelGGL(k_sum_chunks, dim3((e + 255) / 256), dim3(256), 0, s, (const float *)n->part, nch, e,
-                     n->grads + n->woff[l]);
-  hipLaunchKernelGGL(k_sum_chunks, dim3(1), dim3(256), 0, s, (const float *)n->bpart, nch, (long)CO,
-                     n->grads + n->boff[l]);
+  const int nch = (int)std::min<long>(WG_MAX, conv_tiles(geo, npts));
+  hipLaunchKernelGGL((k_conv_wgrad<CI, CO>), dim3(nch), dim3(CT_THREADS), 0, s, in, dz, geo, npts, n->part, n->bpart);
+  constexpr int e = 27 * CO * CI;
+  hipLaunchKernelGGL(k_sum_chunks, dim3((e + 63) / 64 + 1), dim3(1024), 0, s, (const float *)n->part,
+                     (const float *)n->bpart, nch, e, CO, n->grads + n->woff[l], n->grads + n->boff[l]);
 }
 
 // loss over the points at least `halo` from their box's faces (count of
