@@ -24,12 +24,11 @@ typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// float -> bf16, round to nearest even (NaN stays NaN)
-__device__ __forceinline__ bf16 to_bf16(float f) {
-  unsigned u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return (bf16)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (bf16)(u >> 16);
+// float -> bf16, round to nearest even (NaN stays NaN): the hardware's conversion
+__device__ __forceinline__ bf16 to_bf16(float f) { return __builtin_bit_cast(bf16, (__bf16)f); }
+__device__ __forceinline__ uint2 to_bf16(f32x4 v) {
+  typedef __bf16 half4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(uint2, __builtin_convertvector(v, half4));
 }
 __device__ __forceinline__ float from_bf16(bf16 h) { return __uint_as_float((unsigned)h << 16); }
 
@@ -121,22 +120,6 @@ __global__ __launch_bounds__(CT_THREADS) void k_conv_tile(const bf16 *__restrict
   // covers one contiguous run of LDS, free of bank conflicts
   __shared__ __align__(16) bf16 wl[27 * CN * CK];
   __shared__ __align__(16) bf16 xt[CT_HALO * CK];
-  {
-    constexpr int PIECES = 27 * CN * CK / 8, BATCH = 4;
-    for (int base = 0; base < PIECES; base += CT_THREADS * BATCH) {
-      uint4 v[BATCH];
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        const int e = base + threadIdx.x + CT_THREADS * u;
-        v[u] = e < PIECES ? *reinterpret_cast<const uint4 *>(W + (long)e * 8) : uint4{0u, 0u, 0u, 0u};
-      }
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        const int e = base + threadIdx.x + CT_THREADS * u;
-        if (e < PIECES) *reinterpret_cast<uint4 *>(wl + (long)e * 8) = v[u];
-      }
-    }
-  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, kg = lane >> 4;
   const bool per = geo.periodic != 0;
@@ -188,7 +171,26 @@ __global__ __launch_bounds__(CT_THREADS) void k_conv_tile(const bf16 *__restrict
       if (e < PIECES) *reinterpret_cast<uint4 *>(buf + (long)e * 8) = pre[u];
     }
   };
-  if (t0 < t1) fetch(t0);
+  {
+    // the layer's weights, every load in flight together with the first tile's
+    constexpr int WPIECES = 27 * CN * CK / 8, WPER = (WPIECES + CT_THREADS - 1) / CT_THREADS;
+    uint4 v[WPER];
+#pragma unroll
+    for (int u = 0; u < WPER; ++u) {
+      const int e = threadIdx.x + CT_THREADS * u;
+      v[u] = e < WPIECES ? *reinterpret_cast<const uint4 *>(W + (long)e * 8) : uint4{0u, 0u, 0u, 0u};
+    }
+    if (t0 < t1) fetch(t0);
+#pragma unroll
+    for (int u = 0; u < WPER; ++u) {
+      const int e = threadIdx.x + CT_THREADS * u;
+      if (e < WPIECES) *reinterpret_cast<uint4 *>(wl + (long)e * 8) = v[u];
+    }
+  }
+  f32x4 b4[CN / 16];
+#pragma unroll
+  for (int n = 0; n < CN / 16; ++n)
+    b4[n] = MODE == CONV_BACKWARD ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4 *>(bias + n * 16 + 4 * kg);
   for (int tile = t0; tile < t1; ++tile) {
     __syncthreads();  // the previous tile's reads of xt are done
     put(xt);
@@ -224,7 +226,7 @@ __global__ __launch_bounds__(CT_THREADS) void k_conv_tile(const bf16 *__restrict
                   bf16x8, *reinterpret_cast<const uint4 *>(wl + (t * CN + n * 16 + r) * CK + kg * 8));
 #pragma unroll
               for (int j = 0; j < CONV_TILES; ++j)
-                acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[j]), w, acc[j][n],
+                acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(bf16x8, a[j]), acc[j][n],
                                                                     0, 0, 0);
             }
           } else {
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(CT_THREADS) void k_conv_tile(const bf16 *__restrict
               const bf16x4 w = *reinterpret_cast<const bf16x4 *>(wl + (t * CN + n * 16 + r) * CK + kg * 4);
 #pragma unroll
               for (int j = 0; j < CONV_TILES; ++j)
-                acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[j], w, acc[j][n], 0, 0, 0);
+                acc[j][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w, a[j], acc[j][n], 0, 0, 0);
             }
           }
         }
@@ -246,27 +248,31 @@ __global__ __launch_bounds__(CT_THREADS) void k_conv_tile(const bf16 *__restrict
     const int i0 = (rem % nbx) * CT_X, j0 = ((rem / nbx) % nby) * CT_Y, k0 = (rem / (nbx * nby)) * CT_Z;
     const long base = (long)b * XYZ;
     const int kk = k0 + wave;
+    // a lane holds 4 consecutive channels of one point (channels are the matrix
+    // rows): stores of 8 and 16 bytes
+    const int ii = i0 + r;
+    const bool inside = ii < X && kk < Z;
 #pragma unroll
     for (int j = 0; j < CONV_TILES; ++j) {
       const int jj = j0 + j;
-      if (jj >= Y || kk >= Z) continue;
+      if (!inside || jj >= Y) continue;
+      const long o0 = (base + ii + X * ((long)jj + (long)Y * kk)) * CN + 4 * kg;
 #pragma unroll
       for (int n = 0; n < CN / 16; ++n) {
-        const int ch = n * 16 + r;
+        const long o = o0 + n * 16;
+        if (MODE == CONV_GELU) {
+          const f32x4 z = acc[j][n] + b4[n];
+          if (zsave) *reinterpret_cast<uint2 *>(zsave + o) = to_bf16(z);
+          *reinterpret_cast<uint2 *>(out16 + o) = to_bf16(f32x4{gelu(z[0]), gelu(z[1]), gelu(z[2]), gelu(z[3])});
+        } else if (MODE == CONV_LINEAR) {
+          *reinterpret_cast<f32x4 *>(out32 + o) = acc[j][n] + b4[n];
+        } else {
+          const uint2 h = *reinterpret_cast<const uint2 *>(zin + o);
+          f32x4 d;
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int ii = i0 + 4 * kg + rr;
-          if (ii >= X) continue;
-          const long o = (base + ii + X * ((long)jj + (long)Y * kk)) * CN + ch;
-          if (MODE == CONV_GELU) {
-            const float z = acc[j][n][rr] + bias[ch];
-            if (zsave) zsave[o] = to_bf16(z);
-            out16[o] = to_bf16(gelu(z));
-          } else if (MODE == CONV_LINEAR) {
-            out32[o] = acc[j][n][rr] + bias[ch];
-          } else {
-            out16[o] = to_bf16(acc[j][n][rr] * gelu_grad(from_bf16(zin[o])));
-          }
+          for (int rr = 0; rr < 4; ++rr)
+            d[rr] = acc[j][n][rr] * gelu_grad(__uint_as_float(rr % 2 ? (rr / 2 ? h.y : h.x) & 0xffff0000u : (rr / 2 ? h.y : h.x) << 16));
+          *reinterpret_cast<uint2 *>(out16 + o) = to_bf16(d);
         }
       }
     }
