@@ -432,12 +432,12 @@ __global__ __launch_bounds__(1024) void k_sum_chunks(const float *__restrict__ p
   }
 }
 
-// Mean-square loss over the nout real channels of out[p][16] against
+// Mean-square loss over the 5 real channels of out[p][16] against
 // target[c][p], counting only the points at least `halo` away from their
 // box's faces (all points for halo 0); dout[p][16] <- bf16(2 (out - target)
 // / count) (zero elsewhere), partial loss sums per block into lpart.
 __global__ __launch_bounds__(256) void k_mse(const float *__restrict__ out, const float *__restrict__ target,
-                                             long npts, int nout, ConvGeom geo, int halo, float scale,
+                                             long npts, ConvGeom geo, int halo, float scale,
                                              bf16 *__restrict__ dout, float *__restrict__ lpart) {
   __shared__ float red[256];
   const long p = (long)blockIdx.x * 256 + threadIdx.x;
@@ -449,15 +449,20 @@ __global__ __launch_bounds__(256) void k_mse(const float *__restrict__ out, cons
       in = cc.i >= halo && cc.i < geo.X - halo && cc.j >= halo && cc.j < geo.Y - halo && cc.k >= halo &&
            cc.k < geo.Z - halo;
     }
-    for (int c = 0; c < 16; ++c) {
-      float g = 0.f;
-      if (c < nout && in) {
-        const float d = out[p * 16 + c] - target[c * npts + p];
+    const f32x4 o = *reinterpret_cast<const f32x4 *>(out + p * 16);
+    const float o4 = out[p * 16 + 4];
+    float g[8] = {};
+#pragma unroll
+    for (int c = 0; c < 5; ++c)
+      if (in) {
+        const float d = (c < 4 ? o[c & 3] : o4) - target[c * npts + p];
         s += d * d;
-        g = scale * d;
+        g[c] = scale * d;
       }
-      dout[p * 16 + c] = to_bf16(g);
-    }
+    const uint2 lo = to_bf16(f32x4{g[0], g[1], g[2], g[3]}), hi = to_bf16(f32x4{g[4], g[5], g[6], g[7]});
+    uint4 *w = reinterpret_cast<uint4 *>(dout + p * 16);
+    w[0] = uint4{lo.x, lo.y, hi.x, hi.y};
+    w[1] = uint4{0u, 0u, 0u, 0u};
   }
   red[threadIdx.x] = s;
   __syncthreads();
@@ -525,40 +530,64 @@ __global__ void k_pack_weights(const float *__restrict__ w, int CO, int CI, bf16
 }
 
 // Means of the 5 fields of a state, in a fixed summation order: partial
-// sums of MEAN_BLOCKS grid-strided work-groups, then one work-group adds
-// them.  The network sees every sample relative to its own means.
+// sums of MEAN_BLOCKS grid-strided work-groups per field; the kernels that
+// use the means add these up themselves (a launch less, 6 us; reading 10 KB of
+// partial sums in every work-group costs 2).  The network sees every sample
+// relative to its own means.
 constexpr int MEAN_BLOCKS = 256;
+
+// Sums over the work-group's 256 threads, as a tree (t takes t + 128, then t + 64, ...):
+// valid in thread 0
+template <int NF>
+__device__ __forceinline__ void block_sums(double (&s)[NF], double (&red)[NF][128]) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int w = 128; w >= 64; w >>= 1) {
+    __syncthreads();
+    if (t >= w && t < 2 * w) {
+#pragma unroll
+      for (int c = 0; c < NF; ++c) red[c][t - w] = s[c];
+    }
+    __syncthreads();
+    if (t < w) {
+#pragma unroll
+      for (int c = 0; c < NF; ++c) s[c] += red[c][t];
+    }
+  }
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1)
+#pragma unroll
+    for (int c = 0; c < NF; ++c) s[c] += __shfl_down(s[c], w);
+}
+
+// The means of the first NF fields from their partial sums, in every thread
+template <int NF>
+__device__ __forceinline__ void field_means(const double *__restrict__ part, long N, double (&mean)[NF]) {
+  __shared__ double red[NF][128];
+#pragma unroll
+  for (int c = 0; c < NF; ++c) mean[c] = part[c * MEAN_BLOCKS + threadIdx.x];
+  block_sums(mean, red);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int c = 0; c < NF; ++c) red[c][0] = mean[c] / (double)N;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < NF; ++c) mean[c] = red[c][0];
+}
+
+// work-group (b, c): partial sum b of field c
 template <typename Q>
 __global__ __launch_bounds__(256) void k_field_partials(const Q *__restrict__ q, long N,
                                                         double *__restrict__ part) {
-  __shared__ double red[256];
-  for (int c = 0; c < 5; ++c) {
-    double s = 0.0;
-    for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < N; p += (long)gridDim.x * 256) s += (double)q[c * N + p];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) part[c * gridDim.x + blockIdx.x] = red[0];
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(256) void k_field_means(const double *__restrict__ part, int nparts, long N,
-                                                     double *__restrict__ mean) {
-  __shared__ double red[256];
-  for (int c = 0; c < 5; ++c) {
-    red[threadIdx.x] = (int)threadIdx.x < nparts ? part[c * nparts + threadIdx.x] : 0.0;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) mean[c] = red[0] / (double)N;
-    __syncthreads();
-  }
+  __shared__ double red[1][128];
+  q += blockIdx.y * N;
+  double s[1] = {0.0};
+#pragma unroll 4
+  for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < N; p += MEAN_BLOCKS * 256) s[0] += (double)q[p];
+  block_sums(s, red);
+  if (threadIdx.x == 0) part[blockIdx.y * MEAN_BLOCKS + blockIdx.x] = s[0];
 }
 
 // Normalisation of a closure network (device copy, set by the host).
@@ -575,18 +604,31 @@ __device__ __forceinline__ float pressure_scale(const CnnNorm &nm, const double 
   return nm.p_ref > 0.0 ? (float)(mean[4] / nm.p_ref) : 1.f;
 }
 
-// Network input from a state q (5 fields of N points, field-major): channel c
-// of point p = bf16(f32(q[c][p] - mean[c]) inv_std[c]), channels 5..15 zero.
+// Network input from a state q (5 fields of N points, field-major, with their
+// partial sums): channel c of point p = bf16(f32(q[c][p] - mean[c])
+// inv_std[c]), channels 5..15 zero; mean[0..4] set.
 template <typename Q>
-__global__ void k_pack_features(const Q *__restrict__ q, long N, const double *__restrict__ mean,
-                                const CnnNorm *__restrict__ nm, bf16 *__restrict__ feat) {
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_pack_features(const Q *__restrict__ q, long N, const double *__restrict__ part,
+                                                       const CnnNorm *__restrict__ nm, double *__restrict__ mean,
+                                                       bf16 *__restrict__ feat) {
+  const long p = (long)blockIdx.x * 256 + threadIdx.x;
+  Q v[5] = {};
+  if (p < N) {
+#pragma unroll
+    for (int c = 0; c < 5; ++c) v[c] = q[c * N + p];
+  }
+  double m[5];
+  field_means(part, N, m);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+#pragma unroll
+    for (int c = 0; c < 5; ++c) mean[c] = m[c];
+  }
   if (p >= N) return;
   unsigned h[3];
 #pragma unroll
   for (int c = 0; c < 6; c += 2) {
-    const unsigned lo = to_bf16((float)((double)q[c * N + p] - mean[c]) * nm->inv_std[c]);
-    const unsigned hi = c + 1 < 5 ? to_bf16((float)((double)q[(c + 1) * N + p] - mean[c + 1]) * nm->inv_std[c + 1]) : 0u;
+    const unsigned lo = to_bf16((float)((double)v[c] - m[c]) * nm->inv_std[c]);
+    const unsigned hi = c + 1 < 5 ? to_bf16((float)((double)v[c + 1] - m[c + 1]) * nm->inv_std[c + 1]) : 0u;
     h[c / 2] = lo | (hi << 16);
   }
   uint4 *d = reinterpret_cast<uint4 *>(feat + p * 16);
@@ -594,17 +636,37 @@ __global__ void k_pack_features(const Q *__restrict__ q, long N, const double *_
   d[1] = uint4{0u, 0u, 0u, 0u};
 }
 
-// Closure term in the solver's layout: force[v][p] = out[p][v] out_std[v] (x pressure scale) x gain[v]
+// Closure term in the solver's layout: force[v][p] = out[p][v] out_std[v] (x pressure scale) x gain[v],
+// and the partial sums of its first 4 fields
 template <typename T>
-__global__ void k_unpack_closure(const float *__restrict__ out, long N, const CnnNorm *__restrict__ nm,
-                                 const double *__restrict__ mean, T *__restrict__ force) {
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= N) return;
+__global__ __launch_bounds__(256) void k_unpack_closure(const float *__restrict__ out, long N,
+                                                        const CnnNorm *__restrict__ nm,
+                                                        const double *__restrict__ mean, T *__restrict__ force,
+                                                        double *__restrict__ part) {
+  __shared__ double red[4][128];
   const float ps = pressure_scale(*nm, mean);
+  float scale[5], gain[5];
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
-    const float s = v == 4 ? nm->out_std[4] * ps : nm->out_std[v];
-    force[v * N + p] = T(out[p * 16 + v] * s * nm->gain[v]);
+    scale[v] = v == 4 ? nm->out_std[4] * ps : nm->out_std[v];
+    gain[v] = nm->gain[v];
+  }
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < N; p += MEAN_BLOCKS * 256) {
+    const f32x4 o = *reinterpret_cast<const f32x4 *>(out + p * 16);
+    const float o4 = out[p * 16 + 4];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      const T f = T((v < 4 ? o[v & 3] : o4) * scale[v] * gain[v]);
+      force[v * N + p] = f;
+      if (v < 4) s[v & 3] += (double)f;
+    }
+  }
+  block_sums(s, red);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) part[v * MEAN_BLOCKS + blockIdx.x] = s[v];
   }
 }
 
@@ -612,11 +674,18 @@ __global__ void k_unpack_closure(const float *__restrict__ out, long N, const Cn
 // rho u, rho v, rho w): a subfilter term of a conservation law is the
 // divergence of a subfilter flux and adds nothing to the domain total.
 template <typename T>
-__global__ void k_remove_mean(T *__restrict__ force, long N, const double *__restrict__ mean) {
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_remove_mean(T *__restrict__ force, long N, const double *__restrict__ part) {
+  const long p = (long)blockIdx.x * 256 + threadIdx.x;
+  T f[4] = {};
+  if (p < N) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) f[v] = force[v * N + p];
+  }
+  double m[4];
+  field_means(part, N, m);
   if (p >= N) return;
 #pragma unroll
-  for (int v = 0; v < 4; ++v) force[v * N + p] = force[v * N + p] - T(mean[v]);
+  for (int v = 0; v < 4; ++v) force[v * N + p] = f[v] - T(m[v]);
 }
 
 // Normalised targets: tn[c][p] = target[c][p] out_inv_std[c] (/ pressure scale)

@@ -2989,7 +2989,7 @@ int cnn_backward(cruna_hip_cnn *n, hipStream_t s, const ConvGeom &geo, long npts
   const int nb = (int)((npts + 255) / 256);
   const float scale = (float)(2.0 / ((double)counted * 5));
   hipLaunchKernelGGL(k_mse, dim3(nb), dim3(256), 0, s, (const float *)n->out32, (const float *)n->tgt, npts,
-                     5, geo, halo, scale, n->dz_a, n->lpart);
+                     geo, halo, scale, n->dz_a, n->lpart);
   // layer 3 (32 -> 16, linear)
   cnn_wgrad<32, 16>(n, s, 3, geo, npts, n->act[3], n->dz_a);
   launch_conv<16, 32, CONV_BACKWARD>(s, geo, npts, n->dz_a, n->wt + n->wpk[3], nullptr, nullptr, n->dz_b, nullptr,
@@ -3016,27 +3016,28 @@ int cnn_backward(cruna_hip_cnn *n, hipStream_t s, const ConvGeom &geo, long npts
   return CRUNA_HIP_OK;
 }
 
+// the features of a state (device, 5 fields of S^3) in act[0], its field means in fmean
+template <typename Q>
+void cnn_features(cruna_hip_cnn *n, hipStream_t s, const Q *q) {
+  double *part = n->fmean + 8;
+  hipLaunchKernelGGL((k_field_partials<Q>), dim3(MEAN_BLOCKS, 5), dim3(256), 0, s, q, n->N, part);
+  hipLaunchKernelGGL((k_pack_features<Q>), dim3((unsigned)((n->N + 255) / 256)), dim3(256), 0, s, q, n->N,
+                     (const double *)part, (const CnnNorm *)n->dn, n->fmean, n->act[0]);
+}
+
 // closure evaluation on stream s: features of the state q (device, 5
 // fields of S^3), forward, force (5 fields of T) when `force` is set
 template <typename T, typename Q>
 int closure_eval(cruna_hip_cnn *n, hipStream_t s, const Q *q, T *force) {
   const unsigned nb = (unsigned)((n->N + 255) / 256);
-  hipLaunchKernelGGL((k_field_partials<Q>), dim3(MEAN_BLOCKS), dim3(256), 0, s, q, n->N, n->fmean + 8);
-  hipLaunchKernelGGL(k_field_means, dim3(1), dim3(256), 0, s, (const double *)(n->fmean + 8), MEAN_BLOCKS, n->N,
-                     n->fmean);
-  hipLaunchKernelGGL((k_pack_features<Q>), dim3(nb), dim3(256), 0, s, q, n->N, (const double *)n->fmean,
-                     (const CnnNorm *)n->dn, n->act[0]);
+  cnn_features(n, s, q);
   if (int rc = check_launch()) return rc;
   if (int rc = cnn_forward(n, s, conv_geom(n->S, n->S, n->S, true), n->N, false)) return rc;
   if (force) {
-    hipLaunchKernelGGL((k_unpack_closure<T>), dim3(nb), dim3(256), 0, s, (const float *)n->out32, n->N,
-                       (const CnnNorm *)n->dn, (const double *)n->fmean, force);
-    // domain means of the force (after the state's means are consumed)
-    hipLaunchKernelGGL((k_field_partials<T>), dim3(MEAN_BLOCKS), dim3(256), 0, s, (const T *)force, n->N,
-                       n->fmean + 8);
-    hipLaunchKernelGGL(k_field_means, dim3(1), dim3(256), 0, s, (const double *)(n->fmean + 8), MEAN_BLOCKS, n->N,
-                       n->fmean);
-    hipLaunchKernelGGL((k_remove_mean<T>), dim3(nb), dim3(256), 0, s, force, n->N, (const double *)n->fmean);
+    hipLaunchKernelGGL((k_unpack_closure<T>), dim3(MEAN_BLOCKS), dim3(256), 0, s, (const float *)n->out32, n->N,
+                       (const CnnNorm *)n->dn, (const double *)n->fmean, force, n->fmean + 8);
+    // without the domain means of the force
+    hipLaunchKernelGGL((k_remove_mean<T>), dim3(nb), dim3(256), 0, s, force, n->N, (const double *)(n->fmean + 8));
   }
   return check_launch();
 }
@@ -3065,12 +3066,7 @@ int cnn_stage(cruna_hip_cnn *n, const double *q, const double *target, StageWhat
   if (what == STAGE_FORCE) {
     if (int rc = closure_eval<double, double>(n, n->stream, qd, td)) return rc;
   } else {
-    hipLaunchKernelGGL((k_field_partials<double>), dim3(MEAN_BLOCKS), dim3(256), 0, n->stream, (const double *)qd,
-                       n->N, n->fmean + 8);
-    hipLaunchKernelGGL(k_field_means, dim3(1), dim3(256), 0, n->stream, (const double *)(n->fmean + 8), MEAN_BLOCKS,
-                       n->N, n->fmean);
-    hipLaunchKernelGGL((k_pack_features<double>), dim3(nb), dim3(256), 0, n->stream, (const double *)qd, n->N,
-                       (const double *)n->fmean, (const CnnNorm *)n->dn, n->act[0]);
+    cnn_features(n, n->stream, (const double *)qd);
     if (int rc = check_launch()) return rc;
     if (what == STAGE_TRAIN)
       if (int rc = cnn_forward(n, n->stream, conv_geom(n->S, n->S, n->S, true), n->N, true)) return rc;
