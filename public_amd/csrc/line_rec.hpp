@@ -59,6 +59,7 @@ constexpr double REC_MAX_LAMBDA = 0.9;
 constexpr int REC_END = PPT * FE + 2 * PPT;
 constexpr int REC_SCAL = 2 * REC_END;
 constexpr int REC_PW = REC_SCAL + 6;
+constexpr int REC_ROWS = 4;  // most rows of its own in an end block
 
 struct RecOp {
   double s[4];     // stencil c0..c3 (scaled)
@@ -74,6 +75,8 @@ struct RecOp {
   int srow[2];     // bit r: row r of the first / last block has its own explicit row
   int zrow[2];     // bit r: row r of the first / last block is padding
   int rend[2];     // row of the first / last real point in its block
+  int rows[2];     // srow as a list: row k in bits 4k..4k+3, 15 for none
+  int nrow;        // the longer list's length (at most REC_ROWS)
 };
 
 struct HostRecOp {
@@ -151,6 +154,16 @@ inline HostRecOp build_rec_op(OpKind kind, bool per, int n_real, double alpha) {
       if (j < HALO - reach || j >= HALO + PPT + reach) throw std::runtime_error("closure row wider than the halo");
       h.tab[e * REC_END + (p % PPT) * FE + j] += (double)(sc * jc.second);
     }
+  }
+  for (int e = 0; e < 2; ++e) {
+    int k = 0;
+    op.rows[e] = (1 << 4 * REC_ROWS) - 1;
+    for (int r = 0; r < PPT; ++r)
+      if ((op.srow[e] >> r) & 1) {
+        if (k == REC_ROWS) throw std::runtime_error("too many closure rows in a block");
+        op.rows[e] ^= (15 ^ r) << 4 * k++;
+      }
+    op.nrow = std::max(op.nrow, k);
   }
   for (int r = 0; r < PPT; ++r) {
     if (r < pf) op.zrow[0] |= 1 << r;

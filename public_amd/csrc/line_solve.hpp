@@ -332,9 +332,10 @@ __device__ __forceinline__ void line_solve(const LineOp<T> &op, LineLds<T, NTM> 
 // immediate offset away.  Dynamic LDS, so that a work-group takes what its own
 // size needs.
 constexpr int REC_STRIDE = 13, REC_HALO = 8, REC_UL = 8, REC_XF = 10;
+constexpr int REC_TEND = REC_ROWS * FE + 2 * PPT, REC_TSCAL = 2 * REC_TEND, REC_TAB = REC_TSCAL + 6;
 // (a multiple of 16: what follows is accessed in 16-byte pieces)
 __host__ __device__ inline size_t rec_lds_bytes(int threads) {
-  return ((size_t)(threads + 1) * REC_STRIDE * sizeof(double) + 15) / 16 * 16;
+  return ((size_t)((threads + 1) * REC_STRIDE + REC_TAB) * sizeof(double) + 15) / 16 * 16;
 }
 
 template <typename T>
@@ -380,6 +381,10 @@ struct RecLines {
   int nthreads;
   bool wave_line;
   double pwl, pwr;             // open: mu^(8 b - pf), mu^(n-1 - (8 b - pf) - 7)
+  static constexpr int TAB_REGS = 1;
+  double tv[TAB_REGS];         // open: entries of the closure table on their way to LDS
+  bool pending = false;
+  int keep[PPT];               // open: 0 for the thread's padding points, else all bits
 
   static constexpr int SLOT = REC_STRIDE * int(sizeof(double));
   __device__ __forceinline__ double get(int slot, int cell) const {
@@ -418,15 +423,61 @@ struct RecLines {
     if (!PER) {
       for (int t = threadIdx.x; t < REC_STRIDE; t += nthreads)
         *reinterpret_cast<double *>(lds + zero + t * int(sizeof(double))) = 0.0;
-      lds_barrier();
       bind(op);
     }
   }
-  // the powers of mu of an open line's op (the constructor binds its own)
+  // the closure table and powers of mu of an open line's op (the constructor
+  // binds its own): loads issued here, stored to LDS by the next solve
   __device__ __forceinline__ void bind(const RecOp &op) {
     if (!PER) {
       pwl = op.tab[REC_PW + 2 * b];
       pwr = op.tab[REC_PW + 2 * b + 1];
+      const int pad = (b == 0 ? op.zrow[0] : 0) | (b == NB - 1 ? op.zrow[1] : 0);
+#pragma unroll
+      for (int r = 0; r < PPT; ++r) keep[r] = ((pad >> r) & 1) - 1;
+#pragma unroll
+      for (int k = 0; k < TAB_REGS; ++k) {
+        const int t = int(threadIdx.x) + k * nthreads;
+        tv[k] = t < REC_TAB ? table_entry(op, t) : 0.0;
+      }
+      pending = true;
+    }
+  }
+  // entry t of the closure table
+  static __device__ __forceinline__ double table_entry(const RecOp &op, int t) {
+    if (t >= REC_TSCAL) return op.tab[REC_SCAL + t - REC_TSCAL];
+    const int e = t >= REC_TEND ? 1 : 0, o = t - e * REC_TEND;
+    if (o >= REC_ROWS * FE) return op.tab[e * REC_END + PPT * FE + o - REC_ROWS * FE];
+    const int r = (op.rows[e] >> (4 * (o / FE))) & 15;
+    return r < PPT ? op.tab[e * REC_END + r * FE + o % FE] : 0.0;
+  }
+  __device__ __forceinline__ void store_table(const RecOp &op) {
+    lds_barrier();  // the last op's table has been read
+    double *tab = reinterpret_cast<double *>(lds + (nthreads + 1) * SLOT);
+#pragma unroll
+    for (int k = 0; k < TAB_REGS; ++k) {
+      const int t = int(threadIdx.x) + k * nthreads;
+      if (t < REC_TAB) tab[t] = tv[k];
+    }
+    for (int t = int(threadIdx.x) + TAB_REGS * nthreads; t < REC_TAB; t += nthreads) tab[t] = table_entry(op, t);
+    lds_barrier();
+    pending = false;
+  }
+  // the table of the thread's end of the line (any for the blocks between)
+  __device__ __forceinline__ const double *end_table() const {
+    return reinterpret_cast<const double *>(lds + (nthreads + 1) * SLOT) + (b == 0 ? 0 : REC_TEND);
+  }
+  // x where the thread's point is real, else y: two AND / BFI per value with
+  // the masks kept per thread (compares and selects took four times the code)
+  __device__ __forceinline__ double real_or(int r, double x, double y) const {
+    const int2 a = __builtin_bit_cast(int2, x), c = __builtin_bit_cast(int2, y);
+    return __builtin_bit_cast(double, int2{(a.x & keep[r]) | (c.x & ~keep[r]), (a.y & keep[r]) | (c.y & ~keep[r])});
+  }
+  __device__ __forceinline__ void zero_padding(double (&x)[PPT]) const {
+#pragma unroll
+    for (int r = 0; r < PPT; ++r) {
+      const int2 a = __builtin_bit_cast(int2, x[r]);
+      x[r] = __builtin_bit_cast(double, int2{a.x & keep[r], a.y & keep[r]});
     }
   }
   __device__ __forceinline__ void sync() const { line_sync(wave_line); }
@@ -466,6 +517,9 @@ struct RecLines {
 #pragma clang fp contract(off)
     constexpr int H = FILT ? 3 : 2, CELL = 2 * H;
     static_assert(NF * CELL <= REC_HALO && NF <= 2, "the fields' halo cells");
+    if (!PER && pending) store_table(op);
+    const bool end = !PER && (b == 0 || b == NB - 1);
+    const bool padded = !PER && (op.zrow[0] | op.zrow[1]) != 0;
 #pragma unroll
     for (int v = 0; v < NF; ++v)
 #pragma unroll
@@ -495,22 +549,19 @@ struct RecLines {
       }
       if (!PER) {
         // the closures' own rows and the padding of the two end blocks
+        if (__builtin_amdgcn_ballot_w64(end) != 0) {
+          const double *tab = end_table() + HALO - H;
+          const int rows = b == 0 ? op.rows[0] : op.rows[1];
+#pragma unroll 1
+          for (int k = 0; k < op.nrow; ++k) {
+            double acc = 0.0;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const bool mine = b == (e == 0 ? 0 : NB - 1);
-          if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
+            for (int j = 0; j < PPT + 2 * H; ++j) acc = __builtin_fma(tab[k * FE + j], fe[j], acc);
+            const int r = end ? (rows >> (4 * k)) & 15 : 15;
 #pragma unroll
-          for (int r = 0; r < PPT; ++r) {
-            if ((op.srow[e] >> r) & 1) {
-              const cptr<double> a = launder_uniform(op.tab + e * REC_END + r * FE + HALO - H);
-              double acc = 0.0;
-#pragma unroll
-              for (int j = 0; j < PPT + 2 * H; ++j) acc = __builtin_fma(a[j], fe[j], acc);
-              if (mine) x[v][r] = acc;
-            } else if ((op.zrow[e] >> r) & 1) {
-              if (mine) x[v][r] = 0.0;
-            }
+            for (int q = 0; q < PPT; ++q) x[v][q] = q == r ? acc : x[v][q];
           }
+          if (padded) zero_padding(x[v]);
         }
       }
 #pragma unroll
@@ -523,13 +574,8 @@ struct RecLines {
       const double U = window<FILT>(op, lf, -1, REC_UL + v);
 #pragma unroll
       for (int i = 0; i < PPT; ++i) x[v][i] = __builtin_fma(op.lp[i], U, x[v][i]);
-      if (!PER && op.zrow[1] != 0) {  // nothing comes back from behind the last point
-        const bool mine = b == NB - 1;
-        if (__builtin_amdgcn_ballot_w64(mine) != 0)
-#pragma unroll
-          for (int r = 0; r < PPT; ++r)
-            if (((op.zrow[1] >> r) & 1) && mine) x[v][r] = 0.0;
-      }
+      // nothing comes back from behind the last point
+      if (padded && __builtin_amdgcn_ballot_w64(end) != 0) zero_padding(x[v]);
 #pragma unroll
       for (int i = PPT - 2; i >= 0; --i) x[v][i] = __builtin_fma(op.mu, x[v][i + 1], x[v][i]);
       put(REC_XF + v, x[v][0]);
@@ -541,22 +587,21 @@ struct RecLines {
 #pragma unroll
       for (int i = 0; i < PPT; ++i) x[v][i] = __builtin_fma(op.lp[PPT - 1 - i], X, x[v][i]);
     }
-    if (!PER) ends<NF, FILT>(op, f, x);
+    if (!PER) ends<NF, FILT>(op, f, x, end, padded);
   }
 
   // end corrections of an open line, then the padding rows
   template <int NF, bool FILT>
-  __device__ __forceinline__ void ends(const RecOp &op, const double (&f)[NF][PPT], double (&x)[NF][PPT]) {
+  __device__ __forceinline__ void ends(const RecOp &op, const double (&f)[NF][PPT], double (&x)[NF][PPT], bool end,
+                                       bool padded) {
 #pragma clang fp contract(off)
-        const bool end[2] = {b == 0, b == NB - 1};
+    const bool any = __builtin_amdgcn_ballot_w64(end) != 0;
     if (op.nend) {
       double kap[NF];
 #pragma unroll
       for (int v = 0; v < NF; ++v) kap[v] = 0.0;
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        if (__builtin_amdgcn_ballot_w64(end[e]) == 0) continue;
-        const cptr<double> c = launder_uniform(op.tab + e * REC_END + PPT * FE);
+      if (any) {
+        const double *c = end_table() + REC_ROWS * FE;
 #pragma unroll
         for (int v = 0; v < NF; ++v) {
           double a = 0.0, k = 0.0;
@@ -565,7 +610,7 @@ struct RecLines {
             a = __builtin_fma(c[r], x[v][r], a);
             k = __builtin_fma(c[PPT + r], x[v][r], k);
           }
-          if (end[e]) {
+          if (end) {
             put(REC_UL + v, a);  // u_L has been read (the exchange of x_F lies between)
             kap[v] = k;
           }
@@ -573,7 +618,9 @@ struct RecLines {
       }
       sync();
       if (__builtin_amdgcn_ballot_w64(fabs(pwl) > 1e-19 || fabs(pwr) > 1e-19) != 0) {
-        const cptr<double> t = launder_uniform(op.tab + REC_SCAL);
+        const double *t = reinterpret_cast<const double *>(lds + (nthreads + 1) * SLOT) + REC_TSCAL;
+        const double gam = b == 0 ? t[4] : t[5];
+        const int re = end ? (b == 0 ? op.rend[0] : op.rend[1]) : PPT;
 #pragma unroll
         for (int v = 0; v < NF; ++v) {
           const double al = get(line * SLOT, REC_UL + v), ar = get(slot_of(NB - 1), REC_UL + v);
@@ -586,21 +633,24 @@ struct RecLines {
             x[v][i] = __builtin_fma(op.lp[i - 1], l, x[v][i]);
             x[v][PPT - 1 - i] = __builtin_fma(op.lp[i - 1], r, x[v][PPT - 1 - i]);
           }
-          const double k = __builtin_fma(end[0] ? t[4] : t[5], end[0] ? sr : sl, kap[v]);
+          if (any) {
+            const double k = __builtin_fma(gam, b == 0 ? sr : sl, kap[v]);
 #pragma unroll
-          for (int r2 = 0; r2 < PPT; ++r2) {
-            if (r2 == op.rend[0] && end[0]) x[v][r2] += k;
-            if (r2 == op.rend[1] && end[1]) x[v][r2] += k;
+            for (int q = 0; q < PPT; ++q) x[v][q] = q == re ? x[v][q] + k : x[v][q];
           }
         }
       }
     }
-    if ((op.zrow[0] | op.zrow[1]) != 0) {
+    if (padded && any) {
 #pragma unroll
-      for (int v = 0; v < NF; ++v)
+      for (int v = 0; v < NF; ++v) {
+        if (FILT) {
 #pragma unroll
-        for (int r = 0; r < PPT; ++r)
-          if ((((op.zrow[0] >> r) & 1) && end[0]) || (((op.zrow[1] >> r) & 1) && end[1])) x[v][r] = FILT ? f[v][r] : 0.0;
+          for (int r = 0; r < PPT; ++r) x[v][r] = real_or(r, x[v][r], f[v][r]);
+        } else {
+          zero_padding(x[v]);
+        }
+      }
     }
   }
 
