@@ -1571,7 +1571,7 @@ int cruna_hip_set_qref(cruna_hip_ctx *c, const double *qref) {
 int cruna_hip_set_kvector(cruna_hip_ctx *c, const double *kvector) {
   if (!c || !kvector) return fail(CRUNA_HIP_EINVAL, "null argument");
   ++c->gen;
-  for (long i = 0; i < 3 * c->N; ++i)
+  for (long i = 0; i < 3 * real_points(c); ++i)
     if (!std::isfinite(kvector[i])) return fail(CRUNA_HIP_EINVAL, "kvector is not finite");
   if (!c->kvec) HIP_TRY(hipMalloc(&c->kvec, 3 * c->N * sizeof(double)));
   const double kfill[3] = {1.0, 0.0, 0.0};
