@@ -16,48 +16,31 @@ struct BoxRow {
   long aim_shift;              // type 200: offset of the inner neighbour (zero-gradient aim)
 };
 
-// characteristic_q_k1d (src/boundaries/nonreflecting.f90:46-137) on the
-// points of one box: q <- q + (incoming part of prim(aim) - prim(q)).
-// Type 201: aim = qref at the same point (row.aim_shift 0); type 200: aim =
-// q at the inner neighbour (characteristic_zero_grad_init, :665-728), a point
-// outside the one-point-thick box, so the in-place update reads no value it
-// writes.
-// kfield (types 202/205, characteristic_*_k4d): the normal per point,
-// kvector(n1,n2,n3,3), in place of the row's; null: the row's (201/204).
-// shape (type 203, characteristic_q_k4d with shape, :180-185): the change
-// toward aim is scaled by shape at the point before the decomposition.
+// characteristic_q_k1d (src/boundaries/nonreflecting.f90:46-137) at a point:
+// q <- q + (incoming part of prim(aim) - prim(q)), k = (kx, ky, kz) the inward
+// normal; sh (type 203, characteristic_q_k4d with shape, :180-185): the change
+// toward aim is scaled by it before the decomposition.
 template <typename Q, typename A>
-__global__ __launch_bounds__(256) void k_bc_characteristic_q(Q *q, const A *aim_base, BoxRow row,
-                                                              int n1, int n2, long N, double gamma,
-                                                              const double *__restrict__ kfield,
-                                                              const double *__restrict__ shape) {
-  const long nx = row.i1 - row.i0 + 1, ny = row.j1 - row.j0 + 1, nz = row.k1 - row.k0 + 1;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nx * ny * nz) return;
-  const long i = row.i0 + t % nx, j = row.j0 + (t / nx) % ny, k = row.k0 + t / (nx * ny);
-  const long o = i + (long)n1 * (j + (long)n2 * k);
-  const A *aim = aim_base + row.aim_shift;
-  double r = double(q[o]);
-  double u1 = double(q[N + o]) / double(q[o]);
-  double u2 = double(q[2 * N + o]) / double(q[o]);
-  double u3 = double(q[3 * N + o]) / double(q[o]);
-  double p = double(q[4 * N + o]);
-  const double c = sqrt(gamma * double(q[4 * N + o]) / double(q[o]));
-  double dq1 = double(aim[o]) - r;
-  double dq2 = double(aim[N + o]) / double(aim[o]) - u1;
-  double dq3 = double(aim[2 * N + o]) / double(aim[o]) - u2;
-  double dq4 = double(aim[3 * N + o]) / double(aim[o]) - u3;
-  double dq5 = double(aim[4 * N + o]) - p;
-  if (shape) {
-    const double sh = shape[o];
-    dq1 *= sh;
-    dq2 *= sh;
-    dq3 *= sh;
-    dq4 *= sh;
-    dq5 *= sh;
+__device__ __forceinline__ void characteristic_q(Q (&q)[5], const A (&aim)[5], double kx, double ky, double kz,
+                                                 double gamma, const double *sh) {
+  double r = double(q[0]);
+  double u1 = double(q[1]) / double(q[0]);
+  double u2 = double(q[2]) / double(q[0]);
+  double u3 = double(q[3]) / double(q[0]);
+  double p = double(q[4]);
+  const double c = sqrt(gamma * double(q[4]) / double(q[0]));
+  double dq1 = double(aim[0]) - r;
+  double dq2 = double(aim[1]) / double(aim[0]) - u1;
+  double dq3 = double(aim[2]) / double(aim[0]) - u2;
+  double dq4 = double(aim[3]) / double(aim[0]) - u3;
+  double dq5 = double(aim[4]) - p;
+  if (sh) {
+    dq1 *= *sh;
+    dq2 *= *sh;
+    dq3 *= *sh;
+    dq4 *= *sh;
+    dq5 *= *sh;
   }
-  const double kx = -(kfield ? kfield[o] : row.k[0]), ky = -(kfield ? kfield[N + o] : row.k[1]),
-               kz = -(kfield ? kfield[2 * N + o] : row.k[2]);
   // primitive -> characteristic waves (:97-101)
   double R1 = kx * dq1 + kz * dq3 - ky * dq4 - kx * dq5 / (c * c);
   double R2 = ky * dq1 - kz * dq2 + kx * dq4 - ky * dq5 / (c * c);
@@ -80,11 +63,90 @@ __global__ __launch_bounds__(256) void k_bc_characteristic_q(Q *q, const A *aim_
   u2 = u2 + dq3;
   u3 = u3 + dq4;
   p = p + dq5;
-  q[o] = Q(r);
-  q[N + o] = Q(r * u1);
-  q[2 * N + o] = Q(r * u2);
-  q[3 * N + o] = Q(r * u3);
-  q[4 * N + o] = Q(p);
+  q[0] = Q(r);
+  q[1] = Q(r * u1);
+  q[2] = Q(r * u2);
+  q[3] = Q(r * u3);
+  q[4] = Q(p);
+}
+
+// Type 200: a row's aim is q at the inner neighbour (row.aim_shift;
+// characteristic_zero_grad_init, :665-728), a point outside the
+// one-point-thick box, so the in-place update reads no value it writes.
+template <typename Q>
+__global__ __launch_bounds__(256) void k_bc_zero_gradient_q(Q *q, BoxRow row, int n1, int n2, long N, double gamma) {
+  const long nx = row.i1 - row.i0 + 1, ny = row.j1 - row.j0 + 1, nz = row.k1 - row.k0 + 1;
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nx * ny * nz) return;
+  const long i = row.i0 + t % nx, j = row.j0 + (t / nx) % ny, k = row.k0 + t / (nx * ny);
+  const long o = i + (long)n1 * (j + (long)n2 * k);
+  Q v[5], aim[5];
+#pragma unroll
+  for (int c = 0; c < 5; ++c) {
+    v[c] = q[c * N + o];
+    aim[c] = q[c * N + o + row.aim_shift];
+  }
+  characteristic_q(v, aim, -row.k[0], -row.k[1], -row.k[2], gamma, nullptr);
+#pragma unroll
+  for (int c = 0; c < 5; ++c) q[c * N + o] = v[c];
+}
+
+// Consecutive rows of the types 201, 202 and 203, whose aim is qref at the same
+// point: one launch, since they act point by point.  A point is updated by
+// the thread of the first row that holds it, which applies that row and the
+// later ones in their order.  Bound by the latency of a point's loads and the
+// divisions of its rows: launched one by one, the six faces of a 60 x 65 x 70 box
+// took 5 us each, together they take 13.
+// kfield (202/203, characteristic_*_k4d): the normal per point,
+// kvector(n1,n2,n3,3), in place of the row's; shape: 203.
+constexpr int BC_ROWS = 12;
+struct BoxRows {
+  int n;
+  int kvec, shaped;      // bit m: row m takes its normals from kfield / its change is scaled by shape
+  int first[BC_ROWS + 1];  // threads before row m
+  BoxRow row[BC_ROWS];
+};
+template <typename Q>
+__global__ __launch_bounds__(256) void k_bc_characteristic_q(Q *q, const double *__restrict__ qref, BoxRows rows,
+                                                              int n1, int n2, long N, double gamma,
+                                                              const double *__restrict__ kfield,
+                                                              const double *__restrict__ shape) {
+  const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (t >= rows.first[rows.n]) return;
+  int mine = 0, f = 0;
+  BoxRow box = rows.row[0];
+  for (int m = 1; m < rows.n; ++m) {
+    if (t < rows.first[m]) continue;
+    mine = m;
+    f = rows.first[m];
+    box = rows.row[m];
+  }
+  const unsigned nx = box.i1 - box.i0 + 1, ny = box.j1 - box.j0 + 1, p = t - f;
+  const int i = box.i0 + int(p % nx), j = box.j0 + int(p / nx % ny), k = box.k0 + int(p / nx / ny);
+  auto holds = [&](const BoxRow &row) {
+    return i >= row.i0 && i <= row.i1 && j >= row.j0 && j <= row.j1 && k >= row.k0 && k <= row.k1;
+  };
+  for (int m = 0; m < mine; ++m)
+    if (holds(rows.row[m])) return;
+  const long o = i + (long)n1 * (j + (long)n2 * k);
+  Q v[5];
+  double aim[5];
+#pragma unroll
+  for (int c = 0; c < 5; ++c) {
+    v[c] = q[c * N + o];
+    aim[c] = qref[c * N + o];
+  }
+#pragma unroll 1
+  for (int m = 0; m < rows.n; ++m) {
+    const BoxRow &row = rows.row[m];
+    if (m < mine || !holds(row)) continue;
+    const bool kv = (rows.kvec >> m) & 1;
+    const double kx = -(kv ? kfield[o] : row.k[0]), ky = -(kv ? kfield[N + o] : row.k[1]),
+                 kz = -(kv ? kfield[2 * N + o] : row.k[2]);
+    characteristic_q(v, aim, kx, ky, kz, gamma, (rows.shaped >> m) & 1 ? shape + o : nullptr);
+  }
+#pragma unroll
+  for (int c = 0; c < 5; ++c) q[c * N + o] = v[c];
 }
 
 // characteristic_rhs_k1d (src/boundaries/nonreflecting.f90:237-341, type 204)

@@ -468,34 +468,42 @@ bool zone_applies(const cruna_hip_ctx *c, bool outside) {
 template <typename Q>
 int bc_q(cruna_hip_ctx *c, Q *q, bool outside = false) {
   if (int rc = need_bc_inputs(c)) return rc;
+  auto points = [](const BoxRow &b) {
+    return (long)(b.i1 - b.i0 + 1) * (b.j1 - b.j0 + 1) * (b.k1 - b.k0 + 1);
+  };
+  // consecutive 201/202/203 rows, launched together
+  BoxRows rows{};
+  auto flush = [&]() -> int {
+    if (rows.n == 0) return CRUNA_HIP_OK;
+    hipLaunchKernelGGL((k_bc_characteristic_q<Q>), dim3((rows.first[rows.n] + 255) / 256), dim3(256), 0, c->stream, q,
+                       (const double *)c->qref, rows, c->np[0], c->np[1], c->N, c->cfg.gamma, (const double *)c->kvec,
+                       (const double *)c->shape);
+    rows = BoxRows{};
+    return check_launch();
+  };
   for (auto &r : c->bc) {
-    if (r.first == 201) {
-      const BoxRow &b = r.second;
-      const long np = (long)(b.i1 - b.i0 + 1) * (b.j1 - b.j0 + 1) * (b.k1 - b.k0 + 1);
-      hipLaunchKernelGGL((k_bc_characteristic_q<Q, double>), dim3((np + 255) / 256), dim3(256), 0,
-                         c->stream, q, (const double *)c->qref, b, c->np[0], c->np[1], c->N,
-                         c->cfg.gamma, (const double *)nullptr, (const double *)nullptr);
-    } else if (r.first == 202 || r.first == 203) {
-      if (r.first == 203 && !zone_applies(c, outside)) continue;
-      const BoxRow &b = r.second;
-      const long np = (long)(b.i1 - b.i0 + 1) * (b.j1 - b.j0 + 1) * (b.k1 - b.k0 + 1);
-      hipLaunchKernelGGL((k_bc_characteristic_q<Q, double>), dim3((np + 255) / 256), dim3(256), 0,
-                         c->stream, q, (const double *)c->qref, b, c->np[0], c->np[1], c->N,
-                         c->cfg.gamma, (const double *)c->kvec,
-                         r.first == 203 ? (const double *)c->shape : (const double *)nullptr);
-    } else if (r.first == 200) {
-      const BoxRow &b = r.second;
-      const long np = (long)(b.i1 - b.i0 + 1) * (b.j1 - b.j0 + 1) * (b.k1 - b.k0 + 1);
-      hipLaunchKernelGGL((k_bc_characteristic_q<Q, Q>), dim3((np + 255) / 256), dim3(256), 0,
-                         c->stream, q, (const Q *)q, b, c->np[0], c->np[1], c->N, c->cfg.gamma,
-                         (const double *)nullptr, (const double *)nullptr);
-    } else if (r.first == 401) {
-      hipLaunchKernelGGL((k_bc_sponge_q<Q>), dim3((c->N + 255) / 256), dim3(256), 0, c->stream, q,
-                         (const double *)c->qref, (const double *)c->shape, c->N);
+    const BoxRow &b = r.second;
+    if (r.first == 203 && !zone_applies(c, outside)) continue;
+    if (r.first == 201 || r.first == 202 || r.first == 203) {
+      if (rows.n == BC_ROWS || rows.first[rows.n] + points(b) >= (1L << 31) - 256)
+        if (int rc = flush()) return rc;
+      const int m = rows.n++;
+      rows.row[m] = b;
+      if (r.first != 201) rows.kvec |= 1 << m;
+      if (r.first == 203) rows.shaped |= 1 << m;
+      rows.first[m + 1] = rows.first[m] + (int)points(b);
+    } else if (r.first == 200 || r.first == 401) {
+      if (int rc = flush()) return rc;
+      if (r.first == 200)
+        hipLaunchKernelGGL((k_bc_zero_gradient_q<Q>), dim3((points(b) + 255) / 256), dim3(256), 0, c->stream, q, b,
+                           c->np[0], c->np[1], c->N, c->cfg.gamma);
+      else
+        hipLaunchKernelGGL((k_bc_sponge_q<Q>), dim3((c->N + 255) / 256), dim3(256), 0, c->stream, q,
+                           (const double *)c->qref, (const double *)c->shape, c->N);
+      if (int rc = check_launch()) return rc;
     }
-    if (int rc = check_launch()) return rc;
   }
-  return CRUNA_HIP_OK;
+  return flush();
 }
 
 // set_boundary_condition_rhs (boundary_conditions.f90:228-298), rows in order.
