@@ -298,6 +298,13 @@ int build_geom(cruna_hip_ctx *c, int d) {
     STL = auto_tl(np, d, NT_SWEEP32, 32);
   c->sgeom[d] = make_geom(np, d, STL);
   c->swg[d] = NB * STL;
+  // States larger than the 256 MB memory-side cache: the sweeps along x and y go
+  // plane by plane, so a sweep that runs backwards over what the last one
+  // ended with finds its newest planes there (256^3, 25 steps: FP64 259.4 ->
+  // 255.8 ms, FP32-mixed 285.8 -> 281.3).  Smaller states are there anyway,
+  // and keep what an XCD's L2 holds by walking forwards (64^3 1 % faster).
+  const size_t ts = cfg.precision == CRUNA_HIP_FP32_MIXED ? sizeof(float) : sizeof(double);
+  c->geom[d].back = c->sgeom[d].back = 5 * (size_t)c->N * ts > (256u << 20) ? 1 : 0;
   return CRUNA_HIP_OK;
 }
 

@@ -44,6 +44,7 @@ struct SweepGeom {
   int ntiles;     // work-groups in the grid
   int ntiles_in;  // (y/z) tiles along i
   long lines;     // batched launches: lines of the direction, taken TL at a time
+  int back;       // first x sweep and second y sweep walk their tiles backwards
 };
 
 // Thread placement inside a tile.  The LDS slot of a (line, block) pair is the
@@ -57,10 +58,12 @@ struct ThreadPos {
 };
 
 // Work-groups are dealt round-robin to the 8 XCDs; map consecutive tiles to the
-// same XCD so that tiles sharing cache lines meet in the same L2.
-__device__ inline int xcd_tile(int bid, int ntiles) {
-  if (ntiles % 8 != 0) return bid;
-  return (bid % 8) * (ntiles / 8) + bid / 8;
+// same XCD so that tiles sharing cache lines meet in the same L2.  rev: each
+// XCD walks its tiles backwards.
+__device__ inline int xcd_tile(int bid, int ntiles, bool rev = false) {
+  if (ntiles % 8 != 0) return rev ? ntiles - 1 - bid : bid;
+  const int per = ntiles / 8, t = bid / 8;
+  return (bid % 8) * per + (rev ? per - 1 - t : t);
 }
 
 // Element offset of an idle thread's block: 2^28 FP64 elements is the 2 GiB
@@ -124,9 +127,11 @@ __device__ inline ThreadPos thread_pos_tile(const SweepGeom &g, int tile) {
   return t;
 }
 
-template <int DIR>
+// (BACK: a sweep that follows one over the same planes and, where g.back is
+// set, walks them backwards)
+template <int DIR, bool BACK = false>
 __device__ inline ThreadPos thread_pos(const SweepGeom &g) {
-  return thread_pos_tile<DIR>(g, xcd_tile(blockIdx.x, g.ntiles));
+  return thread_pos_tile<DIR>(g, xcd_tile(blockIdx.x, g.ntiles, BACK && g.back));
 }
 
 // Work-group barrier that orders LDS traffic only.  __syncthreads() also waits

@@ -846,7 +846,7 @@ template <typename T, typename Q, int DIR, bool PER, int FORM>
 __global__ __launch_bounds__(NT) void k_sweep1(const Q *__restrict__ qs, T *__restrict__ rhs,
                                                           T *__restrict__ G, Op<T> op, SweepGeom g,
                                                           Phys ph, long N, Metric<T> mt, Penal<T> pe) {
-  const ThreadPos tp = thread_pos<DIR>(g);
+  const ThreadPos tp = thread_pos<DIR, DIR == 0>(g);
   auto ln = make_lines<T, PER>(op, tp);
   if constexpr (DIR == 0 && stress_form<T, FORM>())
     sweep1_x_cart(tp, qs, rhs, G, op, g, ph, N, ln);
@@ -1269,7 +1269,7 @@ __global__ __launch_bounds__(sweep_nt<T>()) void k_sweep2(T *__restrict__ rhs, c
                                                           Op<T> op, Op<T> fop, SweepGeom g, Phys ph,
                                                           long N, RkArgs<T> rk, Metric<T> mt,
                                                           const T *__restrict__ force, Penal<T> pe) {
-  const ThreadPos tp = thread_pos<DIR>(g);
+  const ThreadPos tp = thread_pos<DIR, DIR == 1>(g);
   auto ln = make_lines<T, PER, sweep_nt<T>()>(op, tp);
   sweep2_body<T, DIR, FORM, RK, FF>(tp, rhs, G, op, fop, g, ph, N, rk, mt, force, pe, ln);
 }
