@@ -274,8 +274,13 @@ int build_geom(cruna_hip_ctx *c, int d) {
   int TL = cfg.tile_lines[d];
   if (TL == 0) {
     // x-lines are contiguous: up to 256 threads; y/z tiles take up to 16
-    // neighbouring x-lines (128-byte rows in FP64) in up to 512 threads
-    TL = d == 0 ? auto_tl(np, d, 256, 1 << 20) : auto_tl(np, d, NT, 16);
+    // neighbouring x-lines (128-byte rows in FP64) in up to 512 threads.
+    // FP64 grids with less than a wavefront per SIMD (1024): work-groups of one
+    // wavefront where its lines fill it, spread over more CUs and with no
+    // barriers (a step with filters, x alone: 32^3 169 -> 155 us,
+    // 60 x 65 x 70 481 -> 471; 64^3 228 -> 224, y and z alone 225 each)
+    const bool small = cfg.precision == CRUNA_HIP_FP64 && c->N <= 1024L * 64 * PPT && 64 % NB == 0;
+    TL = d == 0 ? auto_tl(np, d, small ? 64 : 256, 1 << 20) : auto_tl(np, d, small ? 64 : NT, 16);
   } else if (TL < 0 || (TL & (TL - 1)) != 0 || lines_contig % TL != 0 || NB * TL > NT) {
     return fail(CRUNA_HIP_EINVAL, "tile_lines[" + std::to_string(d) + "] = " + std::to_string(TL) +
                                       ": needs a power of two dividing " +
