@@ -49,7 +49,7 @@ constexpr int REC_WIN = 6;  // window terms kept as addresses (more: the slow lo
 // runs on the cyclic reduction of line_solve.hpp
 constexpr double REC_MAX_LAMBDA = 0.9;
 
-// Table of an open line's ends (device memory, read through the scalar cache):
+// Table of an open line's ends (device memory; RecLines copies what it needs to LDS):
 // per end (0 left, 1 right):
 //   [0 .. 8 FE)  dense explicit rows of the end block (scaled)
 //   [8 FE .. +8) C: A_end = C . x~ over the block's rows
