@@ -99,7 +99,8 @@ inline HostRecOp build_rec_op(OpKind kind, bool per, int n_real, double alpha) {
   op.per = per ? 1 : 0;
   const long double al = (long double)lo[mid] / di[mid];
   if (!(std::fabs((double)al) < 0.5)) return h;
-  const long double lam = al == 0.0L ? 0.0L : (1.0L - std::sqrt(1.0L - 4.0L * al * al)) / (2.0L * al);
+  // (this form of the root keeps its digits for small alpha)
+  const long double lam = 2.0L * al / (1.0L + std::sqrt(1.0L - 4.0L * al * al));
   if (std::fabs((double)lam) > REC_MAX_LAMBDA) return h;
   h.usable = true;
   const long double mu = -lam, sc = (1.0L + lam * lam) / di[mid];
@@ -193,7 +194,9 @@ inline HostRecOp build_rec_op(OpKind kind, bool per, int n_real, double alpha) {
     const long double a11 = b[0][0] + b[0][1] * mu, a12 = b[0][0],
                       a21 = b[1][0] + b[1][1] * mu + b[1][2] * mu * mu, a22 = b[1][0];
     const long double det = a11 * a22 - a12 * a21;
-    if (std::fabs((double)det) < 1e-12) throw std::runtime_error("singular end closure");
+    // (relative to the rows: a filter's second one is of the size of alpha)
+    const long double size = std::max(std::fabs(a11), std::fabs(a12)) * std::max(std::fabs(a21), std::fabs(a22));
+    if (!(std::fabs(det) > 1e-12L * size)) throw std::runtime_error("singular end closure");
     const long double i11 = a22 / det, i12 = -a12 / det, i21 = -a21 / det, i22 = a11 / det;
     for (int k = 0; k < 3; ++k) {
       C[e][k] = -(i11 * E[0][k] + i12 * E[1][k]);
