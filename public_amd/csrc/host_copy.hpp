@@ -44,11 +44,7 @@ class HostCopyPool {
   void drop_user() {
     std::lock_guard<std::mutex> l(mu_);
     if (--users_ > 0) return;
-    for (auto &s : slots_) {
-      if (s.ev) (void)hipEventDestroy(s.ev);
-      if (s.pin) (void)hipHostFree(s.pin);
-    }
-    slots_.clear();
+    give_back();
   }
   // host <-> dev on stream s of device `device`.  The host array may be used
   // again (to the device) or holds the values (to the host) when it returns.
@@ -68,34 +64,48 @@ class HostCopyPool {
   }
 
  private:
+  // A thread's chunk, which any device reaches, and the event of its last
+  // transfer: an event belongs to one device and is recorded on that device's
+  // streams only, so it is made anew when the slot serves another one.
   struct Slot {
     void *pin = nullptr;
     hipEvent_t ev = nullptr;
+    int device = -1;  // of ev
+    hipError_t bind(int d) {
+      hipError_t e = hipSetDevice(d);
+      if (e != hipSuccess || (ev && device == d)) return e;
+      if (ev) (void)hipEventDestroy(ev);
+      ev = nullptr;
+      e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+      if (e != hipSuccess) ev = nullptr;
+      device = d;
+      return e;
+    }
   };
   std::mutex mu_;
   int users_ = 0;
-  std::vector<Slot> slots_;
+  Slot slots_[HC_THREADS];
 
-  bool reserve() {
-    if (!slots_.empty()) return true;
-    std::vector<Slot> v(HC_THREADS);
-    bool ok = true;
-    for (auto &s : v)
-      ok = ok && hipHostMalloc(&s.pin, HC_CHUNK, hipHostMallocPortable) == hipSuccess &&
-           hipEventCreateWithFlags(&s.ev, hipEventDisableTiming) == hipSuccess;
-    if (!ok) {
-      (void)hipGetLastError();
-      for (auto &s : v) {
-        if (s.ev) (void)hipEventDestroy(s.ev);
-        if (s.pin) (void)hipHostFree(s.pin);
-      }
-      return false;
+  void give_back() {
+    for (auto &s : slots_) {
+      if (s.ev) (void)hipEventDestroy(s.ev);
+      if (s.pin) (void)hipHostFree(s.pin);
+      s = Slot{};
     }
-    slots_.swap(v);
+  }
+  bool reserve() {
+    if (slots_[HC_THREADS - 1].pin) return true;
+    for (auto &s : slots_)
+      if (hipHostMalloc(&s.pin, HC_CHUNK, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        s.pin = nullptr;
+        give_back();
+        return false;
+      }
     return true;
   }
 
-  // false: no thread could be started, nothing was copied
+  // false: no thread could be started or made its event, nothing was copied
   bool staged(void *dst, const void *src, size_t bytes, bool to_device, int device, hipStream_t s, hipError_t &err) {
     const int nt = (int)std::min<size_t>(HC_THREADS, std::max<size_t>(2, bytes / HC_CHUNK));
     // at least two chunks per thread, so that copies and transfers overlap
@@ -103,10 +113,12 @@ class HostCopyPool {
     chunk = std::min(HC_CHUNK, std::max<size_t>(chunk, 4096));
     const size_t n = (bytes + chunk - 1) / chunk;
     std::atomic<size_t> next{0};
-    std::atomic<int> bad{(int)hipSuccess};
+    std::atomic<int> bad{(int)hipSuccess}, ready{0};
     auto work = [&](int t) {
-      const Slot &slot = slots_[t];
-      hipError_t e = hipSetDevice(device);
+      Slot &slot = slots_[t];
+      hipError_t e = slot.bind(device);
+      if (e != hipSuccess) return;  // the other threads share out its chunks
+      ++ready;
       bool used = false;
       while (e == hipSuccess && bad.load() == (int)hipSuccess) {
         const size_t i = next.fetch_add(1);
@@ -141,6 +153,7 @@ class HostCopyPool {
       if (th.empty()) return false;
     }
     for (auto &t : th) t.join();
+    if (ready.load() == 0) return false;
     err = (hipError_t)bad.load();
     if (err != hipSuccess) (void)hipStreamSynchronize(s);  // nothing uses the pinned chunks any more
     return true;
