@@ -37,14 +37,14 @@ class HostCopyPool {
     static HostCopyPool *p = new HostCopyPool();  // outlives every user
     return *p;
   }
-  void add_user() {
-    std::lock_guard<std::mutex> l(mu_);
-    ++users_;
-  }
+  // (a count of its own: no context waits for another one's copy when it is
+  // made or released)
+  void add_user() { ++users_; }
   void drop_user() {
-    std::lock_guard<std::mutex> l(mu_);
     if (--users_ > 0) return;
-    give_back();
+    // nobody copies any more, unless a user came since: its own end gives back then
+    std::lock_guard<std::mutex> l(mu_);
+    if (users_ == 0) give_back();
   }
   // host <-> dev on stream s of device `device`.  The host array may be used
   // again (to the device) or holds the values (to the host) when it returns.
@@ -82,8 +82,8 @@ class HostCopyPool {
       return e;
     }
   };
-  std::mutex mu_;
-  int users_ = 0;
+  std::mutex mu_;  // held by the copy that uses the slots
+  std::atomic<int> users_{0};
   Slot slots_[HC_THREADS];
 
   void give_back() {

@@ -1,8 +1,9 @@
 // The staged host copies of public_amd/csrc/host_copy.hpp over the HIP model of
-// hip_model/: contexts of several devices.
+// hip_model/: contexts of several devices, users that come and go meanwhile.
 // Prints one line per case: name ok.
 #include <algorithm>
 #include <cstdio>
+#include <future>
 #include <vector>
 
 #include "../../public_amd/csrc/host_copy.hpp"
@@ -33,6 +34,20 @@ int main() {
     std::printf("no_events %d\n", round_trip(5, sizes[1], 9));
     model_no_events = 0;
     std::printf("events_again %d\n", round_trip(5, sizes[1], 9));
+    // while one copy runs, contexts come and go without waiting for it
+    std::vector<char> a(sizes[1], 1), dev(sizes[1]);
+    ModelStream s{0};
+    model_held = false;
+    model_hold = true;
+    auto copy = std::async(std::launch::async, [&] {
+      return HostCopyPool::get().copy(dev.data(), a.data(), a.size(), true, 0, &s);
+    });
+    while (!model_held) std::this_thread::yield();
+    auto other = std::async(std::launch::async, [] { HostCopyUser v; });
+    const bool free = other.wait_for(std::chrono::seconds(5)) == std::future_status::ready;
+    model_hold = false;
+    other.wait();
+    std::printf("users_do_not_wait %d\n", free && copy.get() == hipSuccess && a == dev);
   }
   std::printf("given_back %d\n", model_events == 0 && model_pinned == 0);
   {

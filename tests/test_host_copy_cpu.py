@@ -1,13 +1,14 @@
 """CPU check of the staged host copies' bookkeeping (public_amd/csrc/host_copy.hpp
 over a model of the HIP calls it makes): contexts of several devices in one
-process, and what is given back."""
+process, users that come and go while a copy runs, and what is given back."""
 import os
 import subprocess
 
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-CASES = ["devices", "events_bounded", "no_events", "events_again", "given_back", "made_again", "given_back_again"]
+CASES = ["devices", "events_bounded", "no_events", "events_again", "users_do_not_wait", "given_back", "made_again",
+         "given_back_again"]
 
 
 @pytest.fixture(scope="module")
