@@ -360,7 +360,13 @@ using Op = typename OpOf<T>::type;
 
 // The lines of a work-group: solve(op, f, x) is x = B^-1 A f on the thread's
 // block, solve2 two independent fields at once (all threads together, in the
-// same order).  CR: the cyclic reduction above; one field after the other.
+// same order).  pair is two solves whose results are used at once, use1() and
+// use2(), make2() preparing the second's input: CR, the cyclic reduction above,
+// takes the fields one after the other, and no result or input of the second
+// lives during the first; the recursions take both at once.  (With CR's
+// results used after both solves, the FP32 first-derivative sweeps took 7 to
+// 10 more registers, one wavefront per SIMD less, and the FP32-mixed step of an
+// open 192^3 box 4 % longer.)
 template <typename T, bool PER, int NTM>
 struct CrLines {
   LineLds<T, NTM> &lds;
@@ -373,6 +379,15 @@ struct CrLines {
                                          T (&x2)[PPT]) {
     line_solve<T, PER>(op, lds, tp, f1, x1);
     line_solve<T, PER>(op, lds, tp, f2, x2);
+  }
+  template <typename U1, typename M2, typename U2>
+  __device__ __forceinline__ void pair(const LineOp<T> &op, const T (&f1)[PPT], T (&x1)[PPT], U1 use1, M2 make2,
+                                       const T (&f2)[PPT], T (&x2)[PPT], U2 use2) {
+    line_solve<T, PER>(op, lds, tp, f1, x1);
+    use1();
+    make2();
+    line_solve<T, PER>(op, lds, tp, f2, x2);
+    use2();
   }
   __device__ __forceinline__ void bind(const LineOp<T> &) {}
 };
@@ -682,6 +697,14 @@ struct RecLines {
       x1[i] = r[0][i];
       x2[i] = r[1][i];
     }
+  }
+  template <typename U1, typename M2, typename U2>
+  __device__ __forceinline__ void pair(const RecOp &op, const double (&f1)[PPT], double (&x1)[PPT], U1 use1, M2 make2,
+                                       const double (&f2)[PPT], double (&x2)[PPT], U2 use2) {
+    make2();
+    solve2(op, f1, x1, f2, x2);
+    use1();
+    use2();
   }
 };
 

@@ -409,113 +409,144 @@ __device__ __forceinline__ void sweep1_body(const ThreadPos &tp, const Q *__rest
     io.got(ui);
     if (gsum(i)) io.got(gs);
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) {
-      ui[m] = ui[m] * irho[m];
-      f[m] = EV ? (PH[m] * mom[m]) * ui[m] : mom[m] * ui[m];
-    }
-    if (DIR != 0) io.ld(rhs + (1 + i) * N, r);
-    if (k == 1) io.ld(qs + 4 * N, p);  // in flight for the pressure terms
-    ln.solve2(op, ui, y, f, x);
-    if (DIR != 0) io.got(r);
-    if (k == 1) io.got(p);
+    for (int m = 0; m < PPT; ++m) ui[m] = ui[m] * irho[m];
+    ln.pair(
+        op, ui, y,
+        [&] {
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) {
-      y[m] = y[m] * ih;
-      if (gsum(i)) y[m] = y[m] + gs[m];
-    }
-    io.st(G + gslot(i) * N, y);
-    if constexpr (FUSE) {
+          for (int m = 0; m < PPT; ++m) {
+            y[m] = y[m] * ih;
+            if (gsum(i)) y[m] = y[m] + gs[m];
+          }
+          io.st(G + gslot(i) * N, y);
+          if constexpr (FUSE) {
 #pragma unroll
-      for (int m = 0; m < PPT; ++m) (k == 0 ? zc->s13 : zc->s23)[m] = y[m];
-    }
+            for (int m = 0; m < PPT; ++m) (k == 0 ? zc->s13 : zc->s23)[m] = y[m];
+          }
+        },
+        [&] {
+          if (DIR != 0) io.ld(rhs + (1 + i) * N, r);
+          if (k == 1) io.ld(qs + 4 * N, p);  // in flight for the pressure terms
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
-    if constexpr (FUSE) {
+          for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * mom[m]) * ui[m] : mom[m] * ui[m];
+        },
+        f, x,
+        [&] {
+          if (DIR != 0) io.got(r);
+          if (k == 1) io.got(p);
 #pragma unroll
-      for (int m = 0; m < PPT; ++m) zc->mom(i, m) = r[m];
-    } else {
-      io.st(rhs + (1 + i) * N, r);
-    }
+          for (int m = 0; m < PPT; ++m) r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
+          if constexpr (FUSE) {
+#pragma unroll
+            for (int m = 0; m < PPT; ++m) zc->mom(i, m) = r[m];
+          } else {
+            io.st(rhs + (1 + i) * N, r);
+          }
+        });
   }
 
   // d(u_DIR)/dx_DIR, and mass: -d/dx_DIR (rho u_DIR) (:131-135)
   T ud[PPT];
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) {
-    ud[m] = mom[m] * irho[m];
-    f[m] = EV ? PH[m] * mom[m] : mom[m];
-  }
-  if (DIR != 0) io.ld(rhs, r);
-  ln.solve2(op, ud, y, f, x);
-  if (DIR != 0) io.got(r);
+  for (int m = 0; m < PPT; ++m) ud[m] = mom[m] * irho[m];
+  ln.pair(
+      op, ud, y,
+      [&] {
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) y[m] = y[m] * ih;
-  io.st(G + DIR * N, y);
-  if constexpr (FUSE) {
+        for (int m = 0; m < PPT; ++m) y[m] = y[m] * ih;
+        io.st(G + DIR * N, y);
+        if constexpr (FUSE) {
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) zc->wz[m] = y[m];
-  }
+          for (int m = 0; m < PPT; ++m) zc->wz[m] = y[m];
+        }
+      },
+      [&] {
+        if (DIR != 0) io.ld(rhs, r);
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
-  io.st(rhs, r);
+        for (int m = 0; m < PPT; ++m) f[m] = EV ? PH[m] * mom[m] : mom[m];
+      },
+      f, x,
+      [&] {
+        if (DIR != 0) io.got(r);
+#pragma unroll
+        for (int m = 0; m < PPT; ++m) r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
+        io.st(rhs, r);
+      });
 
   // pressure gradient p_DIR, and momentum DIR: -d/dx_DIR (rho u_DIR u_DIR) - p_DIR
   T pd[PPT];
-  if (DIR != 0) io.ld(rhs + (1 + DIR) * N, r);
+  ln.pair(
+      op, p, pd,
+      [&] {
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * mom[m]) * ud[m] : mom[m] * ud[m];
-  ln.solve2(op, p, pd, f, x);
-  if (DIR != 0) io.got(r);
+        for (int m = 0; m < PPT; ++m) pd[m] = pd[m] * ih;
+      },
+      [&] {
+        if (DIR != 0) io.ld(rhs + (1 + DIR) * N, r);
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) {
-    pd[m] = pd[m] * ih;
-    r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
-    r[m] = r[m] - pd[m];
-  }
-  if constexpr (FUSE) {
+        for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * mom[m]) * ud[m] : mom[m] * ud[m];
+      },
+      f, x,
+      [&] {
+        if (DIR != 0) io.got(r);
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) zc->mom(DIR, m) = r[m];
-  } else {
-    io.st(rhs + (1 + DIR) * N, r);
-  }
+        for (int m = 0; m < PPT; ++m) {
+          r[m] = DIR == 0 ? div(m, -(x[m] * ih)) : r[m] + div(m, -(x[m] * ih));
+          r[m] = r[m] - pd[m];
+        }
+        if constexpr (FUSE) {
+#pragma unroll
+          for (int m = 0; m < PPT; ++m) zc->mom(DIR, m) = r[m];
+        } else {
+          io.st(rhs + (1 + DIR) * N, r);
+        }
+      });
 
   // pressure-equation bracket: gamma/(gamma-1) (-d(p u_DIR)) + u_DIR p_DIR
   // (:180-187), and the inner derivative of the heat flux d/dx_DIR (lambda
   // d/dx_DIR T) (:189-199); the x sweep evaluates the viscosity law and leaves
   // mu in G6 for the later sweeps of the stage
   T e[PPT], tk[PPT], mu[PPT], Jv[PPT];
-  if (DIR != 0) {
-    io.ld(rhs + 4 * N, r);
-    io.ld(G + 6 * N, mu);
-  }
-  if (GT) io.ld(mt.J, Jv);
-  if (DIR != 0) {
-    io.got(r);
-    io.got(mu);
-  }
-  if (GT) io.got(Jv);
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) {
-    f[m] = EV ? (PH[m] * p[m]) * ud[m] : p[m] * ud[m];
-    tk[m] = temperature(ph, irho[m], p[m]);
-  }
-  if (DIR == 0) {
+  for (int m = 0; m < PPT; ++m) f[m] = EV ? (PH[m] * p[m]) * ud[m] : p[m] * ud[m];
+  ln.pair(
+      op, f, x,
+      [&] {
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) mu[m] = viscosity(ph, tk[m]);
-    io.st(G + 6 * N, mu);
-  }
-  if constexpr (FUSE) {
+        for (int m = 0; m < PPT; ++m) e[m] = div(m, T(ph.gt) * (-(x[m] * ih))) + ud[m] * pd[m];
+      },
+      [&] {
+        if (DIR != 0) {
+          io.ld(rhs + 4 * N, r);
+          io.ld(G + 6 * N, mu);
+        }
+        if (GT) io.ld(mt.J, Jv);
+        if (DIR != 0) {
+          io.got(r);
+          io.got(mu);
+        }
+        if (GT) io.got(Jv);
 #pragma unroll
-    for (int m = 0; m < PPT; ++m) zc->mu[m] = mu[m];
-  }
-  ln.solve2(op, f, x, tk, y);
+        for (int m = 0; m < PPT; ++m) tk[m] = temperature(ph, irho[m], p[m]);
+        if (DIR == 0) {
 #pragma unroll
-  for (int m = 0; m < PPT; ++m) {
-    e[m] = div(m, T(ph.gt) * (-(x[m] * ih))) + ud[m] * pd[m];
-    const T lam = GT ? lambda_of(ph, mu[m]) * Jv[m]
-                     : (EV ? PH[m] * lambda_of(ph, mu[m]) : lambda_of(ph, mu[m]));
-    f[m] = lam * (y[m] * hin);
-  }
+          for (int m = 0; m < PPT; ++m) mu[m] = viscosity(ph, tk[m]);
+          io.st(G + 6 * N, mu);
+        }
+        if constexpr (FUSE) {
+#pragma unroll
+          for (int m = 0; m < PPT; ++m) zc->mu[m] = mu[m];
+        }
+      },
+      tk, y,
+      [&] {
+#pragma unroll
+        for (int m = 0; m < PPT; ++m) {
+          const T lam = GT ? lambda_of(ph, mu[m]) * Jv[m]
+                           : (EV ? PH[m] * lambda_of(ph, mu[m]) : lambda_of(ph, mu[m]));
+          f[m] = lam * (y[m] * hin);
+        }
+      });
   ln.solve(op, f, x);
 #pragma unroll
   for (int m = 0; m < PPT; ++m) {
@@ -1225,7 +1256,7 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
     return;
   }
   {
-    // two stresses at once, the first accumulator in flight meanwhile
+    // two stresses at once (FP64), the first accumulator in flight meanwhile
     T x[PPT], y[PPT], k[PPT];
     RkIn<RK, T> in;
     constexpr bool EARLY = RK != RK_YLAST && sizeof(T) == 8;
@@ -1233,17 +1264,23 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
       io.ld(rhs + N, k);
       if constexpr (LAST) rk_load<RK, T>(rk, 1, io, N, in);
     }
-    ln.solve2(op, t1, x, t2, y);
-    asm volatile("" ::: "memory");
-    if (!EARLY) {
-      io.ld(rhs + N, k);
-      if constexpr (LAST) rk_load<RK, T>(rk, 1, io, N, in);
-    }
-    complete(1, x, k, in);
-    asm volatile("" ::: "memory");
-    io.ld(rhs + 2 * N, k);
-    if constexpr (LAST) rk_load<RK, T>(rk, 2, io, N, in);
-    complete(2, y, k, in);
+    ln.pair(
+        op, t1, x,
+        [&] {
+          asm volatile("" ::: "memory");
+          if (!EARLY) {
+            io.ld(rhs + N, k);
+            if constexpr (LAST) rk_load<RK, T>(rk, 1, io, N, in);
+          }
+          complete(1, x, k, in);
+        },
+        [] {}, t2, y,
+        [&] {
+          asm volatile("" ::: "memory");
+          io.ld(rhs + 2 * N, k);
+          if constexpr (LAST) rk_load<RK, T>(rk, 2, io, N, in);
+          complete(2, y, k, in);
+        });
   }
   {
     T x[PPT], k[PPT];
@@ -1311,9 +1348,7 @@ __device__ __forceinline__ void viscous_z_carry(const ThreadPos &tp, T *__restri
     for (int m = 0; m < PPT; ++m) v[m] = zc.mom(i, m) + v[m] * ih;
     st<2>(rhs + (1 + i) * N, B, PS, v);
   };
-  ln.solve2(op, t1, x, t2, y);
-  put(0, x);
-  put(1, y);
+  ln.pair(op, t1, x, [&] { put(0, x); }, [] {}, t2, y, [&] { put(1, y); });
   ln.solve(op, t3, x);
   put(2, x);
 }
