@@ -15,6 +15,7 @@
 
 #include "line_ops.hpp"
 #include "line_rec.hpp"
+#include "tiles.hpp"
 #include "boundary.hpp"
 #include "sweeps.hpp"
 #include "curvilinear.hpp"
@@ -258,14 +259,6 @@ SweepGeom make_geom(const int *np, int d, int TL) {
   return g;
 }
 
-int auto_tl(const int *np, int d, int wg_max, int tl_max) {
-  const long lines_contig = d == 0 ? (long)np[1] * np[2] : np[0];
-  const int NB = np[d] / PPT;
-  int TL = 1;
-  while (NB * TL * 2 <= wg_max && lines_contig % (TL * 2) == 0 && TL * 2 <= tl_max) TL *= 2;
-  return TL;
-}
-
 int build_geom(cruna_hip_ctx *c, int d) {
   const cruna_hip_cfg &cfg = c->cfg;
   const int *np = c->np;
@@ -273,14 +266,7 @@ int build_geom(cruna_hip_ctx *c, int d) {
   const int NB = np[d] / PPT;
   int TL = cfg.tile_lines[d];
   if (TL == 0) {
-    // x-lines are contiguous: up to 256 threads; y/z tiles take up to 16
-    // neighbouring x-lines (128-byte rows in FP64) in up to 512 threads.
-    // FP64 grids with less than a wavefront per SIMD (1024): work-groups of one
-    // wavefront where its lines fill it, spread over more CUs and with no
-    // barriers (a step with filters, x alone: 32^3 169 -> 155 us,
-    // 60 x 65 x 70 481 -> 471; 64^3 228 -> 224, y and z alone 225 each)
-    const bool small = cfg.precision == CRUNA_HIP_FP64 && c->N <= 1024L * 64 * PPT && 64 % NB == 0;
-    TL = d == 0 ? auto_tl(np, d, small ? 64 : 256, 1 << 20) : auto_tl(np, d, small ? 64 : NT, 16);
+    TL = auto_tile_lines(np, d, cfg.precision == CRUNA_HIP_FP64, NT);
   } else if (TL < 0 || (TL & (TL - 1)) != 0 || lines_contig % TL != 0 || NB * TL > NT) {
     return fail(CRUNA_HIP_EINVAL, "tile_lines[" + std::to_string(d) + "] = " + std::to_string(TL) +
                                       ": needs a power of two dividing " +
