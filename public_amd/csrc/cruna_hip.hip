@@ -848,8 +848,7 @@ void launch_filter(cruna_hip_ctx *c, const S *src, double *q64, int nv, T *copy)
   if constexpr (sizeof(T) == 8) {
     if (!c->fop64[DIR].rec) {
       const LineOp<double> &op = c->fcr64[DIR].op;
-      // the field exchange lies behind the (here unused) recursion cells
-      const size_t cr_lds = sweep_lds_bytes<double>(DIR, c->fwg[DIR]);
+      const size_t cr_lds = DIR == 0 ? x_stage_bytes(c->fwg[DIR]) : 0;  // the x sweeps' field exchange
       if (per)
         hipLaunchKernelGGL((k_filter_cr<DIR, true>), grid, block, cr_lds, c->stream, src, q64, op, c->fgeom[DIR], c->N, nv);
       else

@@ -371,6 +371,8 @@ template <typename T, bool PER, int NTM>
 struct CrLines {
   LineLds<T, NTM> &lds;
   const ThreadPos &tp;
+  // dynamic LDS that the engine takes (its own is static)
+  __host__ __device__ static size_t dynamic_bytes(int) { return 0; }
   template <bool FILT = false>
   __device__ __forceinline__ void solve(const LineOp<T> &op, const T (&f)[PPT], T (&x)[PPT]) {
     line_solve<T, PER>(op, lds, tp, f, x);
@@ -394,6 +396,7 @@ struct CrLines {
 
 template <bool PER>
 struct RecLines {
+  __host__ __device__ static size_t dynamic_bytes(int threads) { return rec_lds_bytes(threads); }
   char *lds;                   // dynamic LDS
   int own;                     // byte offset of the thread's slot
   int lf[REC_WIN], rt[REC_WIN];  // slots of blocks b-1, b-2, ... and b+1, b+2, ...

@@ -224,7 +224,7 @@ __device__ __forceinline__ void st(Q *__restrict__ p, long base, long PS, const 
 template <int DIR>
 struct StridedIO {
   long B, PS;
-  __device__ __forceinline__ StridedIO(const ThreadPos &tp, const SweepGeom &g) : B(tp.base), PS(g.PS) {}
+  __device__ __forceinline__ StridedIO(const ThreadPos &tp, const SweepGeom &g, size_t = 0) : B(tp.base), PS(g.PS) {}
   template <typename Q, typename V>
   __device__ __forceinline__ void ld(const Q *__restrict__ p, V (&v)[PPT]) const {
     cruna::ld<DIR>(p, B, PS, v);
@@ -242,10 +242,11 @@ struct FieldIO : StridedIO<DIR> {
 };
 
 constexpr int X_STAGE = 80;  // bytes of LDS per thread of an FP64 x sweep
+inline size_t x_stage_bytes(int threads) { return (size_t)((threads + 63) / 64 * 64) * X_STAGE; }
 // dynamic LDS of a sweep along dir in a work-group of `threads`
 template <typename T>
 size_t sweep_lds_bytes(int dir, int threads) {
-  return line_lds_bytes<T>(threads) + (dir == 0 && sizeof(T) == 8 ? (size_t)((threads + 63) / 64 * 64) * X_STAGE : 0);
+  return line_lds_bytes<T>(threads) + (dir == 0 && sizeof(T) == 8 ? x_stage_bytes(threads) : 0);
 }
 
 template <>
@@ -254,9 +255,12 @@ struct FieldIO<0, double> {
   char *own, *raw;     // LDS: the lane's slot; the place of the chunks it moves
   unsigned off;        // byte offset of its first chunk in a field
   unsigned gstep, lstep;  // distance of its chunks in the field, in LDS
-  __device__ __forceinline__ FieldIO(const ThreadPos &tp, const SweepGeom &) {
+  // (behind the line engine's dynamic LDS, of engine_bytes)
+  __device__ __forceinline__ FieldIO(const ThreadPos &tp, const SweepGeom &g)
+      : FieldIO(tp, g, rec_lds_bytes(blockDim.x)) {}
+  __device__ __forceinline__ FieldIO(const ThreadPos &tp, const SweepGeom &, size_t engine_bytes) {
     const unsigned lane = threadIdx.x & 63;
-    char *stage = line_dyn + rec_lds_bytes(blockDim.x) + (threadIdx.x >> 6) * (64 * X_STAGE);
+    char *stage = line_dyn + engine_bytes + (threadIdx.x >> 6) * (64 * X_STAGE);
     const bool idle = tp.base == IDLE_BASE;
     // lanes with a block: the first ones of the wavefront, their blocks one
     // after the other in memory
@@ -1403,7 +1407,7 @@ constexpr int filter_nt() { return sizeof(T) == 4 ? NT_FILTER32 : NT; }
 template <typename T, int DIR, typename S, typename LOp, typename Lines>
 __device__ __forceinline__ void filter_body(const ThreadPos &tp, const S *src, double *q64, const LOp &op,
                                             const SweepGeom &g, long N, int nv, T *copy, Lines &ln) {
-  const FieldIO<DIR, T> io(tp, g);
+  const FieldIO<DIR, T> io(tp, g, Lines::dynamic_bytes(blockDim.x));
   double a[PPT];
   io.ld(src, a);
   for (int v = 0; v < nv; ++v) {
