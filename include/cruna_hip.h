@@ -296,8 +296,9 @@ int cruna_hip_ensemble_set_role(cruna_hip_ensemble *ens, int i, int role, int nt
 int cruna_hip_ensemble_run(cruna_hip_ensemble *ens, int nsteps);
 /* Batched runs (on by default): when every member is FP64 on a Cartesian grid
  * without boundary rows, closure or weighted filter, the members share their
- * schemes and filter switches (frequency 0 or 1), and the adjoint members run
- * either all over whole trajectories or all over subset checkpoints of one
+ * schemes and filter switches (frequency 0 or 1; no filter that is on has an
+ * |alpha| beyond 0.4972, where filters run on cyclic reduction), and the
+ * adjoint members run either all over whole trajectories or all over subset checkpoints of one
  * length from a subset boundary, cruna_hip_ensemble_run advances whole
  * periods (a step, or a subset) in batched launches: the members split into
  * `bins` of about equal points, and each bin runs one launch per sweep kind

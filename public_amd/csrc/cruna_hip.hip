@@ -2326,7 +2326,10 @@ int batch_period(const cruna_hip_ensemble *e, int nsteps) {
     for (int d = 0; d < 3; ++d) {
       if (c->cfg.scheme[d] != c0->cfg.scheme[d] || c->cfg.wfilter_freq[d] > 0) return 0;
       const int f = c->cfg.filter_freq[d], f0 = c0->cfg.filter_freq[d];
-      if ((f > 1) || (f0 > 1) || ((f > 0) != (f0 > 0)) || !c->fop64[d].rec) return 0;
+      if ((f > 1) || (f0 > 1) || ((f > 0) != (f0 > 0))) return 0;
+      // the batched filters run on the recursions
+      const bool filters = f > 0 || (e->role[i] == CRUNA_HIP_ADJOINT && c->cfg.afilter_freq[d] > 0);
+      if (filters && !c->fop64[d].rec) return 0;
     }
     if (e->role[i] == CRUNA_HIP_ADJOINT) {
       const int si = e->subm[i] ? c->sub_steps : 0;

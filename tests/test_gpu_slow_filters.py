@@ -43,3 +43,26 @@ def test_filtered_steps_match_oracle(shape, scheme, alpha):
         g.run_direct(STEPS)
         err = rel(g.get_state(), O.run_direct(O.Cfg(shape, dx, **kw), q, STEPS))
         assert err < tol, err
+
+
+@pytest.mark.parametrize("alpha, freq, batched", [(0.45, 1, True), (0.498, 1, False), (0.498, 0, True)])
+def test_ensembles_of_slow_filters_match_their_members(alpha, freq, batched):
+    """Filters on cyclic reduction run member by member; without filters alpha does not matter."""
+    from public_amd import FORWARD, Cruna, Ensemble
+    steps, members, states = 4, [], []
+    for k, n in enumerate((32, 48)):
+        members.append(dict(n=(n,) * 3, dx=(0.2,) * 3, mu0=0.01, T0=5.0, dt=1e-4, filter_alpha=alpha,
+                            filter_freq=(freq,) * 3))
+        states.append(_state((n,) * 3, k))
+    with Ensemble(members) as ens:
+        for i, q in enumerate(states):
+            ens[i].set_state(q)
+            ens.set_role(i, FORWARD, 0)
+        ens.run(steps)
+        assert (ens.batched_steps() > 0) == batched
+        for i, q in enumerate(states):
+            kw = dict(members[i])
+            with Cruna(kw.pop("n"), kw.pop("dx"), **kw) as g:
+                g.set_state(q)
+                g.run_direct(steps)
+                assert np.array_equal(ens[i].get_state(), g.get_state())
