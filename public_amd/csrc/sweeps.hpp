@@ -1268,23 +1268,29 @@ __device__ __forceinline__ void sweep2_body(const ThreadPos &tp, T *__restrict__
       io.ld(rhs + N, k);
       if constexpr (LAST) rk_load<RK, T>(rk, 1, io, N, in);
     }
-    ln.pair(
-        op, t1, x,
-        [&] {
-          asm volatile("" ::: "memory");
-          if (!EARLY) {
-            io.ld(rhs + N, k);
-            if constexpr (LAST) rk_load<RK, T>(rk, 1, io, N, in);
-          }
-          complete(1, x, k, in);
-        },
-        [] {}, t2, y,
-        [&] {
-          asm volatile("" ::: "memory");
-          io.ld(rhs + 2 * N, k);
-          if constexpr (LAST) rk_load<RK, T>(rk, 2, io, N, in);
-          complete(2, y, k, in);
-        });
+    auto first = [&] {
+      asm volatile("" ::: "memory");
+      if (!EARLY) {
+        io.ld(rhs + N, k);
+        if constexpr (LAST) rk_load<RK, T>(rk, 1, io, N, in);
+      }
+      complete(1, x, k, in);
+    };
+    auto second = [&] {
+      asm volatile("" ::: "memory");
+      io.ld(rhs + 2 * N, k);
+      if constexpr (LAST) rk_load<RK, T>(rk, 2, io, N, in);
+      complete(2, y, k, in);
+    };
+    if constexpr (LAST) {
+      ln.pair(op, t1, x, first, [] {}, t2, y, second);
+    } else {
+      // (y and z: with an FP32 result used before the next solve, the shear
+      // layer's y sweep took 219 us instead of 186)
+      ln.solve2(op, t1, x, t2, y);
+      first();
+      second();
+    }
   }
   {
     T x[PPT], k[PPT];
