@@ -313,12 +313,21 @@ struct FieldIO<0, double> {
     for (int j = 0; j < NCH; ++j) *reinterpret_cast<double2 *>(own + j * 16) = double2{v[2 * j], v[2 * j + 1]};
     order();
     const __amdgpu_buffer_rsrc_t r = rsrc(p);
+    static_assert(NCH == 4, "the registers held below");
+    bu4 t[NCH];
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
       // (an idle lane's store is dropped; it reads its own slot)
-      const bu4 t = *reinterpret_cast<const bu4 *>(off != FIELD_EXTENT ? raw + k * lstep : own + k * 16);
-      __builtin_amdgcn_raw_buffer_store_b128(t, r, off, k * gstep, 0);
+      t[k] = *reinterpret_cast<const bu4 *>(off != FIELD_EXTENT ? raw + k * lstep : own + k * 16);
+      __builtin_amdgcn_raw_buffer_store_b128(t[k], r, off, k * gstep, 0);
     }
+    // A store of 16 bytes still reads its data registers for two wait states
+    // after it has been issued.  The compiler keeps other instructions off them
+    // for that long, but not where the store's offset is a scalar register, as
+    // here: an x sweep whose next multiplication took the last store's registers
+    // wrote a product's half in place of the data in one line of 1500.  The
+    // registers are held past the wait states.
+    asm volatile("s_nop 1" ::"v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]));
     order();
   }
 };
