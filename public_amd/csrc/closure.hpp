@@ -251,7 +251,7 @@ __global__ __launch_bounds__(CT_THREADS) void k_conv_tile(const bf16 *__restrict
     // a lane holds 4 consecutive channels of one point (channels are the matrix
     // rows): stores of 8 and 16 bytes.  With points as rows, single BF16 stores
     // and a rounding in integers the layers took 27 / 34 / 34 / 20 us at 64^3
-    // (now 21 / 22 / 22 / 16); what bounds them is a tile's phases in turn.
+    // (now 22 / 23 / 23 / 17); what bounds them is a tile's phases in turn.
     const int ii = i0 + r;
     const bool inside = ii < X && kk < Z;
 #pragma unroll

@@ -21,8 +21,7 @@ __global__ void k_adjoint_slot(const double **q0p, int *ntp, const double *traj,
 
 // Subset checkpoints inside a recorded period: the subset counter *sp
 // (device cell) names the checkpoint to restore; every thread copies its
-// share of that state into q (grid-stride, 16-byte pairs; the stride of a
-// state, 5 N, is even or handled by the tail thread).
+// share of that state of M = 5 N values into q, one value at a time (grid-stride).
 __global__ __launch_bounds__(256) void k_restore_ckpt(double *__restrict__ q, const double *__restrict__ ckpt,
                                                       const int *__restrict__ sp, long M) {
   const int s = *sp;

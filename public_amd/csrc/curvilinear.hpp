@@ -45,10 +45,11 @@ __global__ __launch_bounds__(NT) void k_curv_sweep1(const Q *__restrict__ qs, T 
   const FieldIO<DIR, T> io(tp, g);
   const T ih = T(ph.inv_h[DIR]);
   // In FP64, rho, and in the periodic x sweep the momenta, stay in
-  // registers from their first read to the convective fluxes: those sweeps
-  // have the registers for them at two waves per SIMD (the open x sweep
-  // would spill, FP32 sweeps would lose waves); re-reading them there
-  // missed the caches
+  // registers from their first read to the convective fluxes, at two waves per
+  // SIMD (FP32 sweeps would lose waves): re-reading them there missed the
+  // caches.  The periodic x sweep spills 20 bytes per lane for the momenta (36
+  // in the penalised form), 2 % more bytes than its 23 words per point; re-read,
+  // they were 18 % more.  The open y sweep spills 12 bytes
   constexpr bool KEEPR = sizeof(T) == 8, KEEPM = KEEPR && DIR == 0 && PER;
   T M0[PPT], M1[PPT], M2[PPT], rho[PPT], irho[PPT], uh[PPT], x[PPT], f[PPT];
   T mk[KEEPM ? 3 : 1][PPT];
@@ -212,7 +213,13 @@ __global__ __launch_bounds__(NT) void k_curv_sweep2(T *__restrict__ rhs, const T
   constexpr bool LAST = DIR == 0;
   const ThreadPos tp = thread_pos<DIR>(g);
   auto ln = make_lines<T, PER>(op, tp);
-  const StridedIO<DIR> io(tp, g);  // (the exchange through LDS would spill)
+  // These sweeps are at the limit of 256 registers and spill in their x and open
+  // forms: 44 bytes per lane in the periodic x sweep, 60 with the x filter, 276
+  // with it on open lines (penalised forms up to 340).  They are faster than the
+  // cyclic reduction's were without spills all the same: 128^3 x sweep 117 ->
+  // 107 us periodic, 171 -> 120 open.  Field accesses are the threads' own; the
+  // exchange through LDS would take more registers still.
+  const StridedIO<DIR> io(tp, g);
   const T ih = T(ph.inv_h[DIR]);
   T M0[PPT], M1[PPT], M2[PPT], mu[PPT];
   io.ld(mt.M + (DIR + 0) * N, M0);
